@@ -665,6 +665,8 @@ static int pbf_adj_create_impl(const pbf_params* p, int64_t n, int32_t nsteps, i
   }
   a->n = n;
   a->npad = (n + 63) / 64 * 64;
+  // The adjoint reads the lists by particle index: no LDS tiles.
+  X(a)->tile_min = INT64_MAX;
   // Four lanes per particle while that still leaves under ~4M threads
   // (small scenes are latency-bound); PBF_ADJ_LANES = 1, 2 or 4 overrides.
   a->lanes = n <= (1 << 20) ? 4 : 1;

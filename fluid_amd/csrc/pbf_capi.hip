@@ -103,6 +103,7 @@ void free_device(Ctx* x) {
   dfree(d.nbr); dfree(d.ncnt); dfree(d.flags);
   dfree(d.grids); dfree(d.slotScene); dfree(d.runs); dfree(d.stage); dfree(d.dense);
   dfree(d.dense_b);
+  dfree(d.titem); dfree(d.trec); dfree(d.town); dfree(d.tnbr); dfree(d.tflag);
   x->alloc_n = 0;
   x->alloc_cells = 0;
 }
@@ -122,6 +123,30 @@ void drop_graph(Ctx* x) {
 template <class T>
 hipError_t dalloc(T*& p, size_t count) {
   return hipMalloc((void**)&p, std::max<size_t>(count, 1) * sizeof(T));
+}
+
+// Buffers of the LDS tiles, for states that step on them.  Without them (no
+// memory left) the state keeps the other list passes.
+void alloc_tiles(Ctx* x) {
+  pbf::DevState& d = x->d;
+  x->tile_cap = x->tile_units = 0;
+  const size_t n = (size_t)x->n;
+  if (x->n < x->tile_min || x->tile_blocks == 0 || x->tile_blocks > n) return;
+  // A tile of 24 particles or more takes a unit per 64, so tiles this full
+  // need n / 24 units at most; blocks past the capacity go to the queue.
+  const size_t units = n / 40 + 1024, items = n / 64 + 1024;
+  hipError_t e = dalloc(d.titem, items);
+  if (e == hipSuccess) e = dalloc(d.trec, items);
+  if (e == hipSuccess) e = dalloc(d.town, units * 64);
+  if (e == hipSuccess) e = dalloc(d.tnbr, units * 64 * 8 * pbf::kTileChunks);
+  if (e == hipSuccess) e = dalloc(d.tflag, x->tile_blocks);
+  if (e != hipSuccess) {
+    dfree(d.titem); dfree(d.trec); dfree(d.town); dfree(d.tnbr); dfree(d.tflag);
+    (void)hipGetLastError();
+    return;
+  }
+  x->tile_cap = (uint32_t)items;
+  x->tile_units = (uint32_t)units;
 }
 
 int ensure_device(Ctx* x) {
@@ -151,6 +176,7 @@ int ensure_device(Ctx* x) {
   }
   x->alloc_n = n;
   x->alloc_cells = C;
+  alloc_tiles(x);
   return PBF_OK;
 }
 
@@ -207,6 +233,27 @@ int verify_math(Ctx* x) {
   return PBF_OK;
 }
 
+// Base blocks of a single scene's grid, and the place of the record that pads
+// the tiles' lists: beyond h of every particle, its distances in the range
+// of the short sequences (tile_blocks stays 0 where that fails).
+void plan_tiles(Ctx* x) {
+  x->tile_blocks = 0;
+  if (x->nscenes != 1) return;
+  const SimConst k = pbf::consts_for(*x, x->p.dt);
+  const SceneGrid& g = x->grids[0];
+  float far = 0.0f, span = 0.0f;
+  for (int a = 0; a < 3; a++) {
+    far = std::max(far, std::max(fabsf(g.lo[a]), fabsf(g.hi[a])));
+    span = std::max(span, g.hi[a] - g.lo[a]);
+  }
+  x->tile_far = far + 4.0f * k.h;
+  const float reach = 4.0f * (far + span + 4.0f * k.h);  // above every |r|
+  const size_t blocks = pbf::tile_block_count(g);
+  if (x->tile_far - far > 2.0f * k.h && reach * reach < 0x1p100f && k.h6 * reach < 0x1p100f &&
+      blocks < ((size_t)1 << 30))
+    x->tile_blocks = (uint32_t)blocks;
+}
+
 int finish_create(Ctx* x, pbf_ctx** out) {
   uint64_t total = 0;
   for (auto& g : x->grids) {
@@ -220,6 +267,7 @@ int finish_create(Ctx* x, pbf_ctx** out) {
     return fail(nullptr, PBF_ERR_INVALID, m);
   }
   x->ncell = (uint32_t)total;
+  plan_tiles(x);
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e == hipSuccess) e = hipDeviceGetAttribute(&x->ncu, hipDeviceAttributeMultiprocessorCount, dev);
@@ -239,6 +287,8 @@ int finish_create(Ctx* x, pbf_ctx** out) {
     for (pbf::PassRule& r : x->rules) r.wave_max = atoll(w);
   if (const char* w = getenv("PBF_QUAD_MAX"))
     for (pbf::PassRule& r : x->rules) r.quad_max = atoll(w);
+  // PBF_TILE_MIN=n: states of at least n particles step on LDS tiles.
+  if (const char* w = getenv("PBF_TILE_MIN")) x->tile_min = atoll(w);
   if (const char* w = getenv("PBF_DENSE_LIST")) x->dense_list = (uint32_t)atoll(w);
   if (const char* w = getenv("PBF_DENSE_CELL")) x->dense_cell = (uint32_t)atoll(w);
   // PBF_RULE_<PASS>=wave_max,quad_max sets one pass's bounds.
@@ -308,9 +358,13 @@ int run_step(Ctx* x, const SimConst& c, int stage, PassEvents* pe = nullptr,
   // stops keep both (they read them back).  Restored on every return.
   struct SortedV {
     Ctx* x;
-    ~SortedV() { x->sorted_v = true; }
+    ~SortedV() {
+      x->sorted_v = true;
+      x->tile_on = false;
+    }
   } restore{x};
   x->sorted_v = stage != 0;
+  x->tile_on = stage == 0 && pbf::tile_step(*x);
   if (!predicted) PASS(PBF_PASS_PREDICT, pbf::launch_predict(*x, c));
   // A prediction fused into the previous step's last pass sits in vort.
   if (x->small_sort && pbf::sort_in_one_workgroup(*x)) {
@@ -333,6 +387,7 @@ int run_step(Ctx* x, const SimConst& c, int stage, PassEvents* pe = nullptr,
   else
     PASS(PBF_PASS_NEIGHBORS, pbf::launch_nbr_build(*x, c));
   x->has_nbrs = true;
+  x->tile_lists = x->tile_on;
   if (stage == PBF_STAGE_NEIGHBORS) return PBF_OK;
   for (int it = 0; it < x->p.iterations; it++) {
     if (!(fuse && it == 0))
@@ -492,6 +547,10 @@ void derive_constants(const pbf_params& p, float dt, SimConst* c) {
   int e_hi = 100;
   if (c->r9 > 0.0f && isfinite(c->r9)) e_hi = std::min(100, 100 - ilogbf(c->r9) - 1);
   c->div_hi = ldexpf(1.0f, std::max(e_hi, -126));
+  // From 2^-90 or (1.0001 EPS_D)^2, whichever is larger, a correctly rounded
+  // root is at least EPS_D.
+  const float em = p.eps_d * 1.0001f;
+  c->r2_min = std::max(0x1p-90f, em * em);
   c->fast_div = 0;
   c->fast_rcp = 0;
   c->fast_sqrt = 0;
@@ -764,6 +823,7 @@ int enqueue_steps(Ctx* x, float dt, int nsteps) {
     const int grid = std::max(1, std::min(x->nscenes, std::max(1, x->ncu) * per));
     HIPCHK(x, pbf::launch_persistent(*x, k, nsteps, x->pblock, grid));
     x->has_nbrs = true;
+    x->tile_lists = false;
     x->dbg_vel = x->d.velA;
   } else if (x->schedule == PBF_SCHED_GRAPH && nsteps >= 3) {
     // The first step (it predicts) and the last (it commits without

@@ -32,6 +32,7 @@ struct SimConst {
   int fast_div;          // poly6 divides by h^9 with div_seq
   int fast_rcp;          // spiky takes its reciprocal with rcp_seq
   int fast_sqrt;         // spiky takes its square root with sqrt_rn
+  float r2_min;          // |r|^2 from which |r| >= EPS_D for certain (tiled passes)
 };
 
 // Grid and collision box of one scene.
@@ -411,10 +412,35 @@ __device__ __forceinline__ float3 collide(const SceneGrid& g, const SimConst& c,
                      smax(g.lo_e[2], smin(g.hi_e[2], pa[2])));
 }
 
+// Whether a displacement D from p meets no wall of the box and is longer than
+// EPS_D for certain, so that the collision is p + D and the final clamp (box
+// walls only, no mesh).  |D| <= |D.x| + |D.y| + |D.z| =: s; a wall farther
+// than 1.0001 s has t > |D| in collide(), whose roundings (the direction,
+// the difference and the quotient, an ulp or two each) are far below 1e-4,
+// and a component above 1.0001 EPS_D makes |D| exceed EPS_D.  Nearly every
+// particle passes, which spares it a square root and four divisions.  NaN
+// fails the comparisons.
+__device__ __forceinline__ bool moves_free(const SceneGrid& g, const SimConst& c, float3 p,
+                                           float3 D) {
+  const float ax = fabsf(D.x), ay = fabsf(D.y), az = fabsf(D.z);
+  const float s = (ax + ay + az) * 1.0001f;
+  const float room = fminf(fminf(fminf(p.x - g.lo[0], g.hi[0] - p.x),
+                                 fminf(p.y - g.lo[1], g.hi[1] - p.y)),
+                           fminf(p.z - g.lo[2], g.hi[2] - p.z));
+  return room > s && fmaxf(fmaxf(ax, ay), az) > c.eps_d * 1.0001f;
+}
+
+__device__ __forceinline__ float3 move_free(const SceneGrid& g, float3 p, float3 D) {
+  return make_float3(smax(g.lo_e[0], smin(g.hi_e[0], p.x + D.x)),
+                     smax(g.lo_e[1], smin(g.hi_e[1], p.y + D.y)),
+                     smax(g.lo_e[2], smin(g.hi_e[2], p.z + D.z)));
+}
+
 // clamp_response (src/particles.cpp:87-132): prediction with slide.
 __device__ __forceinline__ float3 clamp_response(const SceneGrid& g, const SimConst& c,
                                                  const MeshView& m, float3 p, float3 v) {
   float3 D = make_float3(v.x * c.dt, v.y * c.dt, v.z * c.dt);
+  if (!m.ntri && moves_free(g, c, p, D)) return move_free(g, p, D);
   float total = sqrtf(D.x * D.x + D.y * D.y + D.z * D.z);
   if (total <= c.eps_d) return p;
   float rl = 1.0f / total;
@@ -426,6 +452,7 @@ __device__ __forceinline__ float3 clamp_response(const SceneGrid& g, const SimCo
 // clamp (src/particles.cpp:51-84): position correction, no slide.
 __device__ __forceinline__ float3 clamp_dp(const SceneGrid& g, const SimConst& c,
                                            const MeshView& m, float3 p, float3 dp) {
+  if (!m.ntri && moves_free(g, c, p, dp)) return move_free(g, p, dp);
   float l = sqrtf(dp.x * dp.x + dp.y * dp.y + dp.z * dp.z);
   if (l <= c.eps_d) return p;
   float rl = 1.0f / l;

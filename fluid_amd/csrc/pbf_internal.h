@@ -21,6 +21,24 @@ struct SceneRun {
   uint32_t ncells;  // cells of its grid
 };
 
+// One LDS tile (pbf_tiles.h): its low corner, its cells per axis (4 bits
+// each), its first unit (a wave's lanes and lists) and its particles.
+struct TileItem {
+  int x0, y0, z0;
+  uint32_t dims;
+  uint32_t unit, n;
+};
+// What the passes after the build read of a tile: first unit, particles
+// and its rows (first particle; first slot, particles << 16).
+constexpr int kTileRows = 32;
+struct TileRec {
+  uint2 head;
+  uint2 row[kTileRows];
+};
+constexpr int kTileChunks = 32;  // 16-byte list chunks of 8 entries per lane
+constexpr int kTileZeroSlot = 12;  // kDenseSlot, kDenseBuildSlot, kTileUnitsSlot, kTileItemsSlot
+constexpr int kTileUnitsSlot = 14, kTileItemsSlot = 15;  // low and high word of one counter
+
 // Device state of one context.  All particle arrays are float4 and are kept
 // in cell-sorted order between steps; posA.w carries the particle's load
 // index (its id) as integer bits.
@@ -54,6 +72,11 @@ struct DevState {
   uint8_t* meshFlag = nullptr;    // scene-grid cells near a BVH leaf box (MeshView::flag)
   uint32_t* dense = nullptr;      // particles with long lists, queued by the build (n)
   uint32_t* dense_b = nullptr;    // particles in crowded cells, queued by the sort (n)
+  TileItem* titem = nullptr;      // LDS tiles of the step (pbf_tiles.h)
+  uint8_t* tflag = nullptr;       // base blocks whose particles are tiled
+  TileRec* trec = nullptr;        // rows of each tile
+  uint2* town = nullptr;          // particle, own slot and list length of each lane
+  uint16_t* tnbr = nullptr;       // lists of the tiles, as LDS byte offsets
 };
 
 // Lanes per particle of each list pass, by state size: one wave (64 lanes)
@@ -123,7 +146,7 @@ constexpr int kDenseSlot = 12;
 // each (k_nbr_quad's walk) and run their first lambda on the same quad.
 // PBF_DENSE_CELL overrides the threshold (0: off).
 constexpr uint32_t kDenseCell = 32;
-constexpr int kDenseBuildSlot = 13;
+constexpr int kDenseBuildSlot = 13;  // in a tiled step: the particles without a tile
 
 struct Ctx {
   pbf_params p{};
@@ -167,6 +190,16 @@ struct Ctx {
   // velocity comes from x* - x and the commit rewrites velA), so run_step
   // clears this for full steps; the debug stops and the adjoint keep it.
   bool sorted_v = true;
+  bool tile_lists = false;           // the last step's lists are the tiles'
+  uint32_t tile_blocks = 0;          // base blocks of the grid (0: no tiles)
+  float tile_far = 0.0f;             // x of the padding record
+  bool tile_on = false;              // the running step takes the LDS tiles
+  // States of at least this many particles step on LDS tiles (measured in ms
+  // per step, per-lane passes / tiles: 300,000 particles 0.341 / 0.345, 350,000
+  // 0.397 / 0.385, 400,000 0.451 / 0.417, 700,000 0.695 / 0.578).
+  int64_t tile_min = 400000;
+  uint32_t tile_cap = 0;             // items allocated
+  uint32_t tile_units = 0;           // units allocated
   // Density-field output on the device, kept between calls, and two pinned
   // host slabs through which large results return (allocated on first use).
   float* field_dev = nullptr;
@@ -255,6 +288,10 @@ hipError_t launch_nbr_stats(Ctx& x, unsigned long long* sum, uint32_t* mx);
 // Exclusive scan of in[0..n) into out[0..n], out[n] = total; with clear_in
 // the counts are zero afterwards.
 hipError_t launch_scan_u32(uint32_t* in, uint32_t* out, uint32_t n, uint32_t* partials,
-                           hipStream_t s, bool clear_in = false);
+                           hipStream_t s, bool clear_in = false, uint32_t* zero4 = nullptr);
+// Whether a step of x runs on LDS tiles; base blocks of one scene's grid.
+bool tile_step(const Ctx& x);
+size_t tile_block_count(const SceneGrid& g);
+
 
 }  // namespace pbf

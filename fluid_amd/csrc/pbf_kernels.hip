@@ -27,6 +27,8 @@
 // functions, so both give the same bits.
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "pbf_internal.h"
 
 namespace pbf {
@@ -63,6 +65,14 @@ struct Dev {
   // Nonzero: the prediction stores the advanced v in velA and the sort moves
   // it to velB (read only by debug stops and the adjoint).
   uint32_t move_v;
+  // LDS tiles (pbf_tiles.h; titem NULL: off).
+  TileItem* titem;
+  uint8_t* tflag;
+  TileRec* trec;
+  uint2* town;
+  uint16_t* tnbr;
+  uint32_t tile_items, tile_units;
+  float tile_far;
   uint32_t n;
   int K4;
 };
@@ -99,6 +109,20 @@ Dev dev_of(const Ctx& x) {
   d.dense_cell = x.dense_cell;
   d.move_v = x.sorted_v ? 1u : 0u;
   d.nlane = 0;
+  d.titem = nullptr;
+  if (x.tile_on) {
+    d.titem = s.titem;
+    d.tflag = s.tflag;
+    d.trec = s.trec;
+    d.town = s.town;
+    d.tnbr = s.tnbr;
+    d.tile_items = x.tile_cap;
+    d.tile_units = x.tile_units;
+    d.tile_far = x.tile_far;
+    d.dense = s.dense;
+    d.dense_b = s.dense_b;
+    d.dense_cell = 0xffffffffu;
+  }
   d.n = (uint32_t)x.n;
   d.K4 = k4_of(x);
   return d;
@@ -128,8 +152,10 @@ constexpr int kScanTile = kBlock * kScanItems;
 // partials.  With clear, the counts are set to zero once read.
 __global__ __launch_bounds__(kBlock) void k_scan_block(uint32_t* __restrict__ in,
                                                        uint32_t* __restrict__ out, uint32_t n,
-                                                       uint32_t* __restrict__ partials, bool clear) {
+                                                       uint32_t* __restrict__ partials, bool clear,
+                                                       uint32_t* __restrict__ zero4) {
   __shared__ uint32_t wsum[kBlock / 64];
+  if (zero4 && blockIdx.x == 0 && threadIdx.x < 4) zero4[threadIdx.x] = 0u;
   const uint32_t base = blockIdx.x * kScanTile + threadIdx.x * kScanItems;
   uint32_t v[kScanItems];
   if (base + kScanItems <= n) {
@@ -340,8 +366,8 @@ __device__ __forceinline__ void scatter_one(uint32_t i, const Dev& d) {
 // Everything the particle moves is loaded before the count, and the cell's
 // ids are read four at a time with independent loads, so the loads of one
 // particle overlap instead of waiting on each other.
-__device__ __forceinline__ void rank_one(uint32_t i, const Dev& d,
-                                         const float4* __restrict__ pred) {
+__device__ __forceinline__ uint32_t rank_one(uint32_t i, const Dev& d,
+                                             const float4* __restrict__ pred) {
   const float4 x = d.posA[i];
   const float4 v = d.move_v ? d.velA[i] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
   const float4 q = pred[i];
@@ -362,7 +388,7 @@ __device__ __forceinline__ void rank_one(uint32_t i, const Dev& d,
             (uint32_t)(t + 2 < e && a2 < id) + (uint32_t)(t + 3 < e && a3 < id);
   }
   const uint32_t dst = s + rank;
-  if (dst >= d.n) return;
+  if (dst >= d.n) return 0xffffffffu;
   d.posB[dst] = x;
   if (d.move_v) d.velB[dst] = v;
   d.predQ[dst] = q;
@@ -372,6 +398,7 @@ __device__ __forceinline__ void rank_one(uint32_t i, const Dev& d,
     const uint32_t slot = atomicAdd(&d.flags[kDenseBuildSlot], 1u);
     if (slot < d.n) d.dense_b[slot] = dst;  // each particle once per step: slot < n
   }
+  return dst;
 }
 
 // Distance from coordinate x to the near face of cell k+side of the axis
@@ -1006,7 +1033,7 @@ __global__ __launch_bounds__(kBlock) void k_predict_into(Dev d, SimConst c, Scen
 __global__ __launch_bounds__(kBlock) void k_scatter(Dev d) {
   const uint32_t i = flat_index();
   if (i < d.n) scatter_one(i, d);
-  if (i == 0 && d.dense_b) d.flags[kDenseBuildSlot] = 0u;
+  if (i == 0 && d.dense_b && !d.titem) d.flags[kDenseBuildSlot] = 0u;
 }
 
 __global__ __launch_bounds__(kBlock) void k_rank(Dev d, const float4* pred) {
@@ -1534,6 +1561,20 @@ __global__ __launch_bounds__(kBlock) void k_xsph_quad(Dev d, SimConst c, float4*
   if (i < d.n) xsph_quad_one(i, d, c, out);
 }
 
+// Neighbour list of sorted particle i by load id.
+__device__ __forceinline__ void nbr_export_one(uint32_t i, const Dev& d,
+                                               uint32_t* __restrict__ counts,
+                                               uint32_t* __restrict__ out, int stride) {
+  const uint32_t id = id_of(d.posB[i]);
+  const int cnt = (int)d.ncnt[i];
+  counts[id] = (uint32_t)cnt;
+  const int m = cnt < stride ? cnt : stride;
+  for (int k = 0; k < m; k++)
+    out[(size_t)id * stride + k] = id_of(d.posB[d.nbr[nbr_slot(i, k, d.K4)]]);
+}
+
+#include "pbf_tiles.h"
+
 // Scan, scatter and rank of a small state in one workgroup: the three
 // passes that otherwise take four or five launches, with workgroup barriers
 // between them (every thread of the workgroup shares one CU's cache, so a
@@ -1583,13 +1624,7 @@ __global__ __launch_bounds__(kBlock) void k_unpermute_u32(uint32_t n,
 __global__ __launch_bounds__(kBlock) void k_nbr_export(Dev d, uint32_t* __restrict__ counts,
                                                        uint32_t* __restrict__ out, int stride) {
   const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-  if (i >= d.n) return;
-  const uint32_t id = id_of(d.posB[i]);
-  const int cnt = (int)d.ncnt[i];
-  counts[id] = (uint32_t)cnt;
-  const int m = cnt < stride ? cnt : stride;
-  for (int k = 0; k < m; k++)
-    out[(size_t)id * stride + k] = id_of(d.posB[d.nbr[nbr_slot(i, k, d.K4)]]);
+  if (i < d.n) nbr_export_one(i, d, counts, out, stride);
 }
 
 // Sum and maximum of the neighbour counts (64-bit sum, maximum).
@@ -1664,13 +1699,14 @@ hipError_t launch_fill_u32(uint32_t* p, size_t n, uint32_t v, hipStream_t s) {
 }
 
 hipError_t launch_scan_u32(uint32_t* in, uint32_t* out, uint32_t n, uint32_t* partials,
-                           hipStream_t s, bool clear_in) {
+                           hipStream_t s, bool clear_in, uint32_t* zero4) {
   const uint32_t nb = (n + kScanTile - 1) / kScanTile;
-  if (nb > 0) k_scan_block<<<nb, kBlock, 0, s>>>(in, out, n, partials, clear_in);
+  if (nb > 0) k_scan_block<<<nb, kBlock, 0, s>>>(in, out, n, partials, clear_in, zero4);
   k_scan_partials<<<1, 1024, 0, s>>>(partials, nb, out, n);
   if (nb > 1) k_scan_add<<<blocks_for(n), kBlock, 0, s>>>(out, n, partials);
   return hipGetLastError();
 }
+
 
 static bool multi(const Ctx& x) { return x.nscenes > 1; }
 
@@ -1688,7 +1724,8 @@ hipError_t launch_predict(Ctx& x, const SimConst& c) {
 hipError_t launch_scan(Ctx& x) {
   // The histogram is spent once scanned: the tile pass clears it for the
   // next prediction, which then needs no fill launch of its own.
-  return launch_scan_u32(x.d.cellCount, x.d.cellStart, x.ncell, x.d.blockSums, x.stream, true);
+  return launch_scan_u32(x.d.cellCount, x.d.cellStart, x.ncell, x.d.blockSums, x.stream, true,
+                         x.tile_on ? x.d.flags + kTileZeroSlot : nullptr);
 }
 
 bool sort_in_one_workgroup(const Ctx& x) {
@@ -1701,9 +1738,29 @@ hipError_t launch_sort_small(Ctx& x, const float4* pred) {
   return hipGetLastError();
 }
 
+size_t tile_block_count(const SceneGrid& g) {
+  return (size_t)((g.dims[0] + kTX - 1) / kTX) * (size_t)((g.dims[1] + kTY - 1) / kTY) *
+         (size_t)((g.dims[2] + kTZ - 1) / kTZ);
+}
+
+bool tile_step(const Ctx& x) {
+  return x.d.titem && x.n >= x.tile_min && x.fast_div && x.fast_rcp && x.fast_sqrt &&
+         x.schedule != PBF_SCHED_PERSISTENT && !(x.small_sort && sort_in_one_workgroup(x));
+}
+
+static unsigned tile_grid(const Ctx& x) {
+  const unsigned g = 8u * kTileRun;
+  return kTileQuads + ((unsigned)(x.n / 384) + 1024u + g - 1u) / g * g;
+}
+
 hipError_t launch_scatter_rank(Ctx& x, const float4* pred) {
   const Dev d = dev_of(x);
   k_scatter<<<blocks_for(x.n), kBlock, 0, x.stream>>>(d);
+  if (x.tile_on) {
+    k_tile_items<<<blocks_for(x.tile_blocks), kBlock, 0, x.stream>>>(d, x.grids[0]);
+    k_rank_tiled<<<(unsigned)((x.n + kRankBlock - 1) / kRankBlock), kRankBlock, 0, x.stream>>>(d, pred ? pred : d.predP, x.grids[0]);
+    return hipGetLastError();
+  }
   k_rank<<<blocks_for(x.n), kBlock, 0, x.stream>>>(d, pred ? pred : d.predP);
   return hipGetLastError();
 }
@@ -1749,6 +1806,11 @@ hipError_t launch_nbr_build(Ctx& x, const SimConst& c) {
 
 hipError_t launch_nbr_lambda(Ctx& x, const SimConst& c, float4* out) {
   const Dev d = dev_of(x);
+  if (x.tile_on) {
+    k_tile_build<<<tile_grid(x), kTileBlock, 0, x.stream>>>(d, c, x.grids[0], out);
+    k_queue_build<<<kQueueBuildGrid, kBlock, 0, x.stream>>>(d, c, x.grids[0], out);
+    return hipGetLastError();
+  }
   if (quad(x, kPassBuild)) {
     // The quad build, then the first lambda pass over the finished lists.
     k_nbr_quad<<<quad_grid(x), kBlock, 0, x.stream>>>(d, c.h2, x.grids[0]);
@@ -1775,6 +1837,10 @@ hipError_t launch_nbr_lambda(Ctx& x, const SimConst& c, float4* out) {
 }
 
 hipError_t launch_lambda(Ctx& x, const SimConst& c, const float4* in, float4* out, bool packed) {
+  if (x.tile_on) {
+    k_tile_lambda<<<tile_grid(x), kTileBlock, 0, x.stream>>>(dev_of(x), c, out);
+    return hipGetLastError();
+  }
   if (quad(x, kPassLambda)) {
     if (packed)
       k_lambda_quad<true><<<quad_grid(x), kBlock, 0, x.stream>>>(dev_of(x), c, in, out);
@@ -1802,6 +1868,14 @@ template <int NT>
 static void launch_deltap_nt(const Ctx& x, const Dev& d, const SimConst& c, const float4* in,
                              float4* out, bool last) {
   const unsigned nb = blocks_for(x.n);
+  if (x.tile_on) {
+    const unsigned ng = tile_grid(x);
+    if (last)
+      k_tile_deltap<true, NT><<<ng, kTileBlock, 0, x.stream>>>(d, c, x.grids[0], in);
+    else
+      k_tile_deltap<false, NT><<<ng, kTileBlock, 0, x.stream>>>(d, c, x.grids[0], in);
+    return;
+  }
   if (quad(x, kPassDeltap)) {
     if (last)
       k_deltap_quad<true, NT><<<quad_grid(x), kBlock, 0, x.stream>>>(d, c, x.grids[0], in);
@@ -1849,6 +1923,10 @@ hipError_t launch_deltap(Ctx& x, const SimConst& c, const float4* in, float4* ou
 }
 
 hipError_t launch_xsph(Ctx& x, const SimConst& c, float4* out) {
+  if (x.tile_on) {
+    k_tile_xsph<<<tile_grid(x), kTileBlock, 0, x.stream>>>(dev_of(x), c, out);
+    return hipGetLastError();
+  }
   if (quad(x, kPassXsph)) {
     k_xsph_quad<<<quad_grid(x), kBlock, 0, x.stream>>>(dev_of(x), c, out);
     return hipGetLastError();
@@ -1878,6 +1956,13 @@ hipError_t launch_vort_commit_predict(Ctx& x, const SimConst& c, const float4* i
   // general scan clear it once read), so the next prediction needs no fill.
   const bool small = x.small_sort && sort_in_one_workgroup(x);
   const Dev d = dev_of(x);
+  if (x.tile_on) {
+    // The prediction as a launch of its own: fused, every wave of a tile
+    // would wait for its histogram atomics while it holds the tile's LDS.
+    k_tile_vort<<<tile_grid(x), kTileBlock, 0, x.stream>>>(d, c, in);
+    k_predict_into<false><<<blocks_for(x.n), kBlock, 0, x.stream>>>(d, c, x.grids[0], d.vort);
+    return hipGetLastError();
+  }
   if (wide(x, kPassVort) && !small) {
     // Beyond the smallest states the wide pass commits and the prediction
     // follows as its own launch (the serial tail of one lane per particle,
@@ -1911,6 +1996,10 @@ hipError_t launch_vort_commit_predict(Ctx& x, const SimConst& c, const float4* i
 }
 
 hipError_t launch_vort_commit(Ctx& x, const SimConst& c, const float4* in) {
+  if (x.tile_on) {
+    k_tile_vort<<<tile_grid(x), kTileBlock, 0, x.stream>>>(dev_of(x), c, in);
+    return hipGetLastError();
+  }
   if (quad(x, kPassVort)) {
     k_vort_quad<false><<<quad_grid(x), kBlock, 0, x.stream>>>(dev_of(x), c, x.grids[0], in);
     return hipGetLastError();
@@ -1976,6 +2065,14 @@ hipError_t launch_unpermute_u32(Ctx& x, const float4* ids, const uint32_t* src, 
 }
 
 hipError_t launch_nbr_export(Ctx& x, uint32_t* counts, uint32_t* ids, int stride) {
+  if (x.tile_lists) {
+    x.tile_on = true;
+    const Dev d = dev_of(x);
+    x.tile_on = false;
+    k_tile_export<<<1024, kTileBlock, 0, x.stream>>>(d, counts, ids, stride);
+    k_queue_export<<<256, kBlock, 0, x.stream>>>(d, counts, ids, stride);
+    return hipGetLastError();
+  }
   k_nbr_export<<<blocks_for(x.n), kBlock, 0, x.stream>>>(dev_of(x), counts, ids, stride);
   return hipGetLastError();
 }
