@@ -101,7 +101,7 @@ void free_device(Ctx* x) {
   dfree(d.cell); dfree(d.arrival); dfree(d.cellSorted); dfree(d.tmpId);
   dfree(d.cellCount); dfree(d.cellStart); dfree(d.blockSums);
   dfree(d.nbr); dfree(d.ncnt); dfree(d.flags);
-  dfree(d.grids); dfree(d.slotScene); dfree(d.runs); dfree(d.stage); dfree(d.dense);
+  dfree(d.grids); dfree(d.first); dfree(d.slotScene); dfree(d.runs); dfree(d.stage); dfree(d.dense);
   dfree(d.dense_b);
   dfree(d.titem); dfree(d.trec); dfree(d.town); dfree(d.tnbr); dfree(d.tflag);
   x->alloc_n = 0;
@@ -151,6 +151,9 @@ void alloc_tiles(Ctx* x) {
 
 int ensure_device(Ctx* x) {
   if (x->alloc_n == (size_t)x->n && x->alloc_cells == (size_t)x->ncell && x->d.posA) return PBF_OK;
+  // The captured steps hold these buffers' addresses; a load into the same
+  // buffers keeps them.
+  drop_graph(x);
   free_device(x);
   pbf::DevState& d = x->d;
   const size_t n = (size_t)x->n, np = (size_t)x->npad, C = (size_t)x->ncell;
@@ -165,7 +168,7 @@ int ensure_device(Ctx* x) {
   DA(d.cell, np); DA(d.arrival, np); DA(d.cellSorted, np); DA(d.tmpId, np);
   DA(d.cellCount, C + 4); DA(d.cellStart, C + 4); DA(d.blockSums, nb);
   DA(d.nbr, np * K); DA(d.ncnt, np); DA(d.flags, 64);
-  DA(d.grids, (size_t)x->nscenes); DA(d.slotScene, np); DA(d.runs, (size_t)x->nscenes);
+  DA(d.grids, (size_t)x->nscenes); DA(d.first, (size_t)x->nscenes); DA(d.slotScene, np); DA(d.runs, (size_t)x->nscenes);
   DA(d.stage, 4 * np);
   DA(d.dense, np);
   DA(d.dense_b, np);
@@ -692,6 +695,8 @@ PBF_API int pbf_destroy(pbf_ctx* c) {
   dfree(x->d.meshFlag);
   stage_free(x);
   if (x->flag_host) (void)hipHostFree(x->flag_host);
+  dfree(x->load_dev);
+  dfree(x->load_bad);
   dfree(x->field_dev);
   dfree(x->field_pts);
   if (x->stream) (void)hipStreamDestroy(x->stream);
@@ -720,6 +725,61 @@ PBF_API int pbf_load(pbf_ctx* c, const float* xyz, const float* v, int64_t n) {
 }
 
 namespace {
+// Loads of at least this many particles are checked and packed on the device
+// (us per load call, on the host / on the device: 720 particles 44 / 54, 2,106
+// 67 / 69, 4,096 101 / 89, 20,011 130 / 71, 262,144 650 / 237, 1,000,003
+// 2,640 / 748, 4,096,000 31,000 / 3,580; the copy of 24 bytes per particle
+// from pageable memory, ~29 GB/s, is what remains).
+constexpr int64_t kLoadDeviceMin = 3072;
+
+// Uploads xyz, v and rho (v, rho may be NULL) into load_dev and runs the
+// checks of host::validate_pack there.  The particle state is untouched.
+int load_check(Ctx* x, const float* xyz, const float* v, const float* rho, int64_t n, int* code,
+               int64_t* first) {
+  const size_t m = (size_t)n * 3, need = 2 * m + (rho ? (size_t)n : 0);
+  if (x->load_cap < need) {
+    dfree(x->load_dev);
+    x->load_cap = 0;
+    if (dalloc(x->load_dev, need) != hipSuccess)
+      return fail(x, PBF_ERR_NOMEM, "device allocation failed: load buffer");
+    x->load_cap = need;
+  }
+  if (!x->load_bad && dalloc(x->load_bad, 1) != hipSuccess)
+    return fail(x, PBF_ERR_NOMEM, "device allocation failed: load check");
+  if (!x->flag_host) HIPCHK(x, hipHostMalloc((void**)&x->flag_host, 64, hipHostMallocDefault));
+  if (x->nscenes > 1) {
+    // The boxes and first particles of the scenes (their sizes are fixed, so
+    // this never replaces the buffers of a loaded state).
+    x->n = n;
+    x->npad = (n + 63) / 64 * 64;
+    const int rc = ensure_device(x);
+    if (rc != PBF_OK) return rc;
+    std::vector<uint32_t> first_of(x->offsets.begin(), x->offsets.end());
+    HIPCHK(x, hipMemcpyAsync(x->d.grids, x->grids.data(), x->grids.size() * sizeof(SceneGrid),
+                             hipMemcpyHostToDevice, x->stream));
+    HIPCHK(x, hipMemcpyAsync(x->d.first, first_of.data(), first_of.size() * sizeof(uint32_t),
+                             hipMemcpyHostToDevice, x->stream));
+    HIPCHK(x, hipStreamSynchronize(x->stream));
+  }
+  float *dx = x->load_dev, *dv = dx + m;
+  HIPCHK(x, hipMemcpyAsync(dx, xyz, m * sizeof(float), hipMemcpyHostToDevice, x->stream));
+  if (v) HIPCHK(x, hipMemcpyAsync(dv, v, m * sizeof(float), hipMemcpyHostToDevice, x->stream));
+  if (rho)
+    HIPCHK(x, hipMemcpyAsync(dv + m, rho, (size_t)n * sizeof(float), hipMemcpyHostToDevice,
+                             x->stream));
+  HIPCHK(x, pbf::launch_fill_u32(reinterpret_cast<uint32_t*>(x->load_bad), 2, 0xffffffffu,
+                                 x->stream));
+  HIPCHK(x, pbf::launch_load_check(*x, dx, v ? dv : nullptr, (uint32_t)n, x->load_bad));
+  HIPCHK(x, hipMemcpyAsync(x->flag_host, x->load_bad, sizeof(unsigned long long),
+                           hipMemcpyDeviceToHost, x->stream));
+  HIPCHK(x, hipStreamSynchronize(x->stream));
+  unsigned long long bad;
+  memcpy(&bad, x->flag_host, sizeof bad);
+  *code = bad == ~0ull ? PBF_OK : (bad & 1ull) ? PBF_ERR_OUT_OF_BOX : PBF_ERR_INVALID;
+  *first = (int64_t)(bad >> 1);
+  return PBF_OK;
+}
+
 // pbf_load, with the last densities (rho, may be NULL) restored as well.
 int load_impl(Ctx* x, const float* xyz, const float* v, const float* rho, int64_t n) {
   if (!xyz || n < 1) return fail(x, PBF_ERR_INVALID, "xyz must be non-NULL and n >= 1");
@@ -731,42 +791,58 @@ int load_impl(Ctx* x, const float* xyz, const float* v, const float* rho, int64_
       return fail(x, PBF_ERR_INVALID,
                   "n = " + std::to_string(n) + " but the scenes hold " + std::to_string(tot));
   }
-  // Validate every particle against its scene box and pack the float4
-  // records (host threads; the first failure a sequential pass would meet).
-  std::vector<float> boxes;
-  for (const SceneGrid& g : x->grids) {
-    boxes.insert(boxes.end(), g.lo, g.lo + 3);
-    boxes.insert(boxes.end(), g.hi, g.hi + 3);
-  }
+  HIPCHK(x, hipSetDevice(x->device));
+  // Small loads are checked and packed on the host; larger ones travel as
+  // they are (24 bytes per particle instead of 36) and the device checks and
+  // packs them.
+  const bool on_device = n >= kLoadDeviceMin;
   host::Packed pk;
-  host::validate_pack(xyz, v, rho, n, x->offsets, boxes, 8, &pk);
-  if (pk.code == PBF_ERR_INVALID)
-    return fail(x, PBF_ERR_INVALID, "particle " + std::to_string(pk.first) + " is not finite");
-  if (pk.code == PBF_ERR_OUT_OF_BOX)
+  int code = PBF_OK;
+  int64_t bad = 0;
+  if (on_device) {
+    const int rc = load_check(x, xyz, v, rho, n, &code, &bad);
+    if (rc != PBF_OK) return rc;
+  } else {
+    std::vector<float> boxes;
+    for (const SceneGrid& g : x->grids) {
+      boxes.insert(boxes.end(), g.lo, g.lo + 3);
+      boxes.insert(boxes.end(), g.hi, g.hi + 3);
+    }
+    host::validate_pack(xyz, v, rho, n, x->offsets, boxes, 8, &pk);
+    code = pk.code;
+    bad = pk.first;
+  }
+  if (code == PBF_ERR_INVALID)
+    return fail(x, PBF_ERR_INVALID, "particle " + std::to_string(bad) + " is not finite");
+  if (code == PBF_ERR_OUT_OF_BOX)
     return fail(x, PBF_ERR_OUT_OF_BOX,
-                "particle " + std::to_string(pk.first) + " lies outside the collision box");
+                "particle " + std::to_string(bad) + " lies outside the collision box");
   // The input is accepted.  From here on the device buffers are replaced or
   // overwritten, so the context counts as unloaded until every upload has
   // succeeded: after a failed allocation or copy, pbf_step and pbf_read
   // return PBF_ERR_STATE instead of running on freed or partial buffers.
-  HIPCHK(x, hipSetDevice(x->device));
   x->loaded = false;
   x->has_nbrs = false;
   x->field_ready = false;
-  drop_graph(x);
   if (x->nscenes == 1) x->counts[0] = n;
   x->n = n;
   x->npad = (n + 63) / 64 * 64;
   int rc = ensure_device(x);
   if (rc != PBF_OK) return rc;
   pbf::DevState& d = x->d;
-  HIPCHK(x, hipMemcpyAsync(d.posA, pk.pos.data(), (size_t)n * sizeof(float4),
-                           hipMemcpyHostToDevice, x->stream));
-  HIPCHK(x, hipMemcpyAsync(d.velA, pk.vel.data(), (size_t)n * sizeof(float4),
-                           hipMemcpyHostToDevice, x->stream));
+  if (on_device) {
+    const size_t m = (size_t)n * 3;
+    HIPCHK(x, pbf::launch_load_pack(*x, x->load_dev, v ? x->load_dev + m : nullptr,
+                                    rho ? x->load_dev + 2 * m : nullptr));
+  } else {
+    HIPCHK(x, hipMemcpyAsync(d.posA, pk.pos.data(), (size_t)n * sizeof(float4),
+                             hipMemcpyHostToDevice, x->stream));
+    HIPCHK(x, hipMemcpyAsync(d.velA, pk.vel.data(), (size_t)n * sizeof(float4),
+                             hipMemcpyHostToDevice, x->stream));
+    HIPCHK(x, hipMemcpyAsync(d.slotScene, pk.slot_scene.data(), (size_t)n * sizeof(uint32_t),
+                             hipMemcpyHostToDevice, x->stream));
+  }
   HIPCHK(x, hipMemcpyAsync(d.grids, x->grids.data(), x->grids.size() * sizeof(SceneGrid),
-                           hipMemcpyHostToDevice, x->stream));
-  HIPCHK(x, hipMemcpyAsync(d.slotScene, pk.slot_scene.data(), (size_t)n * sizeof(uint32_t),
                            hipMemcpyHostToDevice, x->stream));
   // Scene runs for the persistent schedule, largest first (longest
   // processing time first balances the workgroups).
@@ -783,7 +859,6 @@ int load_impl(Ctx* x, const float* xyz, const float* v, const float* rho, int64_
                            hipMemcpyHostToDevice, x->stream));
   HIPCHK(x, pbf::launch_fill_u32(d.flags, 64, 0u, x->stream));
   HIPCHK(x, hipStreamSynchronize(x->stream));
-  drop_graph(x);
   x->sim_time = 0.0;
   x->loaded = true;
   x->debug_dirty = false;

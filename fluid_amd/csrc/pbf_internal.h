@@ -65,6 +65,7 @@ struct DevState {
   uint32_t* flags = nullptr;      // [0] max neighbour count seen beyond K
   SceneGrid* grids = nullptr;     // per-scene grids (multi-scene)
   uint32_t* slotScene = nullptr;  // scene of each sorted slot (multi-scene)
+  uint32_t* first = nullptr;      // first particle of each scene
   SceneRun* runs = nullptr;       // scenes, largest first (persistent schedule)
   float* stage = nullptr;         // read-back staging, n * 4 floats
   float4* meshTri = nullptr;      // collider triangles, 6 float4 each (pbf_device.h MeshView)
@@ -208,6 +209,11 @@ struct Ctx {
   size_t field_pts_cap = 0;          // points
   float* stage_host[2] = {nullptr, nullptr};
   hipEvent_t stage_ev[2] = {nullptr, nullptr};
+  // Raw xyz, v and rho of a load on their way to the packed arrays, and the
+  // first particle that failed its check (kept between loads).
+  float* load_dev = nullptr;
+  size_t load_cap = 0;               // floats
+  unsigned long long* load_bad = nullptr;
   uint32_t* flag_host = nullptr;     // pinned word the per-call overflow check reads into
   hipGraph_t graph = nullptr;        // captured step (PBF_SCHED_GRAPH)
   hipGraphExec_t graph_exec = nullptr;
@@ -261,6 +267,11 @@ hipError_t launch_vort_commit(Ctx& x, const SimConst& c, const float4* in);
 // Vorticity and commit fused with the next step's prediction (zeroes the
 // histogram first); the next step then starts at the scan.
 hipError_t launch_vort_commit_predict(Ctx& x, const SimConst& c, const float4* in);
+// A load on the device: the check of uploaded xyz and v (v may be NULL)
+// against the scene boxes, and the packing into posA, velA and slotScene.
+hipError_t launch_load_check(Ctx& x, const float* xyz, const float* v, uint32_t n,
+                             unsigned long long* bad);
+hipError_t launch_load_pack(Ctx& x, const float* xyz, const float* v, const float* rho);
 hipError_t launch_unpermute(Ctx& x, const float4* ids, const float4* src, int first, int count,
                             float* dst);
 hipError_t launch_unpermute_u32(Ctx& x, const float4* ids, const uint32_t* src, uint32_t* dst);

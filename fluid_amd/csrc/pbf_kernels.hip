@@ -624,7 +624,7 @@ __device__ __forceinline__ float3* xv_record(const Dev& d, uint32_t i) {
   return reinterpret_cast<float3*>(d.xv) + 2 * (size_t)i;
 }
 
-template <bool LAST>
+template <bool LAST, bool FREE = false>
 __device__ __forceinline__ void deltap_finish(uint32_t i, const Dev& d, const SimConst& c,
                                               const SceneGrid& g, const float4& xi, float dx,
                                               float dy, float dz);
@@ -656,7 +656,7 @@ __device__ __forceinline__ void deltap_one(uint32_t i, const Dev& d, const SimCo
 // The end of newtonStepUpdatePosition from the summed correction: scale by
 // 1/rho0, clamp (src/particles.cpp:51-84), and store x* (and, in the last
 // iteration, v = (x* - x)/dt).
-template <bool LAST>
+template <bool LAST, bool FREE>
 __device__ __forceinline__ void deltap_finish(uint32_t i, const Dev& d, const SimConst& c,
                                               const SceneGrid& g, const float4& xi, float dx,
                                               float dy, float dz) {
@@ -664,7 +664,7 @@ __device__ __forceinline__ void deltap_finish(uint32_t i, const Dev& d, const Si
   dy = dy * c.inv_rho0;
   dz = dz * c.inv_rho0;
   const float3 p =
-      clamp_dp(g, c, d.mesh, make_float3(xi.x, xi.y, xi.z), make_float3(dx, dy, dz));
+      clamp_dp<FREE>(g, c, d.mesh, make_float3(xi.x, xi.y, xi.z), make_float3(dx, dy, dz));
   if (!LAST) {
     // The next λ pass reads x* from the 12-byte records only (this pass
     // gathers from its input x*).
@@ -1600,6 +1600,66 @@ __global__ __launch_bounds__(kSortSmallBlock) void k_sort_small(Dev d, const flo
   for (uint32_t k = threadIdx.x; k < ncell; k += kSortSmallBlock) d.cellCount[k] = 0u;
 }
 
+// ----------------------------------------------------------------- load --
+// Scene of particle i: the last whose first particle is not after i.
+template <bool MULTI>
+__device__ __forceinline__ uint32_t scene_of(uint32_t i, const uint32_t* __restrict__ first,
+                                             uint32_t nscenes) {
+  uint32_t lo = 0;
+  if (MULTI)
+    for (uint32_t hi = nscenes; hi - lo > 1u;) {
+      const uint32_t mid = (lo + hi) >> 1;
+      if (first[mid] <= i)
+        lo = mid;
+      else
+        hi = mid;
+    }
+  return lo;
+}
+
+// The checks of host::validate_pack on uploaded xyz and v: *bad becomes the
+// smallest (particle << 1 | outside the box) of the particles that fail, an
+// axis at a time, non-finite before outside.
+template <bool MULTI>
+__global__ __launch_bounds__(kBlock) void k_load_check(const float* __restrict__ xyz,
+                                                       const float* __restrict__ v, uint32_t n,
+                                                       const SceneGrid* __restrict__ grids,
+                                                       const uint32_t* __restrict__ first,
+                                                       uint32_t nscenes, SceneGrid g0,
+                                                       unsigned long long* __restrict__ bad) {
+  const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+  if (i >= n) return;
+  const SceneGrid* g = MULTI ? grids + scene_of<MULTI>(i, first, nscenes) : &g0;
+  int code = -1;
+#pragma unroll
+  for (int a = 2; a >= 0; a--) {
+    const float p = xyz[3 * (size_t)i + a], q = v ? v[3 * (size_t)i + a] : 0.0f;
+    if (!isfinite(p) || !isfinite(q))
+      code = 0;
+    else if (p < g->lo[a] || p > g->hi[a])
+      code = 1;
+  }
+  if (code >= 0) atomicMin(bad, ((unsigned long long)i << 1) | (unsigned long long)code);
+}
+
+// posA = (x, load id), velA = (v, rho), slotScene (v, rho may be NULL: zero).
+template <bool MULTI>
+__global__ __launch_bounds__(kBlock) void k_load_pack(const float* __restrict__ xyz,
+                                                      const float* __restrict__ v,
+                                                      const float* __restrict__ rho, uint32_t n,
+                                                      const uint32_t* __restrict__ first,
+                                                      uint32_t nscenes, float4* __restrict__ pos,
+                                                      float4* __restrict__ vel,
+                                                      uint32_t* __restrict__ scene) {
+  const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+  if (i >= n) return;
+  const size_t k = 3 * (size_t)i;
+  pos[i] = make_float4(xyz[k], xyz[k + 1], xyz[k + 2], __uint_as_float(i));
+  const float r = rho ? rho[i] : 0.0f;
+  vel[i] = v ? make_float4(v[k], v[k + 1], v[k + 2], r) : make_float4(0.0f, 0.0f, 0.0f, r);
+  scene[i] = scene_of<MULTI>(i, first, nscenes);
+}
+
 // ------------------------------------------------------------ read-back --
 __global__ __launch_bounds__(kBlock) void k_unpermute(uint32_t n, const float4* __restrict__ ids,
                                                       const float4* __restrict__ src, int first,
@@ -1709,6 +1769,28 @@ hipError_t launch_scan_u32(uint32_t* in, uint32_t* out, uint32_t n, uint32_t* pa
 
 
 static bool multi(const Ctx& x) { return x.nscenes > 1; }
+
+hipError_t launch_load_check(Ctx& x, const float* xyz, const float* v, uint32_t n,
+                             unsigned long long* bad) {
+  if (multi(x))
+    k_load_check<true><<<blocks_for(n), kBlock, 0, x.stream>>>(
+        xyz, v, n, x.d.grids, x.d.first, (uint32_t)x.nscenes, x.grids[0], bad);
+  else
+    k_load_check<false><<<blocks_for(n), kBlock, 0, x.stream>>>(xyz, v, n, nullptr, nullptr, 1u,
+                                                                x.grids[0], bad);
+  return hipGetLastError();
+}
+
+hipError_t launch_load_pack(Ctx& x, const float* xyz, const float* v, const float* rho) {
+  const uint32_t n = (uint32_t)x.n;
+  if (multi(x))
+    k_load_pack<true><<<blocks_for(n), kBlock, 0, x.stream>>>(
+        xyz, v, rho, n, x.d.first, (uint32_t)x.nscenes, x.d.posA, x.d.velA, x.d.slotScene);
+  else
+    k_load_pack<false><<<blocks_for(n), kBlock, 0, x.stream>>>(xyz, v, rho, n, nullptr, 1u,
+                                                               x.d.posA, x.d.velA, x.d.slotScene);
+  return hipGetLastError();
+}
 
 hipError_t launch_predict(Ctx& x, const SimConst& c) {
   hipError_t e = launch_fill_u32(x.d.cellCount, x.ncell, 0u, x.stream);
