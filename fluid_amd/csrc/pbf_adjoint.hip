@@ -62,24 +62,39 @@ struct Pair {
   float dphi;   // phi' / |r|  (H = phi I + dphi r r^T)
 };
 
+// n / z.  FAST: from z's reciprocal, the quotient corrected once by its
+// residual; an overflowed quotient is left as it is.
+template <bool FAST>
+__device__ __forceinline__ float quot(float n, float z) {
+  if (!FAST) return n / z;
+  const float y = rcp_seq(z);
+  const float q = n * y;
+  const float r = fmaf(fmaf(-q, z, n), y, q);
+  return fabsf(q) < INFINITY ? r : q;
+}
+
+// FAST (see adj_fast): the verified short square root and division by h^9,
+// and quot()'s reciprocal, in place of the compiler's expansions.
+template <bool FAST>
 __device__ __forceinline__ Pair pair_of(const SimConst& c, float3 xi, float3 xj) {
   Pair p;
   p.r = xi - xj;
   const float r2 = dot3(p.r, p.r);
-  p.rl = sqrtf(r2);
+  p.rl = FAST ? sqrt_rn(r2) : sqrtf(r2);
   if (r2 < c.h2) {
     const float t = c.h2 - r2;
-    p.W = c.c1 * t * t * t / c.h9;
-    p.gP = (-6.0f * c.c1 * t * t / c.h9) * p.r;
+    const float w = c.c1 * t * t * t, g = -6.0f * c.c1 * t * t;
+    p.W = FAST ? div_seq(w, c.h9, c.r9) : w / c.h9;
+    p.gP = (FAST ? div_seq(g, c.h9, c.r9) : g / c.h9) * p.r;
   } else {
     p.W = 0.0f;
     p.gP = make_float3(0.f, 0.f, 0.f);
   }
   if (p.rl < c.h && p.rl >= c.eps_d) {
     const float q = c.h - p.rl;
-    p.phi = c.m3c2 * q * q / (c.h6 * p.rl);
+    p.phi = quot<FAST>(c.m3c2 * q * q, c.h6 * p.rl);
     // phi'(rho) = -m3c2/h^6 (h - rho)(h + rho)/rho^2
-    p.dphi = (-c.m3c2 / c.h6) * q * (c.h + p.rl) / (r2 * p.rl);
+    p.dphi = quot<FAST>((-c.m3c2 / c.h6) * q * (c.h + p.rl), r2 * p.rl);
     p.g = p.phi * p.r;
   } else {
     p.phi = 0.0f;
@@ -104,24 +119,29 @@ struct AdjDev {
 __device__ __forceinline__ uint32_t idx() { return blockIdx.x * kB + threadIdx.x; }
 
 // The adjoint's neighbour passes can give each particle L consecutive lanes
-// (L = 1, 2, 4): lane q of particle i visits the chunks ch = q, q + L, ...
-// of its list (and the partial last chunk if it falls to q) and the L
-// partial sums are added with a fixed butterfly, so the result is the same
-// on every run.  Small scenes use L = 4 to put four times as many waves on
-// the chip; a lane's sums then hold a quarter of the terms.
-template <int L, class Body>
-__device__ __forceinline__ void nbrs_split(const AdjDev& a, uint32_t i, int q, Body body) {
+// (L = 1, 2, 4, 16): lane q of particle i visits the chunks ch = q, q + L, ...
+// of its list and the L partial sums are added with a fixed butterfly, so
+// the result is the same on every run.  The passes wait for memory: a lane's
+// chain is index chunk -> gathers -> sum, so the four entries of a chunk
+// are gathered together (load) before the first is used (body), and past the
+// list's end i stands in (gathered, not used).  With the short sequences:
+// k_adj_pos 15.3 -> 10.5 us and k_adj_lambda 9.9 -> 7.0 at 32,768 particles
+// (4 lanes), 15 -> 4.9 and 10 -> 4.4 at 1,000 (16 lanes, 4 before).
+template <int L, class Load, class Body>
+__device__ __forceinline__ void nbrs_split(const AdjDev& a, uint32_t i, int q, Load load,
+                                           Body body) {
   const int cnt = (int)a.ncnt[i];
-  const int nfull = cnt >> 2;
-  for (int ch = q; ch < nfull; ch += L) {
+  const int nch = (cnt + 3) >> 2;
+  for (int ch = q; ch < nch; ch += L) {
     const uint4 e = *reinterpret_cast<const uint4*>(a.nbr + nbr_chunk(i, ch, a.K4));
-    body(e.x);
-    body(e.y);
-    body(e.z);
-    body(e.w);
+    const int m = cnt - 4 * ch;  // entries of this chunk, at least one
+    const auto r0 = load(e.x), r1 = load(m > 1 ? e.y : i);
+    const auto r2 = load(m > 2 ? e.z : i), r3 = load(m > 3 ? e.w : i);
+    body(r0);
+    if (m > 1) body(r1);
+    if (m > 2) body(r2);
+    if (m > 3) body(r3);
   }
-  if (q == nfull % L)
-    for (int k = nfull * 4; k < cnt; k++) body(a.nbr[nbr_slot(i, k, a.K4)]);
 }
 
 // Sum over the L lanes of a particle (every lane gets the same value:
@@ -196,7 +216,7 @@ __global__ __launch_bounds__(kB) void k_copy4(uint32_t n, const float4* __restri
 
 // Vorticity confinement, part 1: eta_bar and the direct part of w_bar.
 // xw = (x*_S, |w|), w = (w, .), vb4 = dL/dv_new.
-template <int L>
+template <int L, bool FAST>
 __global__ __launch_bounds__(kB) void k_adj_vort_a(AdjDev a, SimConst c,
                                                    const float4* __restrict__ xw,
                                                    const float4* __restrict__ w,
@@ -208,9 +228,9 @@ __global__ __launch_bounds__(kB) void k_adj_vort_a(AdjDev a, SimConst c,
   if (i >= a.n) return;
   const float3 xi = f3(xw[i]);
   float3 eta = make_float3(0.f, 0.f, 0.f);
-  nbrs_split<L>(a, i, lq, [&](uint32_t j) {
-    const float4 q = xw[j];
-    const Pair p = pair_of(c, xi, f3(q));
+  const auto load = [&](uint32_t j) { return xw[j]; };
+  nbrs_split<L>(a, i, lq, load, [&](const float4& q) {
+    const Pair p = pair_of<FAST>(c, xi, f3(q));
     eta = eta + q.w * p.g;
   });
   eta = lane_sum<L>(eta);
@@ -233,7 +253,7 @@ __global__ __launch_bounds__(kB) void k_adj_vort_a(AdjDev a, SimConst c,
 // Vorticity confinement, part 2: w_bar through |w_j| in eta_j, and x*_bar
 // through g in eta: H_ij (|w_j| eta_bar_i - |w_i| eta_bar_j).  xs_acc starts
 // from dL/dx_new (x_new = x*_S).
-template <int L>
+template <int L, bool FAST>
 __global__ __launch_bounds__(kB) void k_adj_vort_b(AdjDev a, SimConst c,
                                                    const float4* __restrict__ xw,
                                                    const float4* __restrict__ w,
@@ -250,10 +270,12 @@ __global__ __launch_bounds__(kB) void k_adj_vort_b(AdjDev a, SimConst c,
   const float3 ebi = f3(etabar[i]);
   float s = 0.0f;
   float3 xs = make_float3(0.f, 0.f, 0.f);
-  nbrs_split<L>(a, i, lq, [&](uint32_t j) {
-    const float4 q = xw[j];
-    const Pair p = pair_of(c, xi, f3(q));
-    const float3 ebj = f3(etabar[j]);
+  struct Rec { float4 q, eb; };
+  const auto load = [&](uint32_t j) { return Rec{xw[j], etabar[j]}; };
+  nbrs_split<L>(a, i, lq, load, [&](const Rec& n) {
+    const float4 q = n.q;
+    const Pair p = pair_of<FAST>(c, xi, f3(q));
+    const float3 ebj = f3(n.eb);
     s = s - dot3(ebj, p.g);
     xs = xs + hess(p, q.w * ebi - wn * ebj);
   });
@@ -269,7 +291,7 @@ __global__ __launch_bounds__(kB) void k_adj_vort_b(AdjDev a, SimConst c,
 
 // XSPH and vorticity: v2_bar and x*_bar; then v2 = (x*_S - x)/dt.
 // ybar = x*_S bar (all terms), xstart = -v2_bar/dt (the x part of v2).
-template <int L>
+template <int L, bool FAST>
 __global__ __launch_bounds__(kB) void k_adj_xsph(AdjDev a, SimConst c,
                                                  const float4* __restrict__ xs,
                                                  const float4* __restrict__ v2,
@@ -288,11 +310,13 @@ __global__ __launch_bounds__(kB) void k_adj_xsph(AdjDev a, SimConst c,
   const float3 wi = f3(wbar[i]);
   float3 v2b = make_float3(0.f, 0.f, 0.f);
   float3 xb = make_float3(0.f, 0.f, 0.f);
-  nbrs_split<L>(a, i, lq, [&](uint32_t j) {
-    const Pair p = pair_of(c, xi, f3(xs[j]));
-    const float3 u = f3(v2[j]) - vi;
-    const float3 bj = f3(vb3[j]);
-    const float3 ws = wi + f3(wbar[j]);
+  struct Rec { float4 x, v, b, w; };
+  const auto load = [&](uint32_t j) { return Rec{xs[j], v2[j], vb3[j], wbar[j]}; };
+  nbrs_split<L>(a, i, lq, load, [&](const Rec& n) {
+    const Pair p = pair_of<FAST>(c, xi, f3(n.x));
+    const float3 u = f3(n.v) - vi;
+    const float3 bj = f3(n.b);
+    const float3 ws = wi + f3(n.w);
     v2b = v2b + (c.xc * p.W) * (bj - bi) - cross3(p.g, ws);
     xb = xb + (c.xc * dot3(u, bi - bj)) * p.gP + hess(p, cross3(ws, u));
   });
@@ -311,13 +335,16 @@ __global__ __launch_bounds__(kB) void k_adj_xsph(AdjDev a, SimConst c,
 // Solver iteration m, part 1: recompute rho, G, D, lambda at x*_m and
 // lambda_bar = sum_j g_ij . (e_i - e_j), e = ybar / rho0; then
 // C_bar = -lambda_bar/(D+eps), D_bar = -lambda_bar lambda/(D+eps),
-// rho_bar = C_bar/rho0.  aux = (lambda, rho_bar, D_bar, .), Gb = (G, .).
-template <int L>
+// rho_bar = C_bar/rho0.  What part 2 gathers per neighbour goes into three
+// full records, xl = (x*, lambda), er = (e, rho_bar), dg = (D_bar G, D_bar)
+// (four half-used ones before: 64 bytes instead of 48 per neighbour).
+template <int L, bool FAST>
 __global__ __launch_bounds__(kB) void k_adj_lambda(AdjDev a, SimConst c,
                                                    const float4* __restrict__ xs,
                                                    const float4* __restrict__ ybar,
-                                                   float4* __restrict__ aux,
-                                                   float4* __restrict__ Gb,
+                                                   float4* __restrict__ xl,
+                                                   float4* __restrict__ er,
+                                                   float4* __restrict__ dg,
                                                    uint32_t* __restrict__ contacts, SceneGrid g) {
   const uint32_t i = idx() / L;
   const int lq = (int)(idx() % L);
@@ -326,13 +353,15 @@ __global__ __launch_bounds__(kB) void k_adj_lambda(AdjDev a, SimConst c,
   const float3 ei = c.inv_rho0 * f3(ybar[i]);
   float rho = 0.f, D = 0.f, lb = 0.f;
   float3 G = make_float3(0.f, 0.f, 0.f);
-  nbrs_split<L>(a, i, lq, [&](uint32_t j) {
-    const Pair p = pair_of(c, xi, f3(xs[j]));
+  struct Rec { float4 x, y; };
+  const auto load = [&](uint32_t j) { return Rec{xs[j], ybar[j]}; };
+  nbrs_split<L>(a, i, lq, load, [&](const Rec& n) {
+    const Pair p = pair_of<FAST>(c, xi, f3(n.x));
     rho = rho + p.W;
     const float3 gs = c.inv_rho0 * p.g;
     G = G + gs;
     D = D + dot3(gs, gs);
-    lb = lb + dot3(p.g, ei - c.inv_rho0 * f3(ybar[j]));
+    lb = lb + dot3(p.g, ei - c.inv_rho0 * f3(n.y));
   });
   rho = lane_sum<L>(rho);
   G = lane_sum<L>(G);
@@ -344,8 +373,9 @@ __global__ __launch_bounds__(kB) void k_adj_lambda(AdjDev a, SimConst c,
   const float lam = -C / (D + c.eps);
   const float Cb = -lb / (D + c.eps);
   const float Db = -lb * lam / (D + c.eps);
-  aux[i] = make_float4(lam, Cb * c.inv_rho0, Db, 0.f);
-  Gb[i] = make_float4(G.x, G.y, G.z, 0.f);
+  xl[i] = make_float4(xi.x, xi.y, xi.z, lam);
+  er[i] = make_float4(ei.x, ei.y, ei.z, Cb * c.inv_rho0);
+  dg[i] = make_float4(Db * G.x, Db * G.y, Db * G.z, Db);
   if (xi.x <= g.lo_e[0] || xi.y <= g.lo_e[1] || xi.z <= g.lo_e[2] || xi.x >= g.hi_e[0] ||
       xi.y >= g.hi_e[1] || xi.z >= g.hi_e[2])
     atomicAdd(contacts, 1u);
@@ -358,37 +388,35 @@ __global__ __launch_bounds__(kB) void k_adj_lambda(AdjDev a, SimConst c,
 //   + (rho_bar_i + rho_bar_j) gP                 (W in rho)
 //   + H [2 (D_bar_i + D_bar_j) g/rho0^2 + 2 (D_bar_i G_i - D_bar_j G_j)/rho0]  (g in D)
 // and dL/dk += sum_j (e_i . g_ij) (-(W S)^n).
-template <int L>
+template <int L, bool FAST>
 __global__ __launch_bounds__(kB) void k_adj_pos(AdjDev a, SimConst c,
-                                                const float4* __restrict__ xs,
+                                                const float4* __restrict__ xl,
+                                                const float4* __restrict__ er,
+                                                const float4* __restrict__ dg,
                                                 const float4* __restrict__ ybar,
-                                                const float4* __restrict__ aux,
-                                                const float4* __restrict__ Gb,
                                                 float4* __restrict__ ynext,
                                                 double* __restrict__ kpart) {
   const uint32_t i = idx() / L;
   const int lq = (int)(idx() % L);
   if (i >= a.n) return;
-  const float3 xi = f3(xs[i]);
-  const float3 ei = c.inv_rho0 * f3(ybar[i]);
-  const float4 ai = aux[i];
-  const float3 Gi = f3(Gb[i]);
+  const float4 xi4 = xl[i], ei4 = er[i], di4 = dg[i];
+  const float3 xi = f3(xi4), ei = f3(ei4), di = f3(di4);
   const float r02 = c.inv_rho0 * c.inv_rho0;
   float3 acc = make_float3(0.f, 0.f, 0.f);
   float kp = 0.f;
-  nbrs_split<L>(a, i, lq, [&](uint32_t j) {
-    const Pair p = pair_of(c, xi, f3(xs[j]));
-    const float3 ej = c.inv_rho0 * f3(ybar[j]);
-    const float4 aj = aux[j];
-    const float3 de = ei - ej;
+  struct Rec { float4 x, e, d; };
+  const auto load = [&](uint32_t j) { return Rec{xl[j], er[j], dg[j]}; };
+  nbrs_split<L>(a, i, lq, load, [&](const Rec& n) {
+    const float4 xj = n.x, ej = n.e, dj = n.d;
+    const Pair p = pair_of<FAST>(c, xi, f3(xj));
+    const float3 de = ei - f3(ej);
     const float ws = p.W * c.S;
-    const float pw = ipow(ws, c.n_tensile);
+    const float pw1 = ipow(ws, c.n_tensile - 1), pw = c.n_tensile > 0 ? pw1 * ws : 1.0f;
     const float s = c.negk * pw;
-    const float sd = c.n_tensile > 0 ? c.negk * (float)c.n_tensile * c.S * ipow(ws, c.n_tensile - 1)
-                                     : 0.0f;
-    const float3 hv = (ai.x + aj.x + s) * de + (2.0f * (ai.z + aj.z) * r02) * p.g +
-                      (2.0f * c.inv_rho0) * (ai.z * Gi - aj.z * f3(Gb[j]));
-    acc = acc + hess(p, hv) + (sd * dot3(de, p.g) + ai.y + aj.y) * p.gP;
+    const float sd = c.n_tensile > 0 ? c.negk * (float)c.n_tensile * c.S * pw1 : 0.0f;
+    const float3 hv = (xi4.w + xj.w + s) * de + (2.0f * (di4.w + dj.w) * r02) * p.g +
+                      (2.0f * c.inv_rho0) * (di - f3(dj));
+    acc = acc + hess(p, hv) + (sd * dot3(de, p.g) + ei4.w + ej.w) * p.gP;
     kp = kp + dot3(ei, p.g) * (-pw);
   });
   acc = lane_sum<L>(acc);
@@ -602,7 +630,7 @@ int forward_step(pbf_adj* a, const pbf::SimConst& k, AdjTape* slot) {
 // lanes per particle in the neighbour passes.
 // xbar/vbar (load order) hold dL/d(state after the step) on entry and
 // dL/d(state before the step) on exit; ksteps[t] receives this step's dL/dk.
-template <int L>
+template <int L, bool FAST>
 int backward_step_l(pbf_adj* a, const pbf::SimConst& k, int t, const AdjTape& T) {
   pbf::Ctx* c = X(a);
   const uint32_t n = (uint32_t)a->n;
@@ -614,18 +642,20 @@ int backward_step_l(pbf_adj* a, const pbf::SimConst& k, int t, const AdjTape& T)
   const pbf::SceneGrid g = c->grids[0];
   // dL/dv_new and dL/dx_new in sorted order.
   pbf::k_from_id2<<<nb, pbf::kB, 0, s>>>(n, d.posB, a->vbar, a->vb3, a->xbar, a->xbn);
-  pbf::k_adj_vort_a<L><<<nbl, pbf::kB, 0, s>>>(ad, k, d.predP, d.vort, a->vb3, a->etab, a->wb);
-  pbf::k_adj_vort_b<L><<<nbl, pbf::kB, 0, s>>>(ad, k, d.predP, d.vort, a->etab, a->wb, a->xbn,
+  pbf::k_adj_vort_a<L, FAST><<<nbl, pbf::kB, 0, s>>>(ad, k, d.predP, d.vort, a->vb3, a->etab, a->wb);
+  pbf::k_adj_vort_b<L, FAST><<<nbl, pbf::kB, 0, s>>>(ad, k, d.predP, d.vort, a->etab, a->wb, a->xbn,
                                               a->xsacc);
-  pbf::k_adj_xsph<L><<<nbl, pbf::kB, 0, s>>>(ad, k, d.predQ, d.velB, a->vb3, a->wb, a->xsacc,
+  pbf::k_adj_xsph<L, FAST><<<nbl, pbf::kB, 0, s>>>(ad, k, d.predQ, d.velB, a->vb3, a->wb, a->xsacc,
                                             a->yb, a->xst, a->contacts, g);
   AHIP(a, hipGetLastError());
   const int S = c->p.iterations;
   for (int it = S - 1; it >= 0; it--) {
     const float4* xs = d.stash + (size_t)it * np;
-    pbf::k_adj_lambda<L><<<nbl, pbf::kB, 0, s>>>(ad, k, xs, a->yb, a->aux, a->Gb, a->contacts, g);
-    pbf::k_adj_pos<L><<<nbl, pbf::kB, 0, s>>>(ad, k, xs, a->yb, a->aux, a->Gb, a->yb2,
-                                             a->kpart + (size_t)it * np);
+    // etab is free again: it holds the (x*, lambda) records.
+    pbf::k_adj_lambda<L, FAST><<<nbl, pbf::kB, 0, s>>>(ad, k, xs, a->yb, a->etab, a->aux, a->Gb,
+                                                       a->contacts, g);
+    pbf::k_adj_pos<L, FAST><<<nbl, pbf::kB, 0, s>>>(ad, k, a->etab, a->aux, a->Gb, a->yb, a->yb2,
+                                                    a->kpart + (size_t)it * np);
     AHIP(a, hipGetLastError());
     std::swap(a->yb, a->yb2);
   }
@@ -638,11 +668,26 @@ int backward_step_l(pbf_adj* a, const pbf::SimConst& k, int t, const AdjTape& T)
   return PBF_OK;
 }
 
+constexpr int64_t kAdjWideMax = 16384;  // up to here, sixteen lanes per particle
+
+// Whether the adjoint passes can take the short sequences: verified on the
+// device, and every argument in their ranges (the poly6 gradient's numerator
+// 6 c1 t^2 in the division's, |r|^3 and h^6 |r| in the reciprocal's).
+bool adj_fast(const pbf::SimConst& k) {
+  const float tmin = k.h2 - nextafterf(k.h2, 0.0f), lo = 6.0f * k.c1 * tmin * tmin;
+  const float e = k.eps_d, cube = e * e * e;
+  return k.fast_div && k.fast_rcp && k.fast_sqrt && lo >= k.c1 * ((tmin * tmin) * tmin) &&
+         lo >= 0x1p-120f && 6.0f * k.c1 * k.h2 * k.h2 < k.div_hi && e >= 0x1p-40f &&
+         cube >= 0x1p-124f && k.h2 * k.h < 0x1p100f;
+}
+
 int backward_step(pbf_adj* a, const pbf::SimConst& k, int t, const AdjTape& T) {
+  const bool fast = adj_fast(k);
   switch (a->lanes) {
-    case 4: return backward_step_l<4>(a, k, t, T);
-    case 2: return backward_step_l<2>(a, k, t, T);
-    default: return backward_step_l<1>(a, k, t, T);
+    case 16: return fast ? backward_step_l<16, true>(a, k, t, T) : backward_step_l<16, false>(a, k, t, T);
+    case 4: return fast ? backward_step_l<4, true>(a, k, t, T) : backward_step_l<4, false>(a, k, t, T);
+    case 2: return fast ? backward_step_l<2, true>(a, k, t, T) : backward_step_l<2, false>(a, k, t, T);
+    default: return fast ? backward_step_l<1, true>(a, k, t, T) : backward_step_l<1, false>(a, k, t, T);
   }
 }
 
@@ -667,12 +712,14 @@ static int pbf_adj_create_impl(const pbf_params* p, int64_t n, int32_t nsteps, i
   a->npad = (n + 63) / 64 * 64;
   // The adjoint reads the lists by particle index: no LDS tiles.
   X(a)->tile_min = INT64_MAX;
-  // Four lanes per particle while that still leaves under ~4M threads
-  // (small scenes are latency-bound); PBF_ADJ_LANES = 1, 2 or 4 overrides.
-  a->lanes = n <= (1 << 20) ? 4 : 1;
+  // Lanes per particle.  Small scenes are latency-bound: sixteen lanes read
+  // most lists in one round (backward of 5 steps, 4 / 16 lanes: 1,000
+  // particles 877 / 734 us, 8,000 1,047 / 939, 32,768 1,237 / 1,335); four
+  // while that still leaves under ~4M threads.  PBF_ADJ_LANES overrides.
+  a->lanes = n <= kAdjWideMax ? 16 : n <= (1 << 20) ? 4 : 1;
   if (const char* e = getenv("PBF_ADJ_LANES")) {
     const int l = atoi(e);
-    if (l == 1 || l == 2 || l == 4) a->lanes = l;
+    if (l == 1 || l == 2 || l == 4 || l == 16) a->lanes = l;
   }
   a->nsteps = nsteps;
   a->every = every;
