@@ -109,12 +109,14 @@ __device__ __forceinline__ float3 hess(const Pair& p, float3 v) {
 }
 
 struct AdjDev {
-  const float4* ids;    // posB: sorted x with ids in w
   const uint32_t* nbr;
   const uint32_t* ncnt;
   int K4;
   uint32_t n;
 };
+// The neighbour passes take it as four scalars, which arrive in SGPRs (a
+// struct does not).
+#define ADJ_LIST_PARAMS const uint32_t *nbr, const uint32_t *ncnt, int K4, uint32_t n
 
 __device__ __forceinline__ uint32_t idx() { return blockIdx.x * kB + threadIdx.x; }
 
@@ -217,12 +219,14 @@ __global__ __launch_bounds__(kB) void k_copy4(uint32_t n, const float4* __restri
 // Vorticity confinement, part 1: eta_bar and the direct part of w_bar.
 // xw = (x*_S, |w|), w = (w, .), vb4 = dL/dv_new.
 template <int L, bool FAST>
-__global__ __launch_bounds__(kB) void k_adj_vort_a(AdjDev a, SimConst c,
+__global__ __launch_bounds__(kB) void k_adj_vort_a(ADJ_LIST_PARAMS,
                                                    const float4* __restrict__ xw,
                                                    const float4* __restrict__ w,
                                                    const float4* __restrict__ vb4,
                                                    float4* __restrict__ etabar,
-                                                   float4* __restrict__ wbar) {
+                                                   float4* __restrict__ wbar,
+                                                   SimConst c) {
+  const AdjDev a{nbr, ncnt, K4, n};
   const uint32_t i = idx() / L;
   const int lq = (int)(idx() % L);
   if (i >= a.n) return;
@@ -254,13 +258,15 @@ __global__ __launch_bounds__(kB) void k_adj_vort_a(AdjDev a, SimConst c,
 // through g in eta: H_ij (|w_j| eta_bar_i - |w_i| eta_bar_j).  xs_acc starts
 // from dL/dx_new (x_new = x*_S).
 template <int L, bool FAST>
-__global__ __launch_bounds__(kB) void k_adj_vort_b(AdjDev a, SimConst c,
+__global__ __launch_bounds__(kB) void k_adj_vort_b(ADJ_LIST_PARAMS,
                                                    const float4* __restrict__ xw,
                                                    const float4* __restrict__ w,
                                                    const float4* __restrict__ etabar,
                                                    float4* __restrict__ wbar,
                                                    const float4* __restrict__ xb_new,
-                                                   float4* __restrict__ xs_acc) {
+                                                   float4* __restrict__ xs_acc,
+                                                   SimConst c) {
+  const AdjDev a{nbr, ncnt, K4, n};
   const uint32_t i = idx() / L;
   const int lq = (int)(idx() % L);
   if (i >= a.n) return;
@@ -272,10 +278,10 @@ __global__ __launch_bounds__(kB) void k_adj_vort_b(AdjDev a, SimConst c,
   float3 xs = make_float3(0.f, 0.f, 0.f);
   struct Rec { float4 q, eb; };
   const auto load = [&](uint32_t j) { return Rec{xw[j], etabar[j]}; };
-  nbrs_split<L>(a, i, lq, load, [&](const Rec& n) {
-    const float4 q = n.q;
+  nbrs_split<L>(a, i, lq, load, [&](const Rec& nb) {
+    const float4 q = nb.q;
     const Pair p = pair_of<FAST>(c, xi, f3(q));
-    const float3 ebj = f3(n.eb);
+    const float3 ebj = f3(nb.eb);
     s = s - dot3(ebj, p.g);
     xs = xs + hess(p, q.w * ebi - wn * ebj);
   });
@@ -292,7 +298,7 @@ __global__ __launch_bounds__(kB) void k_adj_vort_b(AdjDev a, SimConst c,
 // XSPH and vorticity: v2_bar and x*_bar; then v2 = (x*_S - x)/dt.
 // ybar = x*_S bar (all terms), xstart = -v2_bar/dt (the x part of v2).
 template <int L, bool FAST>
-__global__ __launch_bounds__(kB) void k_adj_xsph(AdjDev a, SimConst c,
+__global__ __launch_bounds__(kB) void k_adj_xsph(ADJ_LIST_PARAMS,
                                                  const float4* __restrict__ xs,
                                                  const float4* __restrict__ v2,
                                                  const float4* __restrict__ vb3,
@@ -300,7 +306,9 @@ __global__ __launch_bounds__(kB) void k_adj_xsph(AdjDev a, SimConst c,
                                                  const float4* __restrict__ xs_acc,
                                                  float4* __restrict__ ybar,
                                                  float4* __restrict__ xstart,
-                                                 uint32_t* __restrict__ contacts, SceneGrid g) {
+                                                 uint32_t* __restrict__ contacts,
+                                                 SimConst c, SceneGrid g) {
+  const AdjDev a{nbr, ncnt, K4, n};
   const uint32_t i = idx() / L;
   const int lq = (int)(idx() % L);
   if (i >= a.n) return;
@@ -312,11 +320,11 @@ __global__ __launch_bounds__(kB) void k_adj_xsph(AdjDev a, SimConst c,
   float3 xb = make_float3(0.f, 0.f, 0.f);
   struct Rec { float4 x, v, b, w; };
   const auto load = [&](uint32_t j) { return Rec{xs[j], v2[j], vb3[j], wbar[j]}; };
-  nbrs_split<L>(a, i, lq, load, [&](const Rec& n) {
-    const Pair p = pair_of<FAST>(c, xi, f3(n.x));
-    const float3 u = f3(n.v) - vi;
-    const float3 bj = f3(n.b);
-    const float3 ws = wi + f3(n.w);
+  nbrs_split<L>(a, i, lq, load, [&](const Rec& nb) {
+    const Pair p = pair_of<FAST>(c, xi, f3(nb.x));
+    const float3 u = f3(nb.v) - vi;
+    const float3 bj = f3(nb.b);
+    const float3 ws = wi + f3(nb.w);
     v2b = v2b + (c.xc * p.W) * (bj - bi) - cross3(p.g, ws);
     xb = xb + (c.xc * dot3(u, bi - bj)) * p.gP + hess(p, cross3(ws, u));
   });
@@ -339,13 +347,15 @@ __global__ __launch_bounds__(kB) void k_adj_xsph(AdjDev a, SimConst c,
 // full records, xl = (x*, lambda), er = (e, rho_bar), dg = (D_bar G, D_bar)
 // (four half-used ones before: 64 bytes instead of 48 per neighbour).
 template <int L, bool FAST>
-__global__ __launch_bounds__(kB) void k_adj_lambda(AdjDev a, SimConst c,
+__global__ __launch_bounds__(kB) void k_adj_lambda(ADJ_LIST_PARAMS,
                                                    const float4* __restrict__ xs,
                                                    const float4* __restrict__ ybar,
                                                    float4* __restrict__ xl,
                                                    float4* __restrict__ er,
                                                    float4* __restrict__ dg,
-                                                   uint32_t* __restrict__ contacts, SceneGrid g) {
+                                                   uint32_t* __restrict__ contacts,
+                                                   SimConst c, SceneGrid g) {
+  const AdjDev a{nbr, ncnt, K4, n};
   const uint32_t i = idx() / L;
   const int lq = (int)(idx() % L);
   if (i >= a.n) return;
@@ -355,13 +365,13 @@ __global__ __launch_bounds__(kB) void k_adj_lambda(AdjDev a, SimConst c,
   float3 G = make_float3(0.f, 0.f, 0.f);
   struct Rec { float4 x, y; };
   const auto load = [&](uint32_t j) { return Rec{xs[j], ybar[j]}; };
-  nbrs_split<L>(a, i, lq, load, [&](const Rec& n) {
-    const Pair p = pair_of<FAST>(c, xi, f3(n.x));
+  nbrs_split<L>(a, i, lq, load, [&](const Rec& nb) {
+    const Pair p = pair_of<FAST>(c, xi, f3(nb.x));
     rho = rho + p.W;
     const float3 gs = c.inv_rho0 * p.g;
     G = G + gs;
     D = D + dot3(gs, gs);
-    lb = lb + dot3(p.g, ei - c.inv_rho0 * f3(n.y));
+    lb = lb + dot3(p.g, ei - c.inv_rho0 * f3(nb.y));
   });
   rho = lane_sum<L>(rho);
   G = lane_sum<L>(G);
@@ -389,13 +399,15 @@ __global__ __launch_bounds__(kB) void k_adj_lambda(AdjDev a, SimConst c,
 //   + H [2 (D_bar_i + D_bar_j) g/rho0^2 + 2 (D_bar_i G_i - D_bar_j G_j)/rho0]  (g in D)
 // and dL/dk += sum_j (e_i . g_ij) (-(W S)^n).
 template <int L, bool FAST>
-__global__ __launch_bounds__(kB) void k_adj_pos(AdjDev a, SimConst c,
+__global__ __launch_bounds__(kB) void k_adj_pos(ADJ_LIST_PARAMS,
                                                 const float4* __restrict__ xl,
                                                 const float4* __restrict__ er,
                                                 const float4* __restrict__ dg,
                                                 const float4* __restrict__ ybar,
                                                 float4* __restrict__ ynext,
-                                                double* __restrict__ kpart) {
+                                                double* __restrict__ kpart,
+                                                SimConst c) {
+  const AdjDev a{nbr, ncnt, K4, n};
   const uint32_t i = idx() / L;
   const int lq = (int)(idx() % L);
   if (i >= a.n) return;
@@ -406,8 +418,8 @@ __global__ __launch_bounds__(kB) void k_adj_pos(AdjDev a, SimConst c,
   float kp = 0.f;
   struct Rec { float4 x, e, d; };
   const auto load = [&](uint32_t j) { return Rec{xl[j], er[j], dg[j]}; };
-  nbrs_split<L>(a, i, lq, load, [&](const Rec& n) {
-    const float4 xj = n.x, ej = n.e, dj = n.d;
+  nbrs_split<L>(a, i, lq, load, [&](const Rec& nb) {
+    const float4 xj = nb.x, ej = nb.e, dj = nb.d;
     const Pair p = pair_of<FAST>(c, xi, f3(xj));
     const float3 de = ei - f3(ej);
     const float ws = p.W * c.S;
@@ -428,14 +440,14 @@ __global__ __launch_bounds__(kB) void k_adj_pos(AdjDev a, SimConst c,
 }
 
 // Predict: x*_0 = x + (v - g dt y) dt -> x_bar = x*_0 bar + xstart, v_bar = dt x*_0 bar.
-__global__ __launch_bounds__(kB) void k_adj_predict(AdjDev a, SimConst c,
+__global__ __launch_bounds__(kB) void k_adj_predict(const float4* __restrict__ ids, uint32_t n,
                                                     const float4* __restrict__ ybar,
                                                     const float4* __restrict__ xstart,
                                                     float4* __restrict__ xbar_id,
-                                                    float4* __restrict__ vbar_id) {
+                                                    float4* __restrict__ vbar_id, SimConst c) {
   const uint32_t i = idx();
-  if (i >= a.n) return;
-  const uint32_t id = __float_as_uint(a.ids[i].w);
+  if (i >= n) return;
+  const uint32_t id = __float_as_uint(ids[i].w);
   const float3 y = f3(ybar[i]);
   const float3 xb = y + f3(xstart[i]);
   const float3 vb = c.dt * y;
@@ -636,26 +648,28 @@ int backward_step_l(pbf_adj* a, const pbf::SimConst& k, int t, const AdjTape& T)
   const uint32_t n = (uint32_t)a->n;
   const size_t np = (size_t)a->npad;
   const AdjTape d = T;
-  pbf::AdjDev ad{d.posB, d.nbr, d.ncnt, pbf::k4_of(*c), n};
+  const int K4 = pbf::k4_of(*c);
   const unsigned nb = pbf::nblk(n), nbl = pbf::nblk((int64_t)n * L);
   hipStream_t s = c->stream;
   const pbf::SceneGrid g = c->grids[0];
   // dL/dv_new and dL/dx_new in sorted order.
   pbf::k_from_id2<<<nb, pbf::kB, 0, s>>>(n, d.posB, a->vbar, a->vb3, a->xbar, a->xbn);
-  pbf::k_adj_vort_a<L, FAST><<<nbl, pbf::kB, 0, s>>>(ad, k, d.predP, d.vort, a->vb3, a->etab, a->wb);
-  pbf::k_adj_vort_b<L, FAST><<<nbl, pbf::kB, 0, s>>>(ad, k, d.predP, d.vort, a->etab, a->wb, a->xbn,
-                                              a->xsacc);
-  pbf::k_adj_xsph<L, FAST><<<nbl, pbf::kB, 0, s>>>(ad, k, d.predQ, d.velB, a->vb3, a->wb, a->xsacc,
-                                            a->yb, a->xst, a->contacts, g);
+  pbf::k_adj_vort_a<L, FAST><<<nbl, pbf::kB, 0, s>>>(d.nbr, d.ncnt, K4, n, d.predP, d.vort, a->vb3,
+                                                     a->etab, a->wb, k);
+  pbf::k_adj_vort_b<L, FAST><<<nbl, pbf::kB, 0, s>>>(d.nbr, d.ncnt, K4, n, d.predP, d.vort, a->etab,
+                                                     a->wb, a->xbn, a->xsacc, k);
+  pbf::k_adj_xsph<L, FAST><<<nbl, pbf::kB, 0, s>>>(d.nbr, d.ncnt, K4, n, d.predQ, d.velB, a->vb3,
+                                                   a->wb, a->xsacc, a->yb, a->xst, a->contacts, k,
+                                                   g);
   AHIP(a, hipGetLastError());
   const int S = c->p.iterations;
   for (int it = S - 1; it >= 0; it--) {
     const float4* xs = d.stash + (size_t)it * np;
     // etab is free again: it holds the (x*, lambda) records.
-    pbf::k_adj_lambda<L, FAST><<<nbl, pbf::kB, 0, s>>>(ad, k, xs, a->yb, a->etab, a->aux, a->Gb,
-                                                       a->contacts, g);
-    pbf::k_adj_pos<L, FAST><<<nbl, pbf::kB, 0, s>>>(ad, k, a->etab, a->aux, a->Gb, a->yb, a->yb2,
-                                                    a->kpart + (size_t)it * np);
+    pbf::k_adj_lambda<L, FAST><<<nbl, pbf::kB, 0, s>>>(d.nbr, d.ncnt, K4, n, xs, a->yb, a->etab,
+                                                       a->aux, a->Gb, a->contacts, k, g);
+    pbf::k_adj_pos<L, FAST><<<nbl, pbf::kB, 0, s>>>(d.nbr, d.ncnt, K4, n, a->etab, a->aux, a->Gb,
+                                                    a->yb, a->yb2, a->kpart + (size_t)it * np, k);
     AHIP(a, hipGetLastError());
     std::swap(a->yb, a->yb2);
   }
@@ -663,7 +677,7 @@ int backward_step_l(pbf_adj* a, const pbf::SimConst& k, int t, const AdjTape& T)
   pbf::k_sum_double_part<<<pbf::kSumParts, pbf::kB, 0, s>>>((uint32_t)(np * (size_t)S), a->kpart,
                                                             a->kslice);
   pbf::k_sum_double<<<1, pbf::kB, 0, s>>>((uint32_t)pbf::kSumParts, a->kslice, a->ksteps + t);
-  pbf::k_adj_predict<<<nb, pbf::kB, 0, s>>>(ad, k, a->yb, a->xst, a->xbar, a->vbar);
+  pbf::k_adj_predict<<<nb, pbf::kB, 0, s>>>(d.posB, n, a->yb, a->xst, a->xbar, a->vbar, k);
   AHIP(a, hipGetLastError());
   return PBF_OK;
 }

@@ -65,7 +65,12 @@ struct Dev {
   // Nonzero: the prediction stores the advanced v in velA and the sort moves
   // it to velB (read only by debug stops and the adjoint).
   uint32_t move_v;
-  // LDS tiles (pbf_tiles.h; titem NULL: off).
+  uint32_t n;
+  int K4;
+};
+// With the LDS tiles (pbf_tiles.h).  Apart: 48 bytes that the other passes'
+// arguments do not carry.
+struct TileDev : Dev {
   TileItem* titem;
   uint8_t* tflag;
   TileRec* trec;
@@ -73,8 +78,6 @@ struct Dev {
   uint16_t* tnbr;
   uint32_t tile_items, tile_units;
   float tile_far;
-  uint32_t n;
-  int K4;
 };
 
 inline unsigned blocks_for(int64_t n) { return (unsigned)((n + kBlock - 1) / kBlock); }
@@ -109,16 +112,7 @@ Dev dev_of(const Ctx& x) {
   d.dense_cell = x.dense_cell;
   d.move_v = x.sorted_v ? 1u : 0u;
   d.nlane = 0;
-  d.titem = nullptr;
   if (x.tile_on) {
-    d.titem = s.titem;
-    d.tflag = s.tflag;
-    d.trec = s.trec;
-    d.town = s.town;
-    d.tnbr = s.tnbr;
-    d.tile_items = x.tile_cap;
-    d.tile_units = x.tile_units;
-    d.tile_far = x.tile_far;
     d.dense = s.dense;
     d.dense_b = s.dense_b;
     d.dense_cell = 0xffffffffu;
@@ -126,6 +120,40 @@ Dev dev_of(const Ctx& x) {
   d.n = (uint32_t)x.n;
   d.K4 = k4_of(x);
   return d;
+}
+
+static TileDev tile_dev_of(const Ctx& x) {
+  const DevState& s = x.d;
+  TileDev d;
+  static_cast<Dev&>(d) = dev_of(x);
+  d.titem = s.titem;
+  d.tflag = s.tflag;
+  d.trec = s.trec;
+  d.town = s.town;
+  d.tnbr = s.tnbr;
+  d.tile_items = x.tile_cap;
+  d.tile_units = x.tile_units;
+  d.tile_far = x.tile_far;
+  return d;
+}
+
+// First arguments of the passes that small and middle states launch: what a
+// wave needs before it can gather.  Leading scalar arguments are preloaded
+// into SGPRs (-amdgpu-kernarg-preload-count) and structs are not, so a wave
+// starts its list and particle loads without first waiting for the argument
+// segment.  The 11 λ passes of the 720-particle scene's step (27 launches)
+// alone: 111.3 -> 106.6 us per step.  All passes: 122.5 -> 113.0 us at 720
+// particles, 168.4 -> 160.4 at 2,106, 104.0 -> 101.7 at 20,011, 147.2 -> 143.6
+// at 70,001.
+#define PBF_LIST_PARAMS const float4 *in, uint32_t *ncnt, uint32_t *nbr, uint32_t n, int K4, uint32_t nb
+#define PBF_LIST_ARGS(in, d, nb) \
+  reinterpret_cast<const float4*>(in), (d).ncnt, (d).nbr, (d).n, (d).K4, (uint32_t)(nb)
+__device__ __forceinline__ void use_list(Dev& d, uint32_t* ncnt, uint32_t* nbr, uint32_t n,
+                                         int K4) {
+  d.ncnt = ncnt;
+  d.nbr = nbr;
+  d.n = n;
+  d.K4 = K4;
 }
 
 __device__ __forceinline__ uint32_t id_of(const float4& p) { return __float_as_uint(p.w); }
@@ -816,8 +844,8 @@ __device__ __forceinline__ void density_one(uint32_t i, const Dev& d, const SimC
 // The list build and the lambda, delta-p and XSPH passes of particle i on
 // the four lanes of a quad; every lane of the quad calls them.  The quad
 // kernels and the dense split's quad workgroups share them.
-__device__ __forceinline__ uint32_t quad_index() {
-  return (xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x) >> 2;
+__device__ __forceinline__ uint32_t quad_index(uint32_t nb) {
+  return (xcd_block(blockIdx.x, nb) * kBlock + threadIdx.x) >> 2;
 }
 
 template <bool PACKED>
@@ -1016,8 +1044,12 @@ __global__ __launch_bounds__(kBlock) void k_predict(Dev d, SimConst c, SceneGrid
 // to `out` (the array where a prediction fused into the previous step's last
 // pass would be) instead of predP.
 template <bool MULTI>
-__global__ __launch_bounds__(kBlock) void k_predict_into(Dev d, SimConst c, SceneGrid g0,
-                                                         float4* out) {
+__global__ __launch_bounds__(kBlock) void k_predict_into(float4* posA, float4* velA, uint32_t n,
+                                                         float4* out, Dev d, SimConst c,
+                                                         SceneGrid g0) {
+  d.posA = posA;
+  d.velA = velA;
+  d.n = n;
   const uint32_t i = flat_index();
   const bool valid = i < d.n;
   uint32_t cl = 0xffffffffu;
@@ -1030,13 +1062,28 @@ __global__ __launch_bounds__(kBlock) void k_predict_into(Dev d, SimConst c, Scen
 // The dense split's queue counters start at zero in every step: the build
 // queue's before the rank pass fills it (here), the list queue's before the
 // build fills it (in k_rank).
-__global__ __launch_bounds__(kBlock) void k_scatter(Dev d) {
+__global__ __launch_bounds__(kBlock) void k_scatter(
+    uint32_t* cell, uint32_t* arrival, uint32_t* start, float4* posA, uint32_t* tmpId, uint32_t n,
+    Dev d, bool tiles) {
+  d.cell = cell;
+  d.arrival = arrival;
+  d.cellStart = start;
+  d.posA = posA;
+  d.tmpId = tmpId;
+  d.n = n;
   const uint32_t i = flat_index();
   if (i < d.n) scatter_one(i, d);
-  if (i == 0 && d.dense_b && !d.titem) d.flags[kDenseBuildSlot] = 0u;
+  if (i == 0 && d.dense_b && !tiles) d.flags[kDenseBuildSlot] = 0u;
 }
 
-__global__ __launch_bounds__(kBlock) void k_rank(Dev d, const float4* pred) {
+__global__ __launch_bounds__(kBlock) void k_rank(const float4* pred, float4* posA, uint32_t* cell,
+                                                  uint32_t* start, uint32_t* tmpId, uint32_t n,
+                                                  Dev d) {
+  d.posA = posA;
+  d.cell = cell;
+  d.cellStart = start;
+  d.tmpId = tmpId;
+  d.n = n;
   const uint32_t i = flat_index();
   if (i < d.n) rank_one(i, d, pred);
   if (i == 0 && d.dense) d.flags[kDenseSlot] = 0u;
@@ -1319,8 +1366,10 @@ __device__ __forceinline__ void wide_list_sums(uint32_t i, int cnt, const Dev& d
 // so the same list; the partial last chunk is padded with its first entry
 // as nbr_one pads it.
 template <bool MULTI>
-__global__ __launch_bounds__(kWide) void k_nbr_lambda_wide(Dev d, SimConst c, SceneGrid g0,
-                                                           float4* out) {
+__global__ __launch_bounds__(kWide) void k_nbr_lambda_wide(
+    PBF_LIST_PARAMS, float4* out, Dev d, SimConst c, SceneGrid g0) {
+  use_list(d, ncnt, nbr, n, K4);
+  d.predQ = const_cast<float4*>(in);
   __shared__ float T[5][kWideRow];
   const uint32_t i = blockIdx.x;
   if (i >= d.n) return;
@@ -1422,8 +1471,10 @@ __global__ __launch_bounds__(kWide) void k_nbr_lambda_wide(Dev d, SimConst c, Sc
 
 // lambda_one, wide.
 template <bool PACKED>
-__global__ __launch_bounds__(kWide) void k_lambda_wide(Dev d, SimConst c, const float4* in,
-                                                       float4* out) {
+__global__ __launch_bounds__(kWide) void k_lambda_wide(
+    PBF_LIST_PARAMS, float4* out, Dev d, SimConst c) {
+  use_list(d, ncnt, nbr, n, K4);
+  if (PACKED) d.xs3 = reinterpret_cast<float3*>(const_cast<float4*>(in));
   __shared__ float T[5][kWideRow];
   const uint32_t i = blockIdx.x;
   if (i >= d.n) return;
@@ -1448,8 +1499,9 @@ __global__ __launch_bounds__(kWide) void k_lambda_wide(Dev d, SimConst c, const 
 
 // deltap_one, wide.
 template <bool MULTI, bool LAST, int NT>
-__global__ __launch_bounds__(kWide) void k_deltap_wide(Dev d, SimConst c, SceneGrid g0,
-                                                       const float4* in) {
+__global__ __launch_bounds__(kWide) void k_deltap_wide(
+    PBF_LIST_PARAMS, Dev d, SimConst c, SceneGrid g0) {
+  use_list(d, ncnt, nbr, n, K4);
   __shared__ float T[3][kWideRow];
   const uint32_t i = blockIdx.x;
   if (i >= d.n) return;
@@ -1463,7 +1515,10 @@ __global__ __launch_bounds__(kWide) void k_deltap_wide(Dev d, SimConst c, SceneG
 }
 
 // xsph_one, wide.
-__global__ __launch_bounds__(kWide) void k_xsph_wide(Dev d, SimConst c, float4* out) {
+__global__ __launch_bounds__(kWide) void k_xsph_wide(
+    PBF_LIST_PARAMS, float4* out, Dev d, SimConst c) {
+  use_list(d, ncnt, nbr, n, K4);
+  d.xv = const_cast<float4*>(in);
   __shared__ float T[7][kWideRow];
   const uint32_t i = blockIdx.x;
   if (i >= d.n) return;
@@ -1483,8 +1538,9 @@ __global__ __launch_bounds__(kWide) void k_xsph_wide(Dev d, SimConst c, float4* 
 // particle: the slot order inside a cell does not matter, the rank orders
 // by id).
 template <bool PREDICT, bool MULTI>
-__global__ __launch_bounds__(kWide) void k_vort_wide(Dev d, SimConst c, SceneGrid g0,
-                                                     const float4* in) {
+__global__ __launch_bounds__(kWide) void k_vort_wide(
+    PBF_LIST_PARAMS, Dev d, SimConst c, SceneGrid g0) {
+  use_list(d, ncnt, nbr, n, K4);
   __shared__ float T[3][kWideRow];
   const uint32_t i = blockIdx.x;
   if (i >= d.n) return;
@@ -1512,21 +1568,27 @@ __global__ __launch_bounds__(kWide) void k_vort_wide(Dev d, SimConst c, SceneGri
 // there are four times the waves of the lane-per-particle passes and each
 // walks a quarter of the list; the sums are the same bits.
 template <bool PACKED>
-__global__ __launch_bounds__(kBlock) void k_lambda_quad(Dev d, SimConst c, const float4* in,
-                                                        float4* out) {
-  const uint32_t i = quad_index();
+__global__ __launch_bounds__(kBlock) void k_lambda_quad(
+    PBF_LIST_PARAMS, float4* out, Dev d, SimConst c) {
+  use_list(d, ncnt, nbr, n, K4);
+  if (PACKED) d.xs3 = reinterpret_cast<float3*>(const_cast<float4*>(in));
+  const uint32_t i = quad_index(nb);
   if (i < d.n) lambda_quad_one<PACKED>(i, d, c, in, out);  // a quad's lanes leave together
 }
 
 template <bool LAST, int NT>
-__global__ __launch_bounds__(kBlock) void k_deltap_quad(Dev d, SimConst c, SceneGrid g,
-                                                        const float4* in) {
-  const uint32_t i = quad_index();
+__global__ __launch_bounds__(kBlock) void k_deltap_quad(
+    PBF_LIST_PARAMS, Dev d, SimConst c, SceneGrid g) {
+  use_list(d, ncnt, nbr, n, K4);
+  const uint32_t i = quad_index(nb);
   if (i < d.n) deltap_quad_one<LAST, NT>(i, d, c, g, in);
 }
 
-__global__ __launch_bounds__(kBlock) void k_nbr_quad(Dev d, float h2, SceneGrid g) {
-  const uint32_t i = quad_index();
+__global__ __launch_bounds__(kBlock) void k_nbr_quad(
+    PBF_LIST_PARAMS, float h2, Dev d, SceneGrid g) {
+  use_list(d, ncnt, nbr, n, K4);
+  d.predQ = const_cast<float4*>(in);
+  const uint32_t i = quad_index(nb);
   if (i < d.n) nbr_quad_one<16>(i, d, h2, g);  // a quad's lanes leave together
 }
 
@@ -1536,9 +1598,10 @@ __global__ __launch_bounds__(kBlock) void k_nbr_quad(Dev d, float h2, SceneGrid 
 // and its histogram slot (one atomic per particle: the sort ranks a cell's
 // particles by id, whatever their slots).
 template <bool PREDICT>
-__global__ __launch_bounds__(kBlock) void k_vort_quad(Dev d, SimConst c, SceneGrid g,
-                                                      const float4* in) {
-  const uint32_t i = quad_index();
+__global__ __launch_bounds__(kBlock) void k_vort_quad(
+    PBF_LIST_PARAMS, Dev d, SimConst c, SceneGrid g) {
+  use_list(d, ncnt, nbr, n, K4);
+  const uint32_t i = quad_index(nb);
   if (i >= d.n) return;
   const float4 xi = in[i];
   float s[3];
@@ -1556,8 +1619,11 @@ __global__ __launch_bounds__(kBlock) void k_vort_quad(Dev d, SimConst c, SceneGr
   }
 }
 
-__global__ __launch_bounds__(kBlock) void k_xsph_quad(Dev d, SimConst c, float4* out) {
-  const uint32_t i = quad_index();
+__global__ __launch_bounds__(kBlock) void k_xsph_quad(
+    PBF_LIST_PARAMS, float4* out, Dev d, SimConst c) {
+  use_list(d, ncnt, nbr, n, K4);
+  d.xv = const_cast<float4*>(in);
+  const uint32_t i = quad_index(nb);
   if (i < d.n) xsph_quad_one(i, d, c, out);
 }
 
@@ -1581,8 +1647,12 @@ __device__ __forceinline__ void nbr_export_one(uint32_t i, const Dev& d,
 // barrier makes the phase's global writes visible).  The same per-particle
 // code as the flat launches: the same bits.
 constexpr int kSortSmallBlock = 1024;
-__global__ __launch_bounds__(kSortSmallBlock) void k_sort_small(Dev d, const float4* pred,
-                                                                uint32_t ncell) {
+__global__ __launch_bounds__(kSortSmallBlock) void k_sort_small(uint32_t* count, uint32_t* start,
+                                                                uint32_t ncell, uint32_t n,
+                                                                const float4* pred, Dev d) {
+  d.cellCount = count;
+  d.cellStart = start;
+  d.n = n;
   __shared__ uint32_t wsum[kSortSmallBlock / 64 + 1];
   // The dense split's queue counters, as k_scatter and k_rank reset them
   // (visible to the rank phase's atomics after the barriers below).
@@ -1816,7 +1886,8 @@ bool sort_in_one_workgroup(const Ctx& x) {
 
 hipError_t launch_sort_small(Ctx& x, const float4* pred) {
   const Dev d = dev_of(x);
-  k_sort_small<<<1, kSortSmallBlock, 0, x.stream>>>(d, pred ? pred : d.predP, x.ncell);
+  k_sort_small<<<1, kSortSmallBlock, 0, x.stream>>>(d.cellCount, d.cellStart, x.ncell, d.n,
+                                                      pred ? pred : d.predP, d);
   return hipGetLastError();
 }
 
@@ -1837,13 +1908,15 @@ static unsigned tile_grid(const Ctx& x) {
 
 hipError_t launch_scatter_rank(Ctx& x, const float4* pred) {
   const Dev d = dev_of(x);
-  k_scatter<<<blocks_for(x.n), kBlock, 0, x.stream>>>(d);
+  k_scatter<<<blocks_for(x.n), kBlock, 0, x.stream>>>(d.cell, d.arrival, d.cellStart, d.posA,
+                                                      d.tmpId, d.n, d, x.tile_on);
   if (x.tile_on) {
-    k_tile_items<<<blocks_for(x.tile_blocks), kBlock, 0, x.stream>>>(d, x.grids[0]);
-    k_rank_tiled<<<(unsigned)((x.n + kRankBlock - 1) / kRankBlock), kRankBlock, 0, x.stream>>>(d, pred ? pred : d.predP, x.grids[0]);
+    k_tile_items<<<blocks_for(x.tile_blocks), kBlock, 0, x.stream>>>(tile_dev_of(x), x.grids[0]);
+    k_rank_tiled<<<(unsigned)((x.n + kRankBlock - 1) / kRankBlock), kRankBlock, 0, x.stream>>>(tile_dev_of(x), pred ? pred : d.predP, x.grids[0]);
     return hipGetLastError();
   }
-  k_rank<<<blocks_for(x.n), kBlock, 0, x.stream>>>(d, pred ? pred : d.predP);
+  k_rank<<<blocks_for(x.n), kBlock, 0, x.stream>>>(pred ? pred : d.predP, d.posA, d.cell,
+                                                   d.cellStart, d.tmpId, d.n, d);
   return hipGetLastError();
 }
 
@@ -1876,7 +1949,8 @@ static Dev split_dev(const Ctx& x, ListPass p, unsigned* grid) {
 hipError_t launch_nbr_build(Ctx& x, const SimConst& c) {
   const Dev d = dev_of(x);
   if (quad(x, kPassBuild)) {
-    k_nbr_quad<<<quad_grid(x), kBlock, 0, x.stream>>>(d, c.h2, x.grids[0]);
+    k_nbr_quad<<<quad_grid(x), kBlock, 0, x.stream>>>(
+        PBF_LIST_ARGS(d.predQ, d, quad_grid(x)), c.h2, d, x.grids[0]);
     return hipGetLastError();
   }
   if (multi(x))
@@ -1889,21 +1963,25 @@ hipError_t launch_nbr_build(Ctx& x, const SimConst& c) {
 hipError_t launch_nbr_lambda(Ctx& x, const SimConst& c, float4* out) {
   const Dev d = dev_of(x);
   if (x.tile_on) {
-    k_tile_build<<<tile_grid(x), kTileBlock, 0, x.stream>>>(d, c, x.grids[0], out);
-    k_queue_build<<<kQueueBuildGrid, kBlock, 0, x.stream>>>(d, c, x.grids[0], out);
+    k_tile_build<<<tile_grid(x), kTileBlock, 0, x.stream>>>(tile_dev_of(x), c, x.grids[0], out);
+    k_queue_build<<<kQueueBuildGrid, kBlock, 0, x.stream>>>(tile_dev_of(x), c, x.grids[0], out);
     return hipGetLastError();
   }
   if (quad(x, kPassBuild)) {
     // The quad build, then the first lambda pass over the finished lists.
-    k_nbr_quad<<<quad_grid(x), kBlock, 0, x.stream>>>(d, c.h2, x.grids[0]);
-    k_lambda_quad<false><<<quad_grid(x), kBlock, 0, x.stream>>>(d, c, x.d.predQ, out);
+    k_nbr_quad<<<quad_grid(x), kBlock, 0, x.stream>>>(
+        PBF_LIST_ARGS(d.predQ, d, quad_grid(x)), c.h2, d, x.grids[0]);
+    k_lambda_quad<false><<<quad_grid(x), kBlock, 0, x.stream>>>(
+        PBF_LIST_ARGS(d.predQ, d, quad_grid(x)), out, d, c);
     return hipGetLastError();
   }
   if (wide(x, kPassBuild)) {
     if (multi(x))
-      k_nbr_lambda_wide<true><<<wide_grid(x), kWide, 0, x.stream>>>(d, c, x.grids[0], out);
+      k_nbr_lambda_wide<true><<<wide_grid(x), kWide, 0, x.stream>>>(
+          PBF_LIST_ARGS(d.predQ, d, wide_grid(x)), out, d, c, x.grids[0]);
     else
-      k_nbr_lambda_wide<false><<<wide_grid(x), kWide, 0, x.stream>>>(d, c, x.grids[0], out);
+      k_nbr_lambda_wide<false><<<wide_grid(x), kWide, 0, x.stream>>>(
+          PBF_LIST_ARGS(d.predQ, d, wide_grid(x)), out, d, c, x.grids[0]);
     return hipGetLastError();
   }
   if (multi(x)) {
@@ -1920,29 +1998,34 @@ hipError_t launch_nbr_lambda(Ctx& x, const SimConst& c, float4* out) {
 
 hipError_t launch_lambda(Ctx& x, const SimConst& c, const float4* in, float4* out, bool packed) {
   if (x.tile_on) {
-    k_tile_lambda<<<tile_grid(x), kTileBlock, 0, x.stream>>>(dev_of(x), c, out);
+    k_tile_lambda<<<tile_grid(x), kTileBlock, 0, x.stream>>>(tile_dev_of(x), c, out);
     return hipGetLastError();
   }
+  const Dev d = dev_of(x);
   if (quad(x, kPassLambda)) {
     if (packed)
-      k_lambda_quad<true><<<quad_grid(x), kBlock, 0, x.stream>>>(dev_of(x), c, in, out);
+      k_lambda_quad<true><<<quad_grid(x), kBlock, 0, x.stream>>>(
+          PBF_LIST_ARGS(d.xs3, d, quad_grid(x)), out, d, c);
     else
-      k_lambda_quad<false><<<quad_grid(x), kBlock, 0, x.stream>>>(dev_of(x), c, in, out);
+      k_lambda_quad<false><<<quad_grid(x), kBlock, 0, x.stream>>>(
+          PBF_LIST_ARGS(in, d, quad_grid(x)), out, d, c);
     return hipGetLastError();
   }
   if (wide(x, kPassLambda)) {
     if (packed)
-      k_lambda_wide<true><<<wide_grid(x), kWide, 0, x.stream>>>(dev_of(x), c, in, out);
+      k_lambda_wide<true><<<wide_grid(x), kWide, 0, x.stream>>>(
+          PBF_LIST_ARGS(d.xs3, d, wide_grid(x)), out, d, c);
     else
-      k_lambda_wide<false><<<wide_grid(x), kWide, 0, x.stream>>>(dev_of(x), c, in, out);
+      k_lambda_wide<false><<<wide_grid(x), kWide, 0, x.stream>>>(
+          PBF_LIST_ARGS(in, d, wide_grid(x)), out, d, c);
     return hipGetLastError();
   }
   unsigned ng = 0;
-  const Dev d = split_dev(x, kPassLambda, &ng);
+  const Dev ds = split_dev(x, kPassLambda, &ng);
   if (packed)
-    k_lambda<true><<<ng, kBlock, 0, x.stream>>>(d, c, in, out);
+    k_lambda<true><<<ng, kBlock, 0, x.stream>>>(ds, c, in, out);
   else
-    k_lambda<false><<<ng, kBlock, 0, x.stream>>>(d, c, in, out);
+    k_lambda<false><<<ng, kBlock, 0, x.stream>>>(ds, c, in, out);
   return hipGetLastError();
 }
 
@@ -1953,30 +2036,36 @@ static void launch_deltap_nt(const Ctx& x, const Dev& d, const SimConst& c, cons
   if (x.tile_on) {
     const unsigned ng = tile_grid(x);
     if (last)
-      k_tile_deltap<true, NT><<<ng, kTileBlock, 0, x.stream>>>(d, c, x.grids[0], in);
+      k_tile_deltap<true, NT><<<ng, kTileBlock, 0, x.stream>>>(tile_dev_of(x), c, x.grids[0], in);
     else
-      k_tile_deltap<false, NT><<<ng, kTileBlock, 0, x.stream>>>(d, c, x.grids[0], in);
+      k_tile_deltap<false, NT><<<ng, kTileBlock, 0, x.stream>>>(tile_dev_of(x), c, x.grids[0], in);
     return;
   }
   if (quad(x, kPassDeltap)) {
     if (last)
-      k_deltap_quad<true, NT><<<quad_grid(x), kBlock, 0, x.stream>>>(d, c, x.grids[0], in);
+      k_deltap_quad<true, NT><<<quad_grid(x), kBlock, 0, x.stream>>>(
+          PBF_LIST_ARGS(in, d, quad_grid(x)), d, c, x.grids[0]);
     else
-      k_deltap_quad<false, NT><<<quad_grid(x), kBlock, 0, x.stream>>>(d, c, x.grids[0], in);
+      k_deltap_quad<false, NT><<<quad_grid(x), kBlock, 0, x.stream>>>(
+          PBF_LIST_ARGS(in, d, quad_grid(x)), d, c, x.grids[0]);
     return;
   }
   if (wide(x, kPassDeltap)) {
     const unsigned ng = wide_grid(x);
     if (multi(x)) {
       if (last)
-        k_deltap_wide<true, true, NT><<<ng, kWide, 0, x.stream>>>(d, c, x.grids[0], in);
+        k_deltap_wide<true, true, NT><<<ng, kWide, 0, x.stream>>>(
+            PBF_LIST_ARGS(in, d, ng), d, c, x.grids[0]);
       else
-        k_deltap_wide<true, false, NT><<<ng, kWide, 0, x.stream>>>(d, c, x.grids[0], in);
+        k_deltap_wide<true, false, NT><<<ng, kWide, 0, x.stream>>>(
+            PBF_LIST_ARGS(in, d, ng), d, c, x.grids[0]);
     } else {
       if (last)
-        k_deltap_wide<false, true, NT><<<ng, kWide, 0, x.stream>>>(d, c, x.grids[0], in);
+        k_deltap_wide<false, true, NT><<<ng, kWide, 0, x.stream>>>(
+            PBF_LIST_ARGS(in, d, ng), d, c, x.grids[0]);
       else
-        k_deltap_wide<false, false, NT><<<ng, kWide, 0, x.stream>>>(d, c, x.grids[0], in);
+        k_deltap_wide<false, false, NT><<<ng, kWide, 0, x.stream>>>(
+            PBF_LIST_ARGS(in, d, ng), d, c, x.grids[0]);
     }
     return;
   }
@@ -2006,20 +2095,23 @@ hipError_t launch_deltap(Ctx& x, const SimConst& c, const float4* in, float4* ou
 
 hipError_t launch_xsph(Ctx& x, const SimConst& c, float4* out) {
   if (x.tile_on) {
-    k_tile_xsph<<<tile_grid(x), kTileBlock, 0, x.stream>>>(dev_of(x), c, out);
+    k_tile_xsph<<<tile_grid(x), kTileBlock, 0, x.stream>>>(tile_dev_of(x), c, out);
     return hipGetLastError();
   }
+  const Dev d = dev_of(x);
   if (quad(x, kPassXsph)) {
-    k_xsph_quad<<<quad_grid(x), kBlock, 0, x.stream>>>(dev_of(x), c, out);
+    k_xsph_quad<<<quad_grid(x), kBlock, 0, x.stream>>>(
+        PBF_LIST_ARGS(d.xv, d, quad_grid(x)), out, d, c);
     return hipGetLastError();
   }
   if (wide(x, kPassXsph)) {
-    k_xsph_wide<<<wide_grid(x), kWide, 0, x.stream>>>(dev_of(x), c, out);
+    k_xsph_wide<<<wide_grid(x), kWide, 0, x.stream>>>(
+        PBF_LIST_ARGS(d.xv, d, wide_grid(x)), out, d, c);
     return hipGetLastError();
   }
   unsigned ng = 0;
-  const Dev d = split_dev(x, kPassXsph, &ng);
-  k_xsph<<<ng, kBlock, 0, x.stream>>>(d, c, out);
+  const Dev ds = split_dev(x, kPassXsph, &ng);
+  k_xsph<<<ng, kBlock, 0, x.stream>>>(ds, c, out);
   return hipGetLastError();
 }
 
@@ -2041,8 +2133,9 @@ hipError_t launch_vort_commit_predict(Ctx& x, const SimConst& c, const float4* i
   if (x.tile_on) {
     // The prediction as a launch of its own: fused, every wave of a tile
     // would wait for its histogram atomics while it holds the tile's LDS.
-    k_tile_vort<<<tile_grid(x), kTileBlock, 0, x.stream>>>(d, c, in);
-    k_predict_into<false><<<blocks_for(x.n), kBlock, 0, x.stream>>>(d, c, x.grids[0], d.vort);
+    k_tile_vort<<<tile_grid(x), kTileBlock, 0, x.stream>>>(tile_dev_of(x), c, in);
+    k_predict_into<false><<<blocks_for(x.n), kBlock, 0, x.stream>>>(
+        d.posA, d.velA, d.n, d.vort, d, c, x.grids[0]);
     return hipGetLastError();
   }
   if (wide(x, kPassVort) && !small) {
@@ -2050,24 +2143,30 @@ hipError_t launch_vort_commit_predict(Ctx& x, const SimConst& c, const float4* i
     // follows as its own launch (the serial tail of one lane per particle,
     // with one histogram atomic each, costs more than the launch).  It is
     // written where the fused prediction would be.
-    k_vort_wide<false, false><<<wide_grid(x), kWide, 0, x.stream>>>(d, c, x.grids[0], in);
+    k_vort_wide<false, false><<<wide_grid(x), kWide, 0, x.stream>>>(
+        PBF_LIST_ARGS(in, d, wide_grid(x)), d, c, x.grids[0]);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     if (multi(x))
-      k_predict_into<true><<<blocks_for(x.n), kBlock, 0, x.stream>>>(d, c, x.grids[0], d.vort);
+      k_predict_into<true><<<blocks_for(x.n), kBlock, 0, x.stream>>>(
+          d.posA, d.velA, d.n, d.vort, d, c, x.grids[0]);
     else
-      k_predict_into<false><<<blocks_for(x.n), kBlock, 0, x.stream>>>(d, c, x.grids[0], d.vort);
+      k_predict_into<false><<<blocks_for(x.n), kBlock, 0, x.stream>>>(
+          d.posA, d.velA, d.n, d.vort, d, c, x.grids[0]);
     return hipGetLastError();
   }
   if (quad(x, kPassVort) && x.n <= kVortPredictQuadMax) {
-    k_vort_quad<true><<<quad_grid(x), kBlock, 0, x.stream>>>(d, c, x.grids[0], in);
+    k_vort_quad<true><<<quad_grid(x), kBlock, 0, x.stream>>>(
+        PBF_LIST_ARGS(in, d, quad_grid(x)), d, c, x.grids[0]);
     return hipGetLastError();
   }
   if (wide(x, kPassVort)) {
     if (multi(x))
-      k_vort_wide<true, true><<<wide_grid(x), kWide, 0, x.stream>>>(d, c, x.grids[0], in);
+      k_vort_wide<true, true><<<wide_grid(x), kWide, 0, x.stream>>>(
+          PBF_LIST_ARGS(in, d, wide_grid(x)), d, c, x.grids[0]);
     else
-      k_vort_wide<true, false><<<wide_grid(x), kWide, 0, x.stream>>>(d, c, x.grids[0], in);
+      k_vort_wide<true, false><<<wide_grid(x), kWide, 0, x.stream>>>(
+          PBF_LIST_ARGS(in, d, wide_grid(x)), d, c, x.grids[0]);
     return hipGetLastError();
   }
   if (multi(x))
@@ -2079,15 +2178,18 @@ hipError_t launch_vort_commit_predict(Ctx& x, const SimConst& c, const float4* i
 
 hipError_t launch_vort_commit(Ctx& x, const SimConst& c, const float4* in) {
   if (x.tile_on) {
-    k_tile_vort<<<tile_grid(x), kTileBlock, 0, x.stream>>>(dev_of(x), c, in);
+    k_tile_vort<<<tile_grid(x), kTileBlock, 0, x.stream>>>(tile_dev_of(x), c, in);
     return hipGetLastError();
   }
+  const Dev d = dev_of(x);
   if (quad(x, kPassVort)) {
-    k_vort_quad<false><<<quad_grid(x), kBlock, 0, x.stream>>>(dev_of(x), c, x.grids[0], in);
+    k_vort_quad<false><<<quad_grid(x), kBlock, 0, x.stream>>>(
+        PBF_LIST_ARGS(in, d, quad_grid(x)), d, c, x.grids[0]);
     return hipGetLastError();
   }
   if (wide(x, kPassVort)) {
-    k_vort_wide<false, false><<<wide_grid(x), kWide, 0, x.stream>>>(dev_of(x), c, x.grids[0], in);
+    k_vort_wide<false, false><<<wide_grid(x), kWide, 0, x.stream>>>(
+        PBF_LIST_ARGS(in, d, wide_grid(x)), d, c, x.grids[0]);
     return hipGetLastError();
   }
   k_vort_commit<<<blocks_for(x.n), kBlock, 0, x.stream>>>(dev_of(x), c, in);
@@ -2149,7 +2251,7 @@ hipError_t launch_unpermute_u32(Ctx& x, const float4* ids, const uint32_t* src, 
 hipError_t launch_nbr_export(Ctx& x, uint32_t* counts, uint32_t* ids, int stride) {
   if (x.tile_lists) {
     x.tile_on = true;
-    const Dev d = dev_of(x);
+    const TileDev d = tile_dev_of(x);
     x.tile_on = false;
     k_tile_export<<<1024, kTileBlock, 0, x.stream>>>(d, counts, ids, stride);
     k_queue_export<<<256, kBlock, 0, x.stream>>>(d, counts, ids, stride);

@@ -80,7 +80,7 @@ struct TileParts {
   int px, py, pz, sx, sy, sz;  // this lane's part
   uint32_t pn;                 // its particles (0: none)
 };
-__device__ __forceinline__ TileParts tile_parts(const Dev& d, const SceneGrid& g, int x0, int y0,
+__device__ __forceinline__ TileParts tile_parts(const TileDev& d, const SceneGrid& g, int x0, int y0,
                                                 int z0, uint32_t (*cs)[8], int level) {
   const uint32_t lane = threadIdx.x & 63u;
   for (uint32_t t = lane; t < kTRows * 8u; t += 64u) {
@@ -135,7 +135,7 @@ __device__ __forceinline__ TileItem tile_item(int x, int y, int z, int sx, int s
   return it;
 }
 
-__global__ __launch_bounds__(kBlock) void k_tile_items(Dev d, SceneGrid g) {
+__global__ __launch_bounds__(kBlock) void k_tile_items(TileDev d, SceneGrid g) {
   __shared__ uint32_t cs_all[kBlock / 64][kTRows][8];
   uint32_t (*cs)[8] = cs_all[threadIdx.x >> 6];
   const int lane = (int)(threadIdx.x & 63u);
@@ -208,7 +208,7 @@ __global__ __launch_bounds__(kBlock) void k_tile_items(Dev d, SceneGrid g) {
 }
 
 // Whether the base block of cell c is tiled.
-__device__ __forceinline__ bool cell_tiled(const Dev& d, const SceneGrid& g, uint32_t c) {
+__device__ __forceinline__ bool cell_tiled(const TileDev& d, const SceneGrid& g, uint32_t c) {
   const uint32_t l = c - g.cell_base;
   const uint32_t nx = (uint32_t)g.dims[0], ny = (uint32_t)g.dims[1];
   const uint32_t r = l / nx, x = l - r * nx;
@@ -220,7 +220,7 @@ __device__ __forceinline__ bool cell_tiled(const Dev& d, const SceneGrid& g, uin
 
 // Appends i to a queue (count in flags[slot]) for the lanes with q set (every
 // lane of the wave calls).
-__device__ __forceinline__ void wave_queue(const Dev& d, uint32_t* queue, int counter, uint32_t i,
+__device__ __forceinline__ void wave_queue(const TileDev& d, uint32_t* queue, int counter, uint32_t i,
                                            bool q) {
   const unsigned long long mask = __ballot(q);
   if (!mask) return;
@@ -236,7 +236,7 @@ __device__ __forceinline__ void wave_queue(const Dev& d, uint32_t* queue, int co
 // The rank pass of a tiled step: particles of the blocks without a tile go
 // to the queue, one counter atomic per workgroup.
 constexpr int kRankBlock = 1024;
-__global__ __launch_bounds__(kRankBlock) void k_rank_tiled(Dev d, const float4* pred, SceneGrid g) {
+__global__ __launch_bounds__(kRankBlock) void k_rank_tiled(TileDev d, const float4* pred, SceneGrid g) {
   __shared__ uint32_t cnt[kRankBlock / 64 + 1];
   const uint32_t i = blockIdx.x * kRankBlock + threadIdx.x;
   uint32_t dst = 0xffffffffu;
@@ -269,7 +269,7 @@ __device__ __forceinline__ uint32_t tile_order(uint32_t b) {
 __device__ __forceinline__ uint32_t tile_span(uint32_t ni) {
   return (ni + 8u * kTileRun - 1u) & ~(8u * kTileRun - 1u);
 }
-__device__ __forceinline__ uint32_t tile_count(const Dev& d) {
+__device__ __forceinline__ uint32_t tile_count(const TileDev& d) {
   return min(d.flags[kTileItemsSlot], d.tile_items);
 }
 // The wave's index in its workgroup, known to be uniform: what it addresses
@@ -277,7 +277,7 @@ __device__ __forceinline__ uint32_t tile_count(const Dev& d) {
 __device__ __forceinline__ uint32_t tile_wave() {
   return (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
 }
-__device__ __forceinline__ uint32_t* tile_list(const Dev& d, uint32_t unit) {
+__device__ __forceinline__ uint32_t* tile_list(const TileDev& d, uint32_t unit) {
   return reinterpret_cast<uint32_t*>(
       d.tnbr + ((size_t)unit * kTileChunks * 64u + (threadIdx.x & 63u)) * 8u);
 }
@@ -291,7 +291,7 @@ struct TileHead {
   uint4 q0;
 };
 template <class Load, class Store>
-__device__ __forceinline__ TileHead tile_fill(const Dev& d, uint32_t item, Load load, Store store) {
+__device__ __forceinline__ TileHead tile_fill(const TileDev& d, uint32_t item, Load load, Store store) {
   const uint32_t wave = tile_wave(), lane = threadIdx.x & 63u;
   using V = decltype(load(0u));
   constexpr int Q = (kTRows + (int)kTileWaves - 1) / (int)kTileWaves;
@@ -324,7 +324,7 @@ __device__ __forceinline__ TileHead tile_fill(const Dev& d, uint32_t item, Load 
 }
 // The lanes and first chunks of unit u of the tile (those of the wave's first
 // unit are there already).
-__device__ __forceinline__ void tile_next(const Dev& d, TileHead& h, uint32_t u) {
+__device__ __forceinline__ void tile_next(const TileDev& d, TileHead& h, uint32_t u) {
   if (u == tile_wave()) return;
   h.own = d.town[(size_t)(h.unit + u) * 64u + (threadIdx.x & 63u)];
   h.q0 = load_chunk(tile_list(d, h.unit + u));
@@ -379,7 +379,7 @@ __device__ __forceinline__ SimConst tile_const(const SimConst& c0) {
 
 // Slot 0 pads the lists: a record at rest beyond h of every particle, whose
 // terms are zero.
-__device__ __forceinline__ float4 tile_sentinel(const Dev& d) {
+__device__ __forceinline__ float4 tile_sentinel(const TileDev& d) {
   return make_float4(d.tile_far, 0.0f, 0.0f, 0.0f);
 }
 
@@ -486,7 +486,7 @@ __device__ __forceinline__ float tile_lambda(const SimConst& c, const uint32_t* 
 }
 
 // The particles whose lists overflow a tile's, a quad each.
-__global__ __launch_bounds__(kBlock) void k_queue_build(Dev d, SimConst c, SceneGrid g,
+__global__ __launch_bounds__(kBlock) void k_queue_build(TileDev d, SimConst c, SceneGrid g,
                                                         float4* out) {
   const uint32_t qn = min(d.flags[kDenseSlot], d.n);
   const uint32_t stride = gridDim.x * (kBlock / 4);
@@ -501,7 +501,7 @@ __global__ __launch_bounds__(kBlock) void k_queue_build(Dev d, SimConst c, Scene
 // nbr_one and the first λ of a tile's particles, a lane each: the rows, the
 // pruning and the order of nbr_one over the tile's records, so the lists are
 // nbr_one's.  Also writes the tile's rows and lanes for the later passes.
-__global__ __launch_bounds__(kTileBlock, 6) void k_tile_build(Dev d, SimConst c0, SceneGrid g,
+__global__ __launch_bounds__(kTileBlock, 6) void k_tile_build(TileDev d, SimConst c0, SceneGrid g,
                                                               float4* out) {
   __shared__ float4 rec[kTileCap + 4];
   __shared__ uint32_t cs[kTRows][8];
@@ -698,7 +698,7 @@ __global__ __launch_bounds__(kTileBlock, 6) void k_tile_build(Dev d, SimConst c0
 // The first kTileQuads workgroups of a pass take the particles without a
 // tile list (both queues), a quad each.
 template <class F>
-__device__ __forceinline__ bool tile_queue(const Dev& d, F f) {
+__device__ __forceinline__ bool tile_queue(const TileDev& d, F f) {
   if (blockIdx.x >= kTileQuads) return false;
   const uint32_t nb = min(d.flags[kDenseBuildSlot], d.n), nl = min(d.flags[kDenseSlot], d.n);
   for (uint32_t q = blockIdx.x * (kTileBlock / 4) + (threadIdx.x >> 2); q < nb + nl;
@@ -709,7 +709,7 @@ __device__ __forceinline__ bool tile_queue(const Dev& d, F f) {
 
 // Runs unit(head) for every unit of every tile of this workgroup.
 template <class Load, class Store, class Unit>
-__device__ __forceinline__ void tile_run(const Dev& d, Load load, Store store, Unit unit) {
+__device__ __forceinline__ void tile_run(const TileDev& d, Load load, Store store, Unit unit) {
   const uint32_t wave = tile_wave(), step = gridDim.x - kTileQuads;
   const uint32_t ni = tile_count(d);
   for (uint32_t b = blockIdx.x - kTileQuads; b < tile_span(ni); b += step) {
@@ -730,7 +730,7 @@ __device__ __forceinline__ void tile_run(const Dev& d, Load load, Store store, U
 // records in flight per lane; four need 78 VGPRs, 198 us against 189), the
 // others run three (delta-p, at 80 VGPRs) or two (XSPH, whose records take
 // 60 KB).
-__global__ __launch_bounds__(kTileBlock) void k_tile_lambda(Dev d, SimConst c0, float4* out) {
+__global__ __launch_bounds__(kTileBlock) void k_tile_lambda(TileDev d, SimConst c0, float4* out) {
   __shared__ float4 rec[kTileCap + 4];
   if (tile_queue(d, [&](uint32_t i) { lambda_quad_one<true>(i, d, c0, nullptr, out); })) return;
   const SimConst c = tile_const(c0);
@@ -748,7 +748,7 @@ __global__ __launch_bounds__(kTileBlock) void k_tile_lambda(Dev d, SimConst c0, 
 }
 
 template <bool LAST, int NT>
-__global__ __launch_bounds__(kTileBlock, 6) void k_tile_deltap(Dev d, SimConst c0, SceneGrid g,
+__global__ __launch_bounds__(kTileBlock, 6) void k_tile_deltap(TileDev d, SimConst c0, SceneGrid g,
                                                                const float4* in) {
   __shared__ float4 rec[kTileCap + 4];
   if (tile_queue(d, [&](uint32_t i) { deltap_quad_one<LAST, NT>(i, d, c0, g, in); })) return;
@@ -778,7 +778,7 @@ __global__ __launch_bounds__(kTileBlock, 6) void k_tile_deltap(Dev d, SimConst c
       });
 }
 
-__global__ __launch_bounds__(kTileBlock) void k_tile_xsph(Dev d, SimConst c0, float4* out) {
+__global__ __launch_bounds__(kTileBlock) void k_tile_xsph(TileDev d, SimConst c0, float4* out) {
   __shared__ float4 rec[kTileCap + 4];
   __shared__ float2 rec2[kTileCap + 4];
   if (tile_queue(d, [&](uint32_t i) { xsph_quad_one(i, d, c0, out); })) return;
@@ -820,7 +820,7 @@ __global__ __launch_bounds__(kTileBlock) void k_tile_xsph(Dev d, SimConst c0, fl
       });
 }
 
-__global__ __launch_bounds__(kTileBlock) void k_tile_vort(Dev d, SimConst c0, const float4* in) {
+__global__ __launch_bounds__(kTileBlock) void k_tile_vort(TileDev d, SimConst c0, const float4* in) {
   __shared__ float4 rec[kTileCap + 4];
   if (tile_queue(d, [&](uint32_t i) {
         const float4 xi = in[i];
@@ -858,7 +858,7 @@ __global__ __launch_bounds__(kTileBlock) void k_tile_vort(Dev d, SimConst c0, co
 
 // The lists of the tiles by load id (k_nbr_export's output): slots back to
 // particles through the tile's rows.
-__global__ __launch_bounds__(kTileBlock) void k_tile_export(Dev d, uint32_t* __restrict__ counts,
+__global__ __launch_bounds__(kTileBlock) void k_tile_export(TileDev d, uint32_t* __restrict__ counts,
                                                             uint32_t* __restrict__ out, int stride) {
   const uint32_t ni = tile_count(d), lane = threadIdx.x & 63u;
   for (uint32_t item = blockIdx.x; item < ni; item += gridDim.x) {
@@ -885,7 +885,7 @@ __global__ __launch_bounds__(kTileBlock) void k_tile_export(Dev d, uint32_t* __r
   }
 }
 
-__global__ __launch_bounds__(kBlock) void k_queue_export(Dev d, uint32_t* __restrict__ counts,
+__global__ __launch_bounds__(kBlock) void k_queue_export(TileDev d, uint32_t* __restrict__ counts,
                                                          uint32_t* __restrict__ out, int stride) {
   const uint32_t nb = min(d.flags[kDenseBuildSlot], d.n), nl = min(d.flags[kDenseSlot], d.n);
   for (uint32_t q = flat_index(); q < nb + nl; q += gridDim.x * kBlock)
