@@ -210,12 +210,6 @@ __global__ __launch_bounds__(kB) void k_count_diff(uint32_t n, const float4* __r
                     __float_as_uint(v.z) == __float_as_uint(b.z);
   if (!same) atomicAdd(count, 1u);
 }
-__global__ __launch_bounds__(kB) void k_copy4(uint32_t n, const float4* __restrict__ src,
-                                              float4* __restrict__ dst) {
-  const uint32_t i = idx();
-  if (i < n) dst[i] = src[i];
-}
-
 // Vorticity confinement, part 1: eta_bar and the direct part of w_bar.
 // xw = (x*_S, |w|), w = (w, .), vb4 = dL/dv_new.
 template <int L, bool FAST>
@@ -346,9 +340,9 @@ __global__ __launch_bounds__(kB) void k_adj_xsph(ADJ_LIST_PARAMS,
 // rho_bar = C_bar/rho0.  What part 2 gathers per neighbour goes into three
 // full records, xl = (x*, lambda), er = (e, rho_bar), dg = (D_bar G, D_bar)
 // (four half-used ones before: 64 bytes instead of 48 per neighbour).
-template <int L, bool FAST>
+template <int L, bool FAST, bool PACKED>
 __global__ __launch_bounds__(kB) void k_adj_lambda(ADJ_LIST_PARAMS,
-                                                   const float4* __restrict__ xs,
+                                                   const float4* __restrict__ xs4,
                                                    const float4* __restrict__ ybar,
                                                    float4* __restrict__ xl,
                                                    float4* __restrict__ er,
@@ -359,14 +353,16 @@ __global__ __launch_bounds__(kB) void k_adj_lambda(ADJ_LIST_PARAMS,
   const uint32_t i = idx() / L;
   const int lq = (int)(idx() % L);
   if (i >= a.n) return;
-  const float3 xi = f3(xs[i]);
+  const float3* __restrict__ xs3 = reinterpret_cast<const float3*>(xs4);
+  const auto xs = [&](uint32_t j) { return PACKED ? xs3[j] : f3(xs4[j]); };
+  const float3 xi = xs(i);
   const float3 ei = c.inv_rho0 * f3(ybar[i]);
   float rho = 0.f, D = 0.f, lb = 0.f;
   float3 G = make_float3(0.f, 0.f, 0.f);
-  struct Rec { float4 x, y; };
-  const auto load = [&](uint32_t j) { return Rec{xs[j], ybar[j]}; };
+  struct Rec { float3 x; float4 y; };
+  const auto load = [&](uint32_t j) { return Rec{xs(j), ybar[j]}; };
   nbrs_split<L>(a, i, lq, load, [&](const Rec& nb) {
-    const Pair p = pair_of<FAST>(c, xi, f3(nb.x));
+    const Pair p = pair_of<FAST>(c, xi, nb.x);
     rho = rho + p.W;
     const float3 gs = c.inv_rho0 * p.g;
     G = G + gs;
@@ -475,10 +471,11 @@ __global__ __launch_bounds__(kB) void k_sum_double_part(uint32_t n, const double
   if (threadIdx.x == 0) part[blockIdx.x] = sh[0];
 }
 
-// Deterministic sum of n doubles (one workgroup, fixed order).
+// Deterministic sum of each n doubles (a workgroup each, fixed order).
 __global__ __launch_bounds__(kB) void k_sum_double(uint32_t n, const double* __restrict__ in,
                                                    double* __restrict__ out) {
   __shared__ double part[kB];
+  in += (size_t)blockIdx.x * n;
   double s = 0.0;
   for (uint32_t i = threadIdx.x; i < n; i += kB) s += in[i];
   part[threadIdx.x] = s;
@@ -487,7 +484,7 @@ __global__ __launch_bounds__(kB) void k_sum_double(uint32_t n, const double* __r
     if ((int)threadIdx.x < w) part[threadIdx.x] += part[threadIdx.x + w];
     __syncthreads();
   }
-  if (threadIdx.x == 0) *out = part[0];
+  if (threadIdx.x == 0) out[blockIdx.x] = part[0];
 }
 
 unsigned nblk(int64_t n) { return (unsigned)((n + kB - 1) / kB); }
@@ -498,8 +495,8 @@ unsigned nblk(int64_t n) { return (unsigned)((n + kB - 1) / kB); }
 // ------------------------------------------------------------- host side --
 // What the backward pass of one step reads of its forward pass, all in the
 // step's sorted order: the sorted ids and state (posB, velB after the
-// solve), x* after the solve (predQ) and after XSPH with |w| (predP), w
-// (vort), the lists, and x*_m for m = 0..S (stash).
+// solve), x*_0 (predQ), x* after XSPH with |w| (predP), w (vort), the lists,
+// and x*_m for m = 1..S (stash: 12-byte records, x*_S as float4).
 struct AdjTape {
   float4 *posB = nullptr, *predP = nullptr, *predQ = nullptr, *vort = nullptr, *velB = nullptr;
   float4* stash = nullptr;
@@ -587,13 +584,15 @@ int save_state(pbf_adj* a, float4* x, float4* v) {
 }
 
 // One forward step from the context's committed state.  With a tape slot,
-// the step's sorted state, lists and x*_m (m = 0..S) are written straight
-// into the slot (the context's buffers are swapped for the slot's during
-// the step) for the backward pass to read.
-int forward_step(pbf_adj* a, const pbf::SimConst& k, AdjTape* slot) {
+// the step's sorted state, lists and x*_m are written straight into the slot
+// (the context's buffers are swapped for the slot's during the step) for the
+// backward pass to read: x*_0 stays in predQ, which no pass after the sort
+// writes, each delta-p pass before the last leaves its 12-byte records in
+// the slot, and the last one's are unpacked there.  first: the first step
+// of a call, before which the histogram is cleared.
+int forward_step(pbf_adj* a, const pbf::SimConst& k, AdjTape* slot, bool first) {
   pbf::Ctx* c = X(a);
   pbf::DevState& d = c->d;
-  const uint32_t n = (uint32_t)a->n;
   const size_t np = (size_t)a->npad;
   const pbf::DevState own = d;
   if (slot) {
@@ -605,28 +604,21 @@ int forward_step(pbf_adj* a, const pbf::SimConst& k, AdjTape* slot) {
     d.nbr = slot->nbr;
     d.ncnt = slot->ncnt;
   }
+  c->sorted_v = false;  // velB holds the solve's v (below), never the advanced one
   auto run = [&]() -> int {
-    AHIP(a, pbf::launch_predict(*c, k));
+    AHIP(a, pbf::launch_predict(*c, k, first));
     AHIP(a, pbf::launch_scan(*c));
     AHIP(a, pbf::launch_scatter_rank(*c));
-    // The list build and the first λ pass in one launch, as in the plain
-    // step; neither changes predQ, so the stash of x* can follow.
+    // The list build and the first λ pass in one launch, as in the plain step.
     AHIP(a, pbf::launch_nbr_lambda(*c, k, d.predP));
-    if (slot) pbf::k_copy4<<<pbf::nblk(n), pbf::kB, 0, c->stream>>>(n, d.predQ, slot->stash);
     for (int it = 0; it < c->p.iterations; it++) {
       const bool last = it == c->p.iterations - 1;
       if (it > 0) AHIP(a, pbf::launch_lambda(*c, k, d.predQ, d.predP, true));
+      float4* const st = slot ? slot->stash + (size_t)it * np : nullptr;  // x* after it
+      if (slot && !last) d.xs3 = reinterpret_cast<float*>(st);
       AHIP(a, pbf::launch_deltap(*c, k, d.predP, d.predQ, last));
-      // The last iteration writes x* and v as XSPH records; the adjoint reads
-      // them from predQ and velB.
-      if (last) AHIP(a, pbf::launch_unpack_record(*c, d.predQ, d.velB));
-      if (slot) {
-        float4* st = slot->stash + (size_t)(it + 1) * np;
-        if (last)
-          pbf::k_copy4<<<pbf::nblk(n), pbf::kB, 0, c->stream>>>(n, d.predQ, st);
-        else
-          AHIP(a, pbf::launch_unpack_xs3(*c, st));  // x* of a pass before the last
-      }
+      // The last iteration writes x* and v as XSPH records.
+      if (slot && last) AHIP(a, pbf::launch_unpack_record(*c, st, d.velB));
     }
     AHIP(a, pbf::launch_xsph(*c, k, d.predP));
     AHIP(a, pbf::launch_vort_commit(*c, k, d.predP));
@@ -635,6 +627,7 @@ int forward_step(pbf_adj* a, const pbf::SimConst& k, AdjTape* slot) {
   };
   const int rc = run();
   d = own;
+  c->sorted_v = true;
   return rc;
 }
 
@@ -652,31 +645,36 @@ int backward_step_l(pbf_adj* a, const pbf::SimConst& k, int t, const AdjTape& T)
   const unsigned nb = pbf::nblk(n), nbl = pbf::nblk((int64_t)n * L);
   hipStream_t s = c->stream;
   const pbf::SceneGrid g = c->grids[0];
+  const int S = c->p.iterations;
+  const float4* xS = d.stash + (size_t)(S - 1) * np;
   // dL/dv_new and dL/dx_new in sorted order.
   pbf::k_from_id2<<<nb, pbf::kB, 0, s>>>(n, d.posB, a->vbar, a->vb3, a->xbar, a->xbn);
   pbf::k_adj_vort_a<L, FAST><<<nbl, pbf::kB, 0, s>>>(d.nbr, d.ncnt, K4, n, d.predP, d.vort, a->vb3,
                                                      a->etab, a->wb, k);
   pbf::k_adj_vort_b<L, FAST><<<nbl, pbf::kB, 0, s>>>(d.nbr, d.ncnt, K4, n, d.predP, d.vort, a->etab,
                                                      a->wb, a->xbn, a->xsacc, k);
-  pbf::k_adj_xsph<L, FAST><<<nbl, pbf::kB, 0, s>>>(d.nbr, d.ncnt, K4, n, d.predQ, d.velB, a->vb3,
+  pbf::k_adj_xsph<L, FAST><<<nbl, pbf::kB, 0, s>>>(d.nbr, d.ncnt, K4, n, xS, d.velB, a->vb3,
                                                    a->wb, a->xsacc, a->yb, a->xst, a->contacts, k,
                                                    g);
   AHIP(a, hipGetLastError());
-  const int S = c->p.iterations;
   for (int it = S - 1; it >= 0; it--) {
-    const float4* xs = d.stash + (size_t)it * np;
     // etab is free again: it holds the (x*, lambda) records.
-    pbf::k_adj_lambda<L, FAST><<<nbl, pbf::kB, 0, s>>>(d.nbr, d.ncnt, K4, n, xs, a->yb, a->etab,
-                                                       a->aux, a->Gb, a->contacts, k, g);
+    if (it > 0)
+      pbf::k_adj_lambda<L, FAST, true><<<nbl, pbf::kB, 0, s>>>(
+          d.nbr, d.ncnt, K4, n, d.stash + (size_t)(it - 1) * np, a->yb, a->etab, a->aux, a->Gb,
+          a->contacts, k, g);
+    else
+      pbf::k_adj_lambda<L, FAST, false><<<nbl, pbf::kB, 0, s>>>(
+          d.nbr, d.ncnt, K4, n, d.predQ, a->yb, a->etab, a->aux, a->Gb, a->contacts, k, g);
     pbf::k_adj_pos<L, FAST><<<nbl, pbf::kB, 0, s>>>(d.nbr, d.ncnt, K4, n, a->etab, a->aux, a->Gb,
                                                     a->yb, a->yb2, a->kpart + (size_t)it * np, k);
     AHIP(a, hipGetLastError());
     std::swap(a->yb, a->yb2);
   }
-  // dL/dk of this step: one fixed-order sum over every iteration's partials.
+  // dL/dk of this step: a fixed-order sum over every iteration's partials (its
+  // slices here; k_sum_double adds them for all steps at the end).
   pbf::k_sum_double_part<<<pbf::kSumParts, pbf::kB, 0, s>>>((uint32_t)(np * (size_t)S), a->kpart,
-                                                            a->kslice);
-  pbf::k_sum_double<<<1, pbf::kB, 0, s>>>((uint32_t)pbf::kSumParts, a->kslice, a->ksteps + t);
+                                                            a->kslice + (size_t)t * pbf::kSumParts);
   pbf::k_adj_predict<<<nb, pbf::kB, 0, s>>>(d.posB, n, a->yb, a->xst, a->xbar, a->vbar, k);
   AHIP(a, hipGetLastError());
   return PBF_OK;
@@ -749,13 +747,13 @@ static int pbf_adj_create_impl(const pbf_params* p, int64_t n, int32_t nsteps, i
   a->tape.resize((size_t)every);
   for (AdjTape& t : a->tape) {
     AA(t.posB, np); AA(t.predP, np + 64); AA(t.predQ, np + 64); AA(t.vort, np); AA(t.velB, np);
-    AA(t.stash, np * (S + 1)); AA(t.nbr, np * K); AA(t.ncnt, np);
+    AA(t.stash, np * (size_t)S); AA(t.nbr, np * K); AA(t.ncnt, np);
   }
   AA(a->xbar, np); AA(a->vbar, np); AA(a->yb, np); AA(a->yb2, np); AA(a->xst, np);
   AA(a->xsacc, np); AA(a->vb3, np); AA(a->etab, np); AA(a->wb, np); AA(a->aux, np);
   AA(a->Gb, np); AA(a->xbn, np);
   AA(a->kpart, np * (size_t)S); AA(a->ksteps, 2 * (size_t)nsteps); AA(a->contacts, 4);
-  AA(a->kslice, (size_t)pbf::kSumParts);
+  AA(a->kslice, (size_t)pbf::kSumParts * (size_t)nsteps);
   // The partials of the padding slots n..npad-1 are never written: zero
   // them once.
   if (e == hipSuccess) e = hipMemset(a->kpart, 0, np * (size_t)S * sizeof(double));
@@ -810,7 +808,7 @@ static int pbf_adj_forward_impl(pbf_adj* a, const float* x0, const float* v0, fl
       const size_t o = (size_t)(t / a->every) * (size_t)a->npad;
       if ((rc = save_state(a, a->ckx + o, a->ckv + o)) != PBF_OK) return rc;
     }
-    if ((rc = forward_step(a, k, nullptr)) != PBF_OK) return rc;
+    if ((rc = forward_step(a, k, nullptr, t == 0)) != PBF_OK) return rc;
   }
   // The final state, against which the backward pass checks its replay of
   // the last segment.
@@ -865,7 +863,7 @@ static int pbf_adj_backward_impl(pbf_adj* a, const float* xbar_T, const float* v
     if ((rc = load_state(a, a->ckx + (size_t)seg * np, a->ckv + (size_t)seg * np)) != PBF_OK)
       return rc;
     for (int t = 0; t < len; t++)
-      if ((rc = forward_step(a, k, &a->tape[(size_t)t])) != PBF_OK) return rc;
+      if ((rc = forward_step(a, k, &a->tape[(size_t)t], t == 0)) != PBF_OK) return rc;
     // The replay must end where the forward pass was at the next checkpoint
     // (or at its end): every particle's x and v, bit for bit.
     {
@@ -880,6 +878,9 @@ static int pbf_adj_backward_impl(pbf_adj* a, const float* xbar_T, const float* v
     for (int t = len - 1; t >= 0; t--)
       if ((rc = backward_step(a, k, t0 + t, a->tape[(size_t)t])) != PBF_OK) return rc;
   }
+  pbf::k_sum_double<<<(unsigned)a->nsteps, pbf::kB, 0, s>>>((uint32_t)pbf::kSumParts, a->kslice,
+                                                            a->ksteps);
+  AHIP(a, hipGetLastError());
   AHIP(a, hipEventRecord(e1, s));
   AHIP(a, hipStreamSynchronize(s));
   float ms = 0.f;

@@ -238,7 +238,9 @@ void derive_grid(const pbf_params& p, const float* lo, const float* hi, SceneGri
 // Kernel launchers (pbf_kernels.hip).  Each returns hipSuccess or the launch
 // error.
 hipError_t launch_fill_u32(uint32_t* p, size_t n, uint32_t v, hipStream_t s);
-hipError_t launch_predict(Ctx& x, const SimConst& c);
+// clear = false: the histogram is zero already (a scan of this context spent
+// the last one).
+hipError_t launch_predict(Ctx& x, const SimConst& c, bool clear = true);
 hipError_t launch_scan(Ctx& x);
 // Counting-sort scatter and (cell, id) rank; pred is where the unsorted
 // predictions are (NULL: predP).

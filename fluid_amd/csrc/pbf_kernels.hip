@@ -1897,8 +1897,9 @@ hipError_t launch_load_pack(Ctx& x, const float* xyz, const float* v, const floa
   return hipGetLastError();
 }
 
-hipError_t launch_predict(Ctx& x, const SimConst& c) {
-  hipError_t e = launch_fill_u32(x.d.cellCount, x.ncell, 0u, x.stream);
+hipError_t launch_predict(Ctx& x, const SimConst& c, bool clear) {
+  const hipError_t e =
+      clear ? launch_fill_u32(x.d.cellCount, x.ncell, 0u, x.stream) : hipSuccess;
   if (e != hipSuccess) return e;
   const Dev d = dev_of(x);
   if (multi(x))

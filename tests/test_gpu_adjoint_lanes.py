@@ -47,3 +47,28 @@ def test_lanes_and_short_sequences(n):
         for a, b in zip(out[1:3], ref[1:3]):
             assert np.isfinite(b).all() and np.abs(a - b).max() <= TOL * np.abs(b).max()
         assert abs(out[3] - ref[3]) <= TOL * abs(ref[3])
+
+
+@pytest.mark.parametrize("iterations", [1, 2])
+def test_few_iterations(orc, iterations):
+    """The tape of one and two solver iterations (x*_0 in the sorted
+    prediction, the last x* unpacked, 12-byte records between): dL/dv0 along
+    itself against FP64 central differences of the oracle, within 1e-3."""
+    sc, target = scenes.diff_block(n_side=8, steps=3)
+    p = sc.params.replace(iterations=iterations)
+    r = Rollout(p, sc.n, 3, checkpoint_every=2)
+    xT, _ = r.forward(sc.x, sc.v, p.k_tensile)
+    t64 = target.astype(np.float64)
+    _, vb, _ = r.backward(((2.0 / sc.n) * (xT.astype(np.float64) - t64)).astype(np.float32))
+    assert r.replay_mismatches() == 0 and r.stats()[1] == 0
+    r.close()
+
+    def loss(v):
+        x, _, _ = orc.step(p.as_dict(), sc.x.astype(np.float64), v, 3, dtype=np.float64)
+        return float(np.mean(np.sum((x - t64) ** 2, axis=1)))
+
+    g = vb.astype(np.float64)
+    gn = float(np.linalg.norm(g))
+    v0, h = sc.v.astype(np.float64), 1e-6
+    fd = (loss(v0 + h * g / gn) - loss(v0 - h * g / gn)) / (2 * h)
+    assert abs(fd - gn) <= 1e-3 * abs(fd)
