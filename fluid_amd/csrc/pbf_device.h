@@ -419,10 +419,10 @@ __device__ __forceinline__ float3 collide(const SceneGrid& g, const SimConst& c,
 // the difference and the quotient, an ulp or two each) are far below 1e-4,
 // and a component above 1.0001 EPS_D makes |D| exceed EPS_D.  Nearly every
 // particle of a large state passes, which spares it a square root and four
-// divisions (delta-p over LDS tiles at 4,096,000 particles 219 -> 209 us; where
-// the gathers bind nothing changes, and a small scene lying on its floor
-// only pays for the test: p.xml 114.8 -> 118 us per step).  NaN fails the
-// comparisons.
+// divisions: delta-p over LDS tiles at 4,096,000 particles 219 -> 209 us, with
+// a quad per particle at 70,001 12.6 -> 11.8, with a wave at 2,106 7.95 ->
+// 7.6, a batch of 128 scenes 78.8 -> 76.8; no change where the gathers bind
+// (300,007) or most particles lie on a wall (720).  NaN fails the comparisons.
 __device__ __forceinline__ bool moves_free(const SceneGrid& g, const SimConst& c, float3 p,
                                            float3 D) {
   const float ax = fabsf(D.x), ay = fabsf(D.y), az = fabsf(D.z);
@@ -451,12 +451,10 @@ __device__ __forceinline__ float3 clamp_response(const SceneGrid& g, const SimCo
   return collide(g, c, p, D, dir, total, total, true);
 }
 
-// clamp (src/particles.cpp:51-84): position correction, no slide.  FREE looks
-// for moves that meet no wall first.
-template <bool FREE>
+// clamp (src/particles.cpp:51-84): position correction, no slide.
 __device__ __forceinline__ float3 clamp_dp(const SceneGrid& g, const SimConst& c,
                                            const MeshView& m, float3 p, float3 dp) {
-  if (FREE && !m.ntri && moves_free(g, c, p, dp)) return move_free(g, p, dp);
+  if (!m.ntri && moves_free(g, c, p, dp)) return move_free(g, p, dp);
   float l = sqrtf(dp.x * dp.x + dp.y * dp.y + dp.z * dp.z);
   if (l <= c.eps_d) return p;
   float rl = 1.0f / l;

@@ -683,7 +683,7 @@ __device__ __forceinline__ float3* xv_record(const Dev& d, uint32_t i) {
   return reinterpret_cast<float3*>(d.xv) + 2 * (size_t)i;
 }
 
-template <bool LAST, bool FREE = false>
+template <bool LAST>
 __device__ __forceinline__ void deltap_finish(uint32_t i, const Dev& d, const SimConst& c,
                                               const SceneGrid& g, const float4& xi, float dx,
                                               float dy, float dz);
@@ -715,7 +715,7 @@ __device__ __forceinline__ void deltap_one(uint32_t i, const Dev& d, const SimCo
 // The end of newtonStepUpdatePosition from the summed correction: scale by
 // 1/rho0, clamp (src/particles.cpp:51-84), and store x* (and, in the last
 // iteration, v = (x* - x)/dt).
-template <bool LAST, bool FREE>
+template <bool LAST>
 __device__ __forceinline__ void deltap_finish(uint32_t i, const Dev& d, const SimConst& c,
                                               const SceneGrid& g, const float4& xi, float dx,
                                               float dy, float dz) {
@@ -723,7 +723,7 @@ __device__ __forceinline__ void deltap_finish(uint32_t i, const Dev& d, const Si
   dy = dy * c.inv_rho0;
   dz = dz * c.inv_rho0;
   const float3 p =
-      clamp_dp<FREE>(g, c, d.mesh, make_float3(xi.x, xi.y, xi.z), make_float3(dx, dy, dz));
+      clamp_dp(g, c, d.mesh, make_float3(xi.x, xi.y, xi.z), make_float3(dx, dy, dz));
   if (!LAST) {
     // The next λ pass reads x* from the 12-byte records only (this pass
     // gathers from its input x*).

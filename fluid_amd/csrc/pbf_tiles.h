@@ -774,7 +774,7 @@ __global__ __launch_bounds__(kTileBlock, 6) void k_tile_deltap(TileDev d, SimCon
             [&](const TilePair& p, const float4& q) {
               add(poly6_sel(c, p.r2), spiky_sel(c, p.rx, p.ry, p.rz, p.r2), q.w);
             });
-        deltap_finish<LAST, true>(h.own.x, d, c, g, xi, dx, dy, dz);
+        deltap_finish<LAST>(h.own.x, d, c, g, xi, dx, dy, dz);
       });
 }
 
