@@ -99,6 +99,12 @@ struct DevState {
 //   XSPH                   8,192:  5.5 / 7.8 / 13.9   16,384:  8.3 / 7.7 / 13.9
 //                         65,536:  -   / 12.6 / 15.2 131,072:  -   / 21.2 / 19.1
 //   vorticity              8,192: 10.3 / -   / 11.6   16,384: 13.8 / -    / 11.9
+// With the arguments preloaded (PBF_LIST_PARAMS) and the vorticity quad that
+// carries the prediction, wave / quad by events (+3 us) on the same blocks:
+//   build + first lambda  12,288: 19.4 / 22.9  16,384: 22.5 / 23.0  20,011: 25.7 / 24.3
+//   lambda                 8,192:  7.0 / 8.0   12,288:  8.5 / 8.0
+//   vorticity              4,096: 10.2 / 9.9    6,000: 10.8 / 9.9    8,192: 11.3 / 9.5
+//                         12,288: 13.4 / 9.3
 //   vorticity commit      16,384:  -   / 5.7 / 10.9   32,768:  -   / 6.6 / 11.3
 //                         65,536:  -   / 8.9 / 11.9   98,304:  -   / 13.6 / 12.6
 // PBF_WIDE_MAX (every pass's wave_max), PBF_QUAD_MAX (every quad_max) and
@@ -108,13 +114,14 @@ enum ListPass : int { kPassBuild, kPassLambda, kPassDeltap, kPassXsph, kPassVort
 struct PassRule {
   int64_t wave_max;
   int64_t quad_max;
+  int64_t wave_multi;  // wave_max of states of several scenes (no quads there)
 };
 constexpr PassRule kPassRules[kListPasses] = {
-    {20480, 114688},  // build + first lambda
-    {12288, 114688},  // lambda
-    {8192, 114688},   // delta-p
-    {12288, 114688},  // XSPH
-    {12288, 81920},   // vorticity (+ commit, + prediction)
+    {16384, 114688, 20480},  // build + first lambda
+    {11264, 114688, 12288},  // lambda
+    {8192, 114688, 8192},    // delta-p
+    {12288, 114688, 12288},  // XSPH
+    {6144, 81920, 12288},    // vorticity (+ commit, + prediction)
 };
 // The vorticity pass that carries the next step's prediction takes its quad
 // only up to this many particles: its histogram slots cost a quad one
