@@ -108,8 +108,10 @@ void free_device(Ctx* x) {
   x->alloc_cells = 0;
 }
 
-// Drops the captured step graph (buffers, dt or schedule changed).
+// Drops the captured step graphs (buffers, dt or schedule changed), once no
+// asynchronous call replays them any more.
 void drop_graph(Ctx* x) {
+  if (x->graph_exec || x->graph1_exec) (void)hipStreamSynchronize(x->stream);
   if (x->graph_exec) (void)hipGraphExecDestroy(x->graph_exec);
   if (x->graph) (void)hipGraphDestroy(x->graph);
   x->graph_exec = nullptr;
@@ -284,7 +286,7 @@ int finish_create(Ctx* x, pbf_ctx** out) {
   // PBF_NO_SMALL_SORT keeps the multi-launch scan and sort for small states
   // too (same bits; for measurement).
   x->small_sort = getenv("PBF_NO_SMALL_SORT") == nullptr;
-  // PBF_STEP_GRAPH=0: one-step calls of the flat schedule keep plain launches.
+  // PBF_STEP_GRAPH=0: the flat schedule replays no captured steps.
   if (const char* w = getenv("PBF_STEP_GRAPH")) x->step_graph = w[0] != '0';
   if (const char* w = getenv("PBF_WIDE_MAX"))
     for (pbf::PassRule& r : x->rules) r.wave_max = r.wave_multi = atoll(w);
@@ -889,6 +891,17 @@ int sync_check(Ctx* x) {
                   std::to_string(x->p.max_neighbors) + ")");
 }
 
+// Steps per captured graph of calls of several steps, and the largest state
+// whose flat schedule replays them.  A replay starts some 6 us after the one
+// before it, so a graph of one step gains only where the host's launches are
+// slower than the passes (720 particles: 27 launches a step); four steps
+// share it (us per step, plain / 1 / 4 / 8 steps per graph: 720 particles
+// 111-121 / 102 / 98.3 / 98.1, 4,096 63-73 / 69.7 / 63.6 / 63.2, 20,011 100-102 /
+// 105.7 / 100.7 / 99.8; the spread of the plain launches is the host's).
+// Capturing four steps costs one call 0.1-1.1 ms.
+constexpr int kGraphSteps = 4;
+constexpr int64_t kFlatGraphMax = 8192;
+
 // Enqueues nsteps steps with the context's schedule.
 int enqueue_steps(Ctx* x, float dt, int nsteps) {
   if (nsteps == 0) return PBF_OK;
@@ -901,17 +914,24 @@ int enqueue_steps(Ctx* x, float dt, int nsteps) {
     x->has_nbrs = true;
     x->tile_lists = false;
     x->dbg_vel = x->d.velA;
-  } else if (x->schedule == PBF_SCHED_GRAPH && nsteps >= 3) {
+  } else if (nsteps >= kGraphSteps + 2 &&
+             (x->schedule == PBF_SCHED_GRAPH ||
+              (x->schedule == PBF_SCHED_FLAT && x->step_graph && x->n <= kFlatGraphMax &&
+               dt == x->last_dtn))) {
     // The first step (it predicts) and the last (it commits without
-    // predicting) are plain launches; every step between replays one
-    // captured step that starts from the prediction fused into the previous
-    // step and ends with the next one, as the flat schedule runs them.
+    // predicting) are plain launches; the steps between replay kGraphSteps
+    // captured steps at a time that start from the prediction fused into
+    // the previous step and end with the next one, as the flat schedule
+    // runs them, and what is left over is launched.  The flat schedule does
+    // so once a second call of several steps in a row has the same dt.
+    x->last_dtn = dt;
     int rc = run_step(x, k, 0, nullptr, false, true);
     if (rc != PBF_OK) return rc;
     if (!x->graph_exec || x->graph_dt != dt) {
       drop_graph(x);
       HIPCHK(x, hipStreamBeginCapture(x->stream, hipStreamCaptureModeThreadLocal));
-      rc = run_step(x, k, 0, nullptr, true, true);
+      for (int s = 0; s < kGraphSteps && rc == PBF_OK; s++)
+        rc = run_step(x, k, 0, nullptr, true, true);
       hipGraph_t g = nullptr;
       const hipError_t e = hipStreamEndCapture(x->stream, &g);
       if (rc != PBF_OK) {
@@ -923,9 +943,11 @@ int enqueue_steps(Ctx* x, float dt, int nsteps) {
       HIPCHK(x, hipGraphInstantiate(&x->graph_exec, g, nullptr, nullptr, 0));
       x->graph_dt = dt;
     }
-    for (int s = 1; s + 1 < nsteps; s++) HIPCHK(x, hipGraphLaunch(x->graph_exec, x->stream));
-    rc = run_step(x, k, 0, nullptr, true, false);
-    if (rc != PBF_OK) return rc;
+    int s = 1;
+    for (; s + kGraphSteps < nsteps; s += kGraphSteps)
+      HIPCHK(x, hipGraphLaunch(x->graph_exec, x->stream));
+    for (; s < nsteps; s++)
+      if ((rc = run_step(x, k, 0, nullptr, true, s + 1 < nsteps)) != PBF_OK) return rc;
   } else if (nsteps == 1 &&
              (x->schedule == PBF_SCHED_GRAPH ||
               (x->schedule == PBF_SCHED_FLAT && x->step_graph && dt == x->last_dt1))) {
@@ -936,6 +958,7 @@ int enqueue_steps(Ctx* x, float dt, int nsteps) {
     // caller who changes dt every call is not made to capture every call.
     x->last_dt1 = dt;
     if (!x->graph1_exec || x->graph1_dt != dt) {
+      if (x->graph1_exec) (void)hipStreamSynchronize(x->stream);
       if (x->graph1_exec) (void)hipGraphExecDestroy(x->graph1_exec);
       if (x->graph1) (void)hipGraphDestroy(x->graph1);
       x->graph1_exec = nullptr;
@@ -955,8 +978,9 @@ int enqueue_steps(Ctx* x, float dt, int nsteps) {
     }
     HIPCHK(x, hipGraphLaunch(x->graph1_exec, x->stream));
   } else {
-    // Flat schedule, and the graph schedule for calls of two steps.
+    // Flat schedule, and the graph schedule for calls of a few steps.
     if (nsteps == 1) x->last_dt1 = dt;
+    if (nsteps >= kGraphSteps + 2) x->last_dtn = dt;
     for (int s = 0; s < nsteps; s++) {
       const int rc = run_step(x, k, 0, nullptr, s > 0, s + 1 < nsteps);
       if (rc != PBF_OK) return rc;

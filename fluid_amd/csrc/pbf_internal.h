@@ -222,7 +222,7 @@ struct Ctx {
   size_t load_cap = 0;               // floats
   unsigned long long* load_bad = nullptr;
   uint32_t* flag_host = nullptr;     // pinned word the per-call overflow check reads into
-  hipGraph_t graph = nullptr;        // captured step (PBF_SCHED_GRAPH)
+  hipGraph_t graph = nullptr;        // captured steps, for calls of several
   hipGraphExec_t graph_exec = nullptr;
   float graph_dt = 0.0f;
   hipGraph_t graph1 = nullptr;       // captured whole step, for calls of one step
@@ -230,6 +230,7 @@ struct Ctx {
   float graph1_dt = 0.0f;
   bool step_graph = true;            // flat schedule: replay graph1 when dt repeats
   float last_dt1 = -1.0f;            // dt of the previous one-step call
+  float last_dtn = -1.0f;            // dt of the previous call of several steps
   std::string err;
 };
 
