@@ -83,9 +83,10 @@ __device__ __forceinline__ Pair pair_of(const SimConst& c, float3 xi, float3 xj)
   p.rl = FAST ? sqrt_rn(r2) : sqrtf(r2);
   if (r2 < c.h2) {
     const float t = c.h2 - r2;
-    const float w = c.c1 * t * t * t, g = -6.0f * c.c1 * t * t;
-    p.W = FAST ? div_seq(w, c.h9, c.r9) : w / c.h9;
-    p.gP = (FAST ? div_seq(g, c.h9, c.r9) : g / c.h9) * p.r;
+    const float c1 = FAST ? c.c1s : c.c1;
+    const float w = c1 * t * t * t, g = -6.0f * c1 * t * t;
+    p.W = FAST ? div_seq(w, c.h9s, c.r9s) : w / c.h9;
+    p.gP = (FAST ? div_seq(g, c.h9s, c.r9s) : g / c.h9) * p.r;
   } else {
     p.W = 0.0f;
     p.gP = make_float3(0.f, 0.f, 0.f);
@@ -689,7 +690,7 @@ bool adj_fast(const pbf::SimConst& k) {
   const float tmin = k.h2 - nextafterf(k.h2, 0.0f), lo = 6.0f * k.c1 * tmin * tmin;
   const float e = k.eps_d, cube = e * e * e;
   return k.fast_div && k.fast_rcp && k.fast_sqrt && lo >= k.c1 * ((tmin * tmin) * tmin) &&
-         lo >= 0x1p-120f && 6.0f * k.c1 * k.h2 * k.h2 < k.div_hi && e >= 0x1p-40f &&
+         lo >= 0x1p-120f && 6.0f * k.c1 * k.h2 * k.h2 < pbf::div_hi(k) && e >= 0x1p-40f &&
          cube >= 0x1p-124f && k.h2 * k.h < 0x1p100f;
 }
 

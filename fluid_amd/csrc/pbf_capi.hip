@@ -204,8 +204,8 @@ int verify_math(Ctx* x) {
   // monotonic.
   const float t = k.h2, amax = k.c1 * ((t * t) * t);
   const float tmin = k.h2 - nextafterf(k.h2, 0.0f), amin = k.c1 * ((tmin * tmin) * tmin);
-  const bool div_range = amin >= 0x1p-126f && amax < k.div_hi;
-  const int e_hi = ilogbf(k.div_hi), e_lo = div_range ? ilogbf(amin) : e_hi;
+  const bool div_range = amin >= 0x1p-126f && amax < pbf::div_hi(k);
+  const int e_hi = ilogbf(pbf::div_hi(k)), e_lo = div_range ? ilogbf(amin) : e_hi;
   uint32_t hb9;
   memcpy(&hb9, &k.h9, sizeof hb9);
   const uint64_t key = ((uint64_t)hb9 << 32) | (uint32_t)(e_lo + 1024);
@@ -217,7 +217,7 @@ int verify_math(Ctx* x) {
     HIPCHK(x, hipMalloc((void**)&bad, 4 * sizeof(uint32_t)));
     uint32_t hb[4] = {1, 1, 1, 1};
     hipError_t e = pbf::launch_fill_u32(bad, 4, 0u, x->stream);
-    if (e == hipSuccess) e = pbf::launch_verify_math(k.h9, k.r9, e_lo, e_hi, bad, x->stream);
+    if (e == hipSuccess) e = pbf::launch_verify_math(k, e_lo, e_hi, bad, x->stream);
     if (e == hipSuccess) e = hipMemcpyAsync(hb, bad, sizeof hb, hipMemcpyDeviceToHost, x->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(x->stream);
     (void)hipFree(bad);
@@ -517,6 +517,16 @@ namespace pbf {
 // intpow by repeated multiplication (src/bsdf.h:49-57), the tensile scale
 // 1/poly6((0,0,dq*h)) (src/particles.cpp:151), 1/rho0 for the vector
 // divisions (vector3D.h:100-102), g*dt (:180), dt*eps_v (:242).
+constexpr int kDivScale = 64, kDivTop = 60;  // 2^k of div_seq; numerators below 2^kDivTop then
+
+// Numerators below div_hi keep a * (1/h^9) below 2^100 and 2^k a finite.
+float div_hi(const SimConst& c) {
+  const float r9 = 1.0f / c.h9;
+  int e_hi = c.h9s == c.h9 ? 100 : kDivTop;
+  if (r9 > 0.0f && isfinite(r9)) e_hi = std::min(e_hi, 100 - ilogbf(r9) - 1);
+  return ldexpf(1.0f, std::max(e_hi, -126));
+}
+
 void derive_constants(const pbf_params& p, float dt, SimConst* c) {
   c->h = p.h;
   c->h2 = p.h * p.h;
@@ -546,13 +556,16 @@ void derive_constants(const pbf_params& p, float dt, SimConst* c) {
   c->inv_dt = 1.0f / dt;
   c->gdt = p.gravity * dt;
   c->n_tensile = p.n_tensile;
-  // Short division by h^9: numerators below div_hi keep a * (1/h^9) below
-  // 2^100.  The flags stay off until a device has checked the sequences
+  // Short division by h^9, scaled by 2^kDivScale where everything stays in
+  // range.  The flags stay off until a device has checked the sequences
   // (consts_for).
-  c->r9 = 1.0f / h9;
-  int e_hi = 100;
-  if (c->r9 > 0.0f && isfinite(c->r9)) e_hi = std::min(100, 100 - ilogbf(c->r9) - 1);
-  c->div_hi = ldexpf(1.0f, std::max(e_hi, -126));
+  const float r9 = 1.0f / h9, big = 6.0f * c->c1 * std::max(c->h2 * c->h2, c->h2 * c->h2 * c->h2);
+  const bool scale = big < ldexpf(1.0f, kDivTop) && isfinite(ldexpf(h9, kDivScale)) &&
+                     ldexpf(r9, -kDivScale) >= 0x1p-100f;
+  const int k2 = scale ? kDivScale : 0;
+  c->c1s = ldexpf(c->c1, k2);
+  c->h9s = ldexpf(h9, k2);
+  c->r9s = ldexpf(r9, -k2);
   // From 2^-90 or (1.0001 EPS_D)^2, whichever is larger, a correctly rounded
   // root is at least EPS_D.
   const float em = p.eps_d * 1.0001f;

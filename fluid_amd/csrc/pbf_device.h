@@ -27,8 +27,7 @@ struct SimConst {
   float gdt;             // g * dt
   float eps_d;           // EPS_D
   int n_tensile;         // N
-  float r9;              // 1/h^9 rounded to nearest (for div_seq)
-  float div_hi;          // div_seq is checked for numerators below div_hi
+  float c1s, h9s, r9s;   // c1, h^9 and RN(1/h^9) by 2^k, 2^k and 2^-k (for div_seq)
   int fast_div;          // poly6 divides by h^9 with div_seq
   int fast_rcp;          // spiky takes its reciprocal with rcp_seq
   int fast_sqrt;         // spiky takes its square root with sqrt_rn
@@ -590,16 +589,23 @@ __device__ __forceinline__ float rcp_seq(float z) {
   return fmaf(e, y, y);
 }
 
-// div_seq: a / b as a * RN(1/b) with two FMA residual corrections.
+// div_seq: a / b as a * RN(1/b) with one FMA residual correction, which
+//   rounds correctly where the residual is exact (Markstein's division from a
+//   correctly rounded reciprocal).  The residual of the smallest poly6
+//   numerators would be subnormal, so a and b both come multiplied by 2^k and
+//   rb by 2^-k: the kernels form the numerator from c1s = 2^k c1, the
+//   quotient is the same.
 //   Checked for b = h^9 on 0 and on the binades from that of amin up to
-//   div_hi, where the poly6 numerator c1 (h^2 - r^2)^3 is 0 or lies in
+//   div_hi(), where the poly6 numerator c1 (h^2 - r^2)^3 is 0 or lies in
 //   [amin, amax] (amin from the smallest positive h^2 - r^2); the host
-//   requires amin to be normal and amax below div_hi.
+//   requires amin to be normal and amax below div_hi().
+//   A second correction without the scale held down to h = 0.03, this holds
+//   down to 0.002, and its two instructions were 3% of a list pass over LDS
+//   tiles (4,096,000 particles: lambda 199.6 -> 193.8 us, delta-p 216.7 -> 209.7,
+//   XSPH 272 -> 264, build 700 -> 680).
 __device__ __forceinline__ float div_seq(float a, float b, float rb) {
-  float q = a * rb;
-  float e = fmaf(-q, b, a);
-  q = fmaf(e, rb, q);
-  e = fmaf(-q, b, a);
+  const float q = a * rb;
+  const float e = fmaf(-q, b, a);
   return fmaf(e, rb, q);
 }
 
@@ -611,9 +617,9 @@ __device__ __forceinline__ float div_seq(float a, float b, float rb) {
 // (a round-to-nearest sum is -0 only when both terms are -0).
 __device__ __forceinline__ float poly6_sel(const SimConst& c, float r2) {
   const float t = c.h2 - r2;
-  const float a = (r2 >= c.h2) ? 0.0f : c.c1 * ((t * t) * t);
-  if (c.fast_div) return div_seq(a, c.h9, c.r9);
-  return a / c.h9;
+  const float t3 = (r2 >= c.h2) ? 0.0f : (t * t) * t;
+  if (c.fast_div) return div_seq(c.c1s * t3, c.h9s, c.r9s);
+  return c.c1 * t3 / c.h9;
 }
 
 // poly6 with the reference's branch (most candidates of a query point lie
@@ -622,9 +628,9 @@ __device__ __forceinline__ float poly6_sel(const SimConst& c, float r2) {
 __device__ __forceinline__ float poly6_br(const SimConst& c, float r2) {
   if (r2 >= c.h2) return 0.0f;
   const float t = c.h2 - r2;
-  const float a = c.c1 * ((t * t) * t);
-  if (c.fast_div) return div_seq(a, c.h9, c.r9);
-  return a / c.h9;
+  const float t3 = (t * t) * t;
+  if (c.fast_div) return div_seq(c.c1s * t3, c.h9s, c.r9s);
+  return c.c1 * t3 / c.h9;
 }
 
 __device__ __forceinline__ float3 spiky_sel(const SimConst& c, float rx, float ry, float rz,

@@ -241,6 +241,8 @@ inline int k4_of(const Ctx& x) { return (x.p.max_neighbors + 3) / 4; }
 // Host-side derivation of the step constants, in float, in the order the
 // reference evaluates them.
 void derive_constants(const pbf_params& p, float dt, SimConst* c);
+// div_seq is checked for numerators (unscaled) below div_hi.
+float div_hi(const SimConst& c);
 void derive_grid(const pbf_params& p, const float* lo, const float* hi, SceneGrid* g);
 
 // Kernel launchers (pbf_kernels.hip).  Each returns hipSuccess or the launch
@@ -300,7 +302,7 @@ struct DensityLattice {
 hipError_t launch_density_field(Ctx& x, const SimConst& c, int scene, const float* pts,
                                 const DensityLattice* lattice, uint32_t m, float* out);
 hipError_t launch_persistent(Ctx& x, const SimConst& c, int nsteps, int block, int grid);
-hipError_t launch_verify_math(float b, float rb, int div_e_lo, int div_e_hi, uint32_t* bad,
+hipError_t launch_verify_math(const SimConst& c, int div_e_lo, int div_e_hi, uint32_t* bad,
                               hipStream_t s);
 // Step constants of a context, with its verified short-division flags.
 SimConst consts_for(const Ctx& x, float dt);

@@ -1811,16 +1811,16 @@ __global__ __launch_bounds__(kBlock) void k_nbr_stats(uint32_t n, const uint32_t
 // reciprocal ([2^-100, 2^100)) and the square root ([2^-96, 2^128); below
 // 2^-96, including 0 and the subnormals, a result neither NaN nor under
 // 2^-47 counts as a mismatch).
-__global__ __launch_bounds__(kBlock) void k_verify_math(float b, float rb, int div_e_lo,
+__global__ __launch_bounds__(kBlock) void k_verify_math(SimConst c, float scale, int div_e_lo,
                                                         int div_e_hi, uint32_t* __restrict__ bad) {
   const uint32_t m = blockIdx.x * kBlock + threadIdx.x;
   if (m >= (1u << 23)) return;
   auto differ = [](float u, float v) { return __float_as_uint(u) != __float_as_uint(v) ? 1u : 0u; };
   uint32_t nd = 0, nr = 0, ns = 0;
-  if (m == 0) nd += differ(div_seq(0.0f, b, rb), 0.0f / b);
+  if (m == 0) nd += differ(div_seq(0.0f, c.h9s, c.r9s), 0.0f / c.h9);
   for (int e = div_e_lo; e < div_e_hi; e++) {
     const float a = __uint_as_float(((uint32_t)(e + 127) << 23) | m);
-    nd += differ(div_seq(a, b, rb), a / b);
+    nd += differ(div_seq(a * scale, c.h9s, c.r9s), a / c.h9);
   }
   for (int e = -100; e < 100; e++) {
     const float z = __uint_as_float(((uint32_t)(e + 127) << 23) | m);
@@ -1844,9 +1844,10 @@ __global__ __launch_bounds__(kBlock) void k_verify_math(float b, float rb, int d
 
 }  // namespace
 
-hipError_t launch_verify_math(float b, float rb, int div_e_lo, int div_e_hi, uint32_t* bad,
+hipError_t launch_verify_math(const SimConst& c, int div_e_lo, int div_e_hi, uint32_t* bad,
                               hipStream_t s) {
-  k_verify_math<<<(1u << 23) / kBlock, kBlock, 0, s>>>(b, rb, div_e_lo, div_e_hi, bad);
+  const float scale = ldexpf(1.0f, ilogbf(c.c1s) - ilogbf(c.c1));
+  k_verify_math<<<(1u << 23) / kBlock, kBlock, 0, s>>>(c, scale, div_e_lo, div_e_hi, bad);
   return hipGetLastError();
 }
 

@@ -371,8 +371,8 @@ __device__ __forceinline__ float in_vgpr(float a) {
 __device__ __forceinline__ SimConst tile_const(const SimConst& c0) {
   SimConst c = c0;
   c.fast_div = c.fast_rcp = c.fast_sqrt = 1;
-  c.r9 = in_vgpr(c.r9);
-  c.h9 = in_vgpr(c.h9);
+  c.r9s = in_vgpr(c.r9s);
+  c.h9s = in_vgpr(c.h9s);
   c.inv_rho0 = in_vgpr(c.inv_rho0);
   return c;
 }
@@ -402,7 +402,7 @@ __device__ __forceinline__ TilePair tile_pair(const float3& xi, const R& q) {
 // the clamped difference is 0 and so are the terms.
 __device__ __forceinline__ float tile_w(const SimConst& c, float r2) {
   const float t = fmaxf(c.h2 - r2, 0.0f);
-  return div_seq(c.c1 * ((t * t) * t), c.h9, c.r9);
+  return div_seq(c.c1s * ((t * t) * t), c.h9s, c.r9s);
 }
 __device__ __forceinline__ float3 tile_g(const SimConst& c, const TilePair& p) {
   const float rl = sqrt_rn(p.r2);
