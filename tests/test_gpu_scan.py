@@ -39,3 +39,28 @@ def test_cell_starts_at_tile_edges(orc, dims):
     ox, ov, _ = orc.step(p, x, v, 2, orc.NBR_GRID)
     assert np.array_equal(gx.view(np.uint32), ox.view(np.uint32))
     assert np.array_equal(gv.view(np.uint32), ov.view(np.uint32))
+
+
+@pytest.mark.parametrize("dims", [(1, 1, 1), (7, 5, 7), (32, 16, 16), (33, 16, 16), (32, 32, 32)])
+@pytest.mark.parametrize("n", [1, 64, 1024, 1025, 2049, 2560])
+def test_single_workgroup_sort(orc, dims, n):
+    """The single-workgroup sort at one to three particles a thread, with the
+    cell starts in LDS (8,192 cells) and beyond, many particles a cell."""
+    h = 0.1
+    box = [(k - 0.5) * h for k in dims]
+    p = scene_params(h, h / 2, (0, 0, 0), box, dt=0.005, max_neighbors=1024)
+    r = np.random.default_rng(n + sum(dims))
+    # At most ~900 particles within h of one another.
+    if dims == (1, 1, 1) and n > 900:
+        pytest.skip("more neighbours than a list holds")
+    x = (np.array(box) * r.uniform(0.0, 1.0, (n, 3))).astype(np.float32)
+    x = np.minimum(x, np.array(box, np.float32))
+    v = r.uniform(-0.5, 0.5, x.shape).astype(np.float32)
+    f = Particles(p)
+    f.load(x, v)
+    f.time_step(nsteps=2)
+    gx, gv, _ = f.read()
+    f.close()
+    ox, ov, _ = orc.step(p, x, v, 2, orc.NBR_GRID)
+    assert np.array_equal(gx.view(np.uint32), ox.view(np.uint32))
+    assert np.array_equal(gv.view(np.uint32), ov.view(np.uint32))
