@@ -256,10 +256,11 @@ hipError_t launch_scan(Ctx& x);
 // predictions are (NULL: predP).
 hipError_t launch_scatter_rank(Ctx& x, const float4* pred = nullptr);
 // Scan, scatter and rank in one single-workgroup launch, for states of at
-// most kSortSmallMax particles over at most kSortSmallCells cells (measured:
-// 8 us at 720 particles, 18 us at 2,106, but 36 us at 4,096, where the five
-// launches of the general path take less).
-constexpr int64_t kSortSmallMax = 2560;
+// most kSortSmallMax particles over at most kSortSmallCells cells: four
+// particles a thread.  The vorticity pass then carries the next prediction,
+// so four launches fewer a step (us per step, general path / this: 2,700
+// particles 59.4 / 55.2, 3,500 62.2 / 59.4, 4,096 64.2 / 61.7).
+constexpr int64_t kSortSmallMax = 4096;
 constexpr uint32_t kSortSmallCells = 1u << 15;
 bool sort_in_one_workgroup(const Ctx& x);
 hipError_t launch_sort_small(Ctx& x, const float4* pred = nullptr);

@@ -1687,7 +1687,7 @@ __device__ __forceinline__ void nbr_export_one(uint32_t i, const Dev& d,
 // The chain of loads is what takes the time, so all that a particle moves is
 // loaded before the scan, and the ids of the cells (and the cell starts, where
 // they fit) stay in LDS: the reference's scenes have ~30 particles a cell,
-// whose ids a thread read four at a time from L2 for each of its up to three
+// whose ids a thread read four at a time from L2 for each of its up to four
 // particles (by events, 2,106 particles 17.2 -> 9.0 us, 2,000 in a dam 11.1 ->
 // 7.2, 720 7.0 -> 6.1).
 constexpr int kSortSmallBlock = 1024;
@@ -1696,7 +1696,7 @@ __global__ __launch_bounds__(kSortSmallBlock) void k_sort_small(uint32_t* count,
                                                                 uint32_t ncell, uint32_t n,
                                                                 const float4* pred, Dev d) {
   constexpr uint32_t B = kSortSmallBlock;
-  static_assert(kSortSmallMax <= 3 * kSortSmallBlock, "three particles a thread");
+  static_assert(kSortSmallMax <= 4 * kSortSmallBlock, "four particles a thread");
   __shared__ uint32_t wsum[kSortSmallBlock / 64 + 1];
   __shared__ uint32_t ids[kSortSmallMax];
   __shared__ uint32_t starts[kSortSmallStarts + 1];
@@ -1709,8 +1709,8 @@ __global__ __launch_bounds__(kSortSmallBlock) void k_sort_small(uint32_t* count,
     if (i < n) m = Item{d.posA[i], pred[i], d.cell[i], d.arrival[i]};
     return m;
   };
-  const uint32_t i0 = threadIdx.x, i1 = i0 + B, i2 = i1 + B;
-  const Item m0 = load(i0), m1 = load(i1), m2 = load(i2);
+  const uint32_t i0 = threadIdx.x, i1 = i0 + B, i2 = i1 + B, i3 = i2 + B;
+  const Item m0 = load(i0), m1 = load(i1), m2 = load(i2), m3 = load(i3);
   // The dense split's queue counters, as k_scatter and k_rank reset them
   // (visible to the rank phase's atomics after the barriers below).
   if (threadIdx.x == 0) {
@@ -1729,6 +1729,7 @@ __global__ __launch_bounds__(kSortSmallBlock) void k_sort_small(uint32_t* count,
   scatter(i0, m0);
   scatter(i1, m1);
   scatter(i2, m2);
+  scatter(i3, m3);
   // The histogram is spent (the scan above read it): zero it for the next
   // step's prediction, which then needs no fill launch of its own.
   for (uint32_t k = threadIdx.x; k < ncell; k += B) count[k] = 0u;
@@ -1755,6 +1756,7 @@ __global__ __launch_bounds__(kSortSmallBlock) void k_sort_small(uint32_t* count,
   rank(i0, m0);
   rank(i1, m1);
   rank(i2, m2);
+  rank(i3, m3);
 }
 
 // ----------------------------------------------------------------- load --

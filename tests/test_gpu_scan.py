@@ -42,10 +42,11 @@ def test_cell_starts_at_tile_edges(orc, dims):
 
 
 @pytest.mark.parametrize("dims", [(1, 1, 1), (7, 5, 7), (32, 16, 16), (33, 16, 16), (32, 32, 32)])
-@pytest.mark.parametrize("n", [1, 64, 1024, 1025, 2049, 2560])
+@pytest.mark.parametrize("n", [1, 64, 1024, 1025, 2049, 3073, 4096, 4097])
 def test_single_workgroup_sort(orc, dims, n):
-    """The single-workgroup sort at one to three particles a thread, with the
-    cell starts in LDS (8,192 cells) and beyond, many particles a cell."""
+    """The single-workgroup sort at one to four particles a thread and one
+    particle beyond, with the cell starts in LDS (8,192 cells) and in global
+    memory, many particles a cell."""
     h = 0.1
     box = [(k - 0.5) * h for k in dims]
     p = scene_params(h, h / 2, (0, 0, 0), box, dt=0.005, max_neighbors=1024)
