@@ -367,7 +367,9 @@ def pass_table(prof, sc, steps: int, nbar: float, counters) -> dict:
             continue
         per_launch_s = ms / launches * 1e-3
         state = STATE_BYTES[name] * sc.n + (8 * ncell if name == "scan" else 0)
-        listb = (4.0 * nbar + 4.0) * sc.n if name in LIST_PASSES else 0.0
+        # Tiled lists (states of 400,000 particles or more) hold 16-bit entries.
+        entry = 2.0 if sc.n >= 400_000 else 4.0
+        listb = (entry * nbar + 4.0) * sc.n if name in LIST_PASSES else 0.0
         pd = {
             "ms_per_step": ms / steps,
             "launches_per_step": launches / steps,

@@ -145,7 +145,8 @@ static TileDev tile_dev_of(const Ctx& x) {
 // alone: 111.3 -> 106.6 us per step.  All passes: 122.5 -> 113.0 us at 720
 // particles, 168.4 -> 160.4 at 2,106, 104.0 -> 101.7 at 20,011, 147.2 -> 143.6
 // at 70,001.
-#define PBF_LIST_PARAMS const float4 *in, uint32_t *ncnt, uint32_t *nbr, uint32_t n, int K4, uint32_t nb
+#define PBF_LIST_PARAMS \
+  const float4 *in, uint32_t *ncnt, uint32_t *nbr, uint32_t n, int K4, uint32_t nb
 #define PBF_LIST_ARGS(in, d, nb) \
   reinterpret_cast<const float4*>(in), (d).ncnt, (d).nbr, (d).n, (d).K4, (uint32_t)(nb)
 __device__ __forceinline__ void use_list(Dev& d, uint32_t* ncnt, uint32_t* nbr, uint32_t n,
@@ -251,9 +252,10 @@ __global__ __launch_bounds__(1024) void k_scan_partials(uint32_t* __restrict__ p
 // k_scan_partials, or with FOLD the sum of the tile totals before b, which
 // the workgroup adds up itself (then out[n] = the total as well).  The scan
 // of a few thousand to a few million cells is launches and their latency:
-// FOLD saves the one-workgroup launch between (scan of 20,011 particles
-// 10.4 -> 8.4 us, 1M 14.3 -> 11.6, 4M 32.6 -> 28.8).  A workgroup reads up to
-// nb totals; kScanFold keeps that at 16 loads a thread.
+// FOLD saves the one-workgroup launch between, and four cells a thread instead
+// of one serve both (scan of 20,011 particles 10.4 -> 8.4 us, 1M 14.3 -> 11.6;
+// 4M, 5.4M cells and not folded, 32.6 -> 28.8).  A workgroup reads up to nb
+// totals; kScanFold keeps that at 16 loads a thread.
 constexpr uint32_t kScanFold = 4096;
 template <bool FOLD>
 __global__ __launch_bounds__(kBlock) void k_scan_add(uint32_t* __restrict__ out, uint32_t n,
@@ -2007,7 +2009,8 @@ hipError_t launch_scatter_rank(Ctx& x, const float4* pred) {
                                                       d.tmpId, d.n, d, x.tile_on);
   if (x.tile_on) {
     k_tile_items<<<blocks_for(x.tile_blocks), kBlock, 0, x.stream>>>(tile_dev_of(x), x.grids[0]);
-    k_rank_tiled<<<(unsigned)((x.n + kRankBlock - 1) / kRankBlock), kRankBlock, 0, x.stream>>>(tile_dev_of(x), pred ? pred : d.predP, x.grids[0]);
+    k_rank_tiled<<<(unsigned)((x.n + kRankBlock - 1) / kRankBlock), kRankBlock, 0, x.stream>>>(
+        tile_dev_of(x), pred ? pred : d.predP, x.grids[0]);
     return hipGetLastError();
   }
   k_rank<<<blocks_for(x.n), kBlock, 0, x.stream>>>(pred ? pred : d.predP, d.posA, d.cell,

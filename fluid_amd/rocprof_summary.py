@@ -24,12 +24,20 @@ import re
 
 # Kernel name prefix -> pass name of the step (pbf.h PBF_PASS_* order).
 PASS_OF = [
+    ("k_predict_into", "vorticity"),    # the next step's prediction, after the commit
     ("k_predict", "predict"),
     ("k_scan_block", "scan"),
     ("k_scan_partials", "scan"),
     ("k_scan_add", "scan"),
     ("k_scatter", "sort"),
-    ("k_rank", "sort"),
+    ("k_rank", "sort"),                 # also k_rank_tiled
+    ("k_tile_items", "sort"),
+    ("k_tile_build", "neighbors"),      # over LDS tiles, with the first lambda
+    ("k_queue_build", "neighbors"),
+    ("k_tile_lambda", "lambda"),
+    ("k_tile_deltap", "deltap"),
+    ("k_tile_xsph", "xsph"),
+    ("k_tile_vort", "vorticity"),
     ("k_nbr_build", "neighbors"),
     ("k_nbr_lambda", "neighbors"),      # list build fused with the first lambda
     ("k_lambda", "lambda"),
@@ -39,7 +47,7 @@ PASS_OF = [
 ]
 # Kernels that stand in for one another in a pass (one or the other runs in a
 # given step): averaged by dispatches like template variants, not added up.
-VARIANT_OF = {"k_vort_commit_predict": "k_vort_commit"}
+VARIANT_OF = {"k_vort_commit_predict": "k_vort_commit", "k_rank_tiled": "k_rank"}
 COPY_BYTES = 256 << 20
 
 
@@ -60,7 +68,7 @@ VALU_PEAK_LANE_OPS = 256 * 128 * 2.4e9  # published FP32 rate, FMA counted once
 def side_of(kernel: str):
     # The prediction without movement sorts the committed state for the
     # density queries; it is not the step's prediction.
-    if kernel.startswith("k_predict") and kernel.endswith("false>"):
+    if kernel.startswith("k_predict<") and kernel.endswith("false>"):
         return "sort of the committed state"
     for prefix, p in SIDE_OF:
         if kernel.startswith(prefix):
