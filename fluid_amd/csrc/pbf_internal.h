@@ -143,8 +143,10 @@ constexpr int64_t kVortPredictQuadMax = 24576;
 // steps): 1.32 ms per step without, 0.97 at 128 (0.99 at 64, 1.07 at 256),
 // 0.93 with the build split below as well; uniform blocks of 131,072 and
 // 262,144 particles (no list above 128, no cell above 32) within 0.6%; the
-// 4,096,000-particle run 0.6% slower, hence the bound on n.
-constexpr uint32_t kDenseList = 128;
+// 4,096,000-particle run 0.6% slower, hence the bound on n.  With the cells
+// below at 48, 200 steps: 178.2 ms at 96 (178.5 at 112, 178.7 at 80), 179.8 at
+// 128 and cells of 32; 300,007 particles in free fall unchanged.
+constexpr uint32_t kDenseList = 96;
 constexpr int64_t kDenseMaxN = int64_t{1} << 20;
 constexpr int kDenseSlot = 12;
 // The list build is split the same way, by what is known before it: the
@@ -152,8 +154,9 @@ constexpr int kDenseSlot = 12;
 // particles (count in flags[kDenseBuildSlot]), and quad workgroups appended
 // to the per-lane build + first lambda launch build their lists with a quad
 // each (k_nbr_quad's walk) and run their first lambda on the same quad.
-// PBF_DENSE_CELL overrides the threshold (0: off).
-constexpr uint32_t kDenseCell = 32;
+// PBF_DENSE_CELL overrides the threshold (0: off).  178.2 ms at 48 and lists of
+// 96, 178.4 at 40 and 56, 178.4 at 64.
+constexpr uint32_t kDenseCell = 48;
 constexpr int kDenseBuildSlot = 13;  // in a tiled step: the particles without a tile
 
 struct Ctx {

@@ -56,6 +56,8 @@ constexpr uint32_t kTileRun = 8;          // consecutive tiles per XCD
 // column compresses: 1.49 ms per step without, 1.24 at 2.5, 1.23 at 4, 1.29
 // at 6; the 4,096,000-particle run 3.20, 3.36, 3.24, 3.24).
 constexpr float kTileSpike = 4.0f;
+// Cells up to kTileCrowd and lists up to kTileLong never stand out.
+constexpr uint32_t kTileCrowd = 32, kTileLong = 128;
 static_assert(kTRows <= kTileRows && kTX <= 5 && kTX * kTY * kTZ <= 64 && kTileCap <= 4096, "tile");
 
 __device__ __forceinline__ uint32_t tile_blocks(const SceneGrid& g, uint32_t* nbx, uint32_t* nby) {
@@ -580,9 +582,9 @@ __global__ __launch_bounds__(kTileBlock, 6) void k_tile_build(TileDev d, SimCons
     // the mean cell suggests (a cell of the size of h and its neighbours
     // hold 3.9 neighbours per particle of the mean cell).
     const float mean = (float)(rowO[R - 1] + (cs[R - 1][7] - cs[R - 1][0])) / (float)(wx * R);
-    const uint32_t crowd = max(kDenseCell, (uint32_t)(kTileSpike * mean));
+    const uint32_t crowd = max(kTileCrowd, (uint32_t)(kTileSpike * mean));
     const uint32_t cap = min(min((uint32_t)d.K4 * kChunk, 8u * (uint32_t)kTileChunks),
-                             max(kDenseList, (uint32_t)(kTileSpike * 3.9f * mean)));
+                             max(kTileLong, (uint32_t)(kTileSpike * 3.9f * mean)));
     const uint32_t nu = (it.n + 63u) >> 6;
     for (uint32_t u = wave; u < nu; u += kTileWaves) {
       const uint32_t p = u * 64u + lane, unit = it.unit + u;
