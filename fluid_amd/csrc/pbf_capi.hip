@@ -109,8 +109,11 @@ void free_device(Ctx* x) {
 }
 
 // Drops the captured step graphs (buffers, dt or schedule changed), once no
-// asynchronous call replays them any more.
+// asynchronous call replays them any more.  The flat schedule then captures
+// again only after two calls of the same dt: a caller who asks for densities
+// between its calls (which swaps buffers) is not made to capture every time.
 void drop_graph(Ctx* x) {
+  x->last_dt1 = x->last_dtn = -1.0f;
   if (x->graph_exec || x->graph1_exec) (void)hipStreamSynchronize(x->stream);
   if (x->graph_exec) (void)hipGraphExecDestroy(x->graph_exec);
   if (x->graph) (void)hipGraphDestroy(x->graph);
@@ -942,6 +945,7 @@ int enqueue_steps(Ctx* x, float dt, int nsteps) {
     if (rc != PBF_OK) return rc;
     if (!x->graph_exec || x->graph_dt != dt) {
       drop_graph(x);
+      x->last_dtn = dt;
       HIPCHK(x, hipStreamBeginCapture(x->stream, hipStreamCaptureModeThreadLocal));
       for (int s = 0; s < kGraphSteps && rc == PBF_OK; s++)
         rc = run_step(x, k, 0, nullptr, true, true);

@@ -66,3 +66,23 @@ def test_replays_equal_plain_launches(orc, side):
     assert _same(ref, flat.read()) and _same(ref, graph.read())
     for c in (plain, flat, graph):
         c.close()
+
+
+def test_buffer_swaps_between_calls():
+    """Densities and a density lattice between the calls swap the state's
+    buffers under the captured steps."""
+    sc, _ = scenes.diff_block(n_side=10, steps=1)
+    plain, flat = _ctx(sc.params, sc.x, sc.v, env="0"), _ctx(sc.params, sc.x, sc.v)
+    graph = _ctx(sc.params, sc.x, sc.v, schedule="graph")
+    for k, n in enumerate((7, 7, 7, 10, 1, 1, 1, 6, 6, 6)):
+        out = []
+        for c in (plain, flat, graph):
+            c.time_step(nsteps=n)
+            rho = c.estimate_densities() if k in (1, 3, 5, 7) else np.zeros(1, np.float32)
+            if k in (2, 7):
+                p = sc.params
+                rho = c.density_lattice(p.box_lo, p.box_hi, 0.5, (4, 4, 4))
+            out.append((np.ascontiguousarray(rho, np.float32), *c.read()))
+        assert _same(out[0], out[1]) and _same(out[0], out[2]), (k, n)
+    for c in (plain, flat, graph):
+        c.close()
