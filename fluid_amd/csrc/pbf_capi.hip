@@ -1584,16 +1584,17 @@ __global__ __launch_bounds__(256) void k_noalloc_unpack(uint32_t n, const float4
   v[o] = q.x; v[o + 1] = q.y; v[o + 2] = q.z;
 }
 
-// Restores the fields of a context that a workspace run borrows.
+// Restores the fields of a context that a workspace run borrows: all that
+// run_step writes of it.
 struct Borrow {
   Ctx* x;
   pbf::DevState d;
   int64_t n, npad;
   const float4 *dbg_pred, *dbg_vel;
-  bool has_nbrs;
+  bool has_nbrs, tile_lists;
   explicit Borrow(Ctx* c)
       : x(c), d(c->d), n(c->n), npad(c->npad), dbg_pred(c->dbg_pred), dbg_vel(c->dbg_vel),
-        has_nbrs(c->has_nbrs) {}
+        has_nbrs(c->has_nbrs), tile_lists(c->tile_lists) {}
   ~Borrow() {
     x->d = d;
     x->n = n;
@@ -1601,6 +1602,7 @@ struct Borrow {
     x->dbg_pred = dbg_pred;
     x->dbg_vel = dbg_vel;
     x->has_nbrs = has_nbrs;
+    x->tile_lists = tile_lists;
   }
 };
 
