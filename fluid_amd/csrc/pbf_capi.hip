@@ -1545,6 +1545,11 @@ size_t carve_state(unsigned char* base, size_t n, size_t ncell, size_t K, pbf::D
   d->stage = nullptr;
   d->dense = nullptr;  // no dense split here
   d->dense_b = nullptr;
+  d->titem = nullptr;  // no LDS tiles either (tile_step): they are the context's own state's
+  d->tflag = nullptr;
+  d->trec = nullptr;
+  d->town = nullptr;
+  d->tnbr = nullptr;
   return off;
 }
 

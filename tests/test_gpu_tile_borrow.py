@@ -55,3 +55,10 @@ def check_state_kept(tile_min, n_borrowed):
 @pytest.mark.parametrize("n", [500, 1999])
 def test_lists_survive_a_borrowed_run_below_the_tile_threshold(n):
     check_state_kept(2000, n)
+
+
+@pytest.mark.parametrize("n", [1, 1000, 3375, 5832])
+def test_borrowed_runs_take_no_tiles_of_the_loaded_state(n):
+    """The workspace holds no tiles and no queues, so its run keeps the other
+    passes, also for more particles than the context's tiles are sized for."""
+    check_state_kept(1, n)
