@@ -994,6 +994,12 @@ int enqueue_steps(Ctx* x, float dt, int nsteps) {
       x->graph1_dt = dt;
     }
     HIPCHK(x, hipGraphLaunch(x->graph1_exec, x->stream));
+    // What run_step notes of a step on the host: a load since the capture
+    // has taken it back.
+    x->has_nbrs = true;
+    x->tile_lists = pbf::tile_step(*x);
+    x->dbg_pred = x->d.predP;
+    x->dbg_vel = x->d.velA;
   } else {
     // Flat schedule, and the graph schedule for calls of a few steps.
     if (nsteps == 1) x->last_dt1 = dt;
