@@ -573,6 +573,7 @@ void derive_constants(const pbf_params& p, float dt, SimConst* c) {
   // root is at least EPS_D.
   const float em = p.eps_d * 1.0001f;
   c->r2_min = std::max(0x1p-90f, em * em);
+  c->move_min = std::max(0x1p-60f, em);
   c->fast_div = 0;
   c->fast_rcp = 0;
   c->fast_sqrt = 0;

@@ -32,6 +32,7 @@ struct SimConst {
   int fast_rcp;          // spiky takes its reciprocal with rcp_seq
   int fast_sqrt;         // spiky takes its square root with sqrt_rn
   float r2_min;          // |r|^2 from which |r| >= EPS_D for certain (tiled passes)
+  float move_min;        // component of a move from which its length > EPS_D for certain
 };
 
 // Grid and collision box of one scene.
@@ -416,8 +417,9 @@ __device__ __forceinline__ float3 collide(const SceneGrid& g, const SimConst& c,
 // walls only, no mesh).  |D| <= |D.x| + |D.y| + |D.z| =: s; a wall farther
 // than 1.0001 s has t > |D| in collide(), whose roundings (the direction,
 // the difference and the quotient, an ulp or two each) are far below 1e-4,
-// and a component above 1.0001 EPS_D makes |D| exceed EPS_D.  Nearly every
-// particle of a large state passes, which spares it a square root and four
+// and a component above 1.0001 EPS_D makes |D| exceed EPS_D, if its square is
+// in the normal range: below, |D| may round to 0 and the particle stays where
+// it is (move_min is at least 2^-60).  Nearly every particle of a large state passes, which spares it a square root and four
 // divisions: delta-p over LDS tiles at 4,096,000 particles 219 -> 209 us, with
 // a quad per particle at 70,001 12.6 -> 11.8, with a wave at 2,106 7.95 ->
 // 7.6, a batch of 128 scenes 78.8 -> 76.8; no change where the gathers bind
@@ -429,7 +431,7 @@ __device__ __forceinline__ bool moves_free(const SceneGrid& g, const SimConst& c
   const float room = fminf(fminf(fminf(p.x - g.lo[0], g.hi[0] - p.x),
                                  fminf(p.y - g.lo[1], g.hi[1] - p.y)),
                            fminf(p.z - g.lo[2], g.hi[2] - p.z));
-  return room > s && fmaxf(fmaxf(ax, ay), az) > c.eps_d * 1.0001f;
+  return room > s && fmaxf(fmaxf(ax, ay), az) > c.move_min;
 }
 
 __device__ __forceinline__ float3 move_free(const SceneGrid& g, float3 p, float3 D) {
