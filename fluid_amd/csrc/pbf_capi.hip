@@ -243,7 +243,10 @@ int verify_math(Ctx* x) {
 
 // Base blocks of a single scene's grid, and the place of the record that pads
 // the tiles' lists: beyond h of every particle, its distances in the range
-// of the short sequences (tile_blocks stays 0 where that fails).
+// of the short sequences.  A padding term is 0 times the particle's own λ (and
+// the tensile scale), or its own velocity, so those have to be finite for
+// certain: λ = -C/(D + eps) with |C| <= K W(0)/rho0 + 1 here, the velocity
+// (x* - x)/dt in tile_step.  tile_blocks stays 0 where any of it fails.
 void plan_tiles(Ctx* x) {
   x->tile_blocks = 0;
   if (x->nscenes != 1) return;
@@ -251,14 +254,20 @@ void plan_tiles(Ctx* x) {
   const SceneGrid& g = x->grids[0];
   float far = 0.0f, span = 0.0f;
   for (int a = 0; a < 3; a++) {
-    far = std::max(far, std::max(fabsf(g.lo[a]), fabsf(g.hi[a])));
-    span = std::max(span, g.hi[a] - g.lo[a]);
+    // Positions lie between lo and hi or, clamped, at lo_e or hi_e.
+    const float lo = std::min(g.lo[a], std::min(g.lo_e[a], g.hi_e[a]));
+    const float hi = std::max(g.hi[a], std::max(g.lo_e[a], g.hi_e[a]));
+    far = std::max(far, std::max(fabsf(lo), fabsf(hi)));
+    span = std::max(span, hi - lo);
   }
   x->tile_far = far + 4.0f * k.h;
-  const float reach = 4.0f * (far + span + 4.0f * k.h);  // above every |r|
+  x->tile_reach = 4.0f * (far + span + 4.0f * k.h);  // above every |r| and |x* - x|
+  const float reach = x->tile_reach;
+  const double w0 = (double)k.c1 * k.h2 * k.h2 * k.h2 / k.h9;
+  const double lam = (4.0 * pbf::k4_of(*x) * w0 / k.rho0 + 1.0) / k.eps;
   const size_t blocks = pbf::tile_block_count(g);
   if (x->tile_far - far > 2.0f * k.h && reach * reach < 0x1p100f && k.h6 * reach < 0x1p100f &&
-      blocks < ((size_t)1 << 30))
+      lam < 1e37 && is_finite_f(k.S) && blocks < ((size_t)1 << 30))
     x->tile_blocks = (uint32_t)blocks;
 }
 
@@ -373,7 +382,7 @@ int run_step(Ctx* x, const SimConst& c, int stage, PassEvents* pe = nullptr,
     }
   } restore{x};
   x->sorted_v = stage != 0;
-  x->tile_on = stage == 0 && pbf::tile_step(*x);
+  x->tile_on = stage == 0 && pbf::tile_step(*x, c);
   if (!predicted) PASS(PBF_PASS_PREDICT, pbf::launch_predict(*x, c));
   // A prediction fused into the previous step's last pass sits in vort.
   if (x->small_sort && pbf::sort_in_one_workgroup(*x)) {
@@ -998,7 +1007,7 @@ int enqueue_steps(Ctx* x, float dt, int nsteps) {
     // What run_step notes of a step on the host: a load since the capture
     // has taken it back.
     x->has_nbrs = true;
-    x->tile_lists = pbf::tile_step(*x);
+    x->tile_lists = pbf::tile_step(*x, k);
     x->dbg_pred = x->d.predP;
     x->dbg_vel = x->d.velA;
   } else {

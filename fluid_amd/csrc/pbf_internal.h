@@ -204,6 +204,7 @@ struct Ctx {
   bool tile_lists = false;           // the last step's lists are the tiles'
   uint32_t tile_blocks = 0;          // base blocks of the grid (0: no tiles)
   float tile_far = 0.0f;             // x of the padding record
+  float tile_reach = 0.0f;           // above every distance of two positions
   bool tile_on = false;              // the running step takes the LDS tiles
   // States of at least this many particles step on LDS tiles (measured in ms
   // per step, per-lane passes / tiles: 300,000 particles 0.341 / 0.345, 350,000
@@ -317,8 +318,7 @@ hipError_t launch_nbr_stats(Ctx& x, unsigned long long* sum, uint32_t* mx);
 hipError_t launch_scan_u32(uint32_t* in, uint32_t* out, uint32_t n, uint32_t* partials,
                            hipStream_t s, bool clear_in = false, uint32_t* zero4 = nullptr);
 // Whether a step of x runs on LDS tiles; base blocks of one scene's grid.
-bool tile_step(const Ctx& x);
+bool tile_step(const Ctx& x, const SimConst& c);
 size_t tile_block_count(const SceneGrid& g);
-
 
 }  // namespace pbf

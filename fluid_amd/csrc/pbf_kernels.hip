@@ -1993,8 +1993,8 @@ size_t tile_block_count(const SceneGrid& g) {
          (size_t)((g.dims[2] + kTZ - 1) / kTZ);
 }
 
-bool tile_step(const Ctx& x) {
-  return x.d.titem && x.n >= x.tile_min && x.fast_div && x.fast_rcp && x.fast_sqrt &&
+bool tile_step(const Ctx& x, const SimConst& c) {
+  return x.d.titem && x.n >= x.tile_min && c.inv_dt * x.tile_reach < 1e37f && x.fast_div && x.fast_rcp && x.fast_sqrt &&
          x.schedule != PBF_SCHED_PERSISTENT && !(x.small_sort && sort_in_one_workgroup(x));
 }
 

@@ -380,7 +380,8 @@ __device__ __forceinline__ SimConst tile_const(const SimConst& c0) {
 }
 
 // Slot 0 pads the lists: a record at rest beyond h of every particle, whose
-// terms are zero.
+// terms are zero: its factors of the particle's own values, which plan_tiles
+// and tile_step hold finite, are.
 __device__ __forceinline__ float4 tile_sentinel(const TileDev& d) {
   return make_float4(d.tile_far, 0.0f, 0.0f, 0.0f);
 }
@@ -401,7 +402,10 @@ __device__ __forceinline__ TilePair tile_pair(const float3& xi, const R& q) {
 
 // poly6 and the spiky gradient without selections: the bits of poly6_sel and
 // spiky_sel for |r| >= EPS_D, except for the sign of zero terms.  Beyond h
-// the clamped difference is 0 and so are the terms.
+// the clamped difference is 0 and so are the terms.  A NaN distance would give
+// 0 here; there is none, as every position is finite: a load refuses others
+// and each move ends in a clamp to the box (smin and smax let NaN become hi_e),
+// and plan_tiles bounds the squares.
 __device__ __forceinline__ float tile_w(const SimConst& c, float r2) {
   const float t = fmaxf(c.h2 - r2, 0.0f);
   return div_seq(c.c1s * ((t * t) * t), c.h9s, c.r9s);
