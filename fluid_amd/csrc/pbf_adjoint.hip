@@ -63,7 +63,9 @@ struct Pair {
 };
 
 // n / z.  FAST: from z's reciprocal, the quotient corrected once by its
-// residual; an overflowed quotient is left as it is.
+// residual; an overflowed quotient is left as it is.  With the reciprocal
+// correctly rounded (rcp_seq, checked on the device) and the residual exact
+// (adj_fast), this rounds correctly (Markstein), as div_seq does.
 template <bool FAST>
 __device__ __forceinline__ float quot(float n, float z) {
   if (!FAST) return n / z;
@@ -684,14 +686,20 @@ int backward_step_l(pbf_adj* a, const pbf::SimConst& k, int t, const AdjTape& T)
 constexpr int64_t kAdjWideMax = 16384;  // up to here, sixteen lanes per particle
 
 // Whether the adjoint passes can take the short sequences: verified on the
-// device, and every argument in their ranges (the poly6 gradient's numerator
-// 6 c1 t^2 in the division's, |r|^3 and h^6 |r| in the reciprocal's).
+// device, and every argument in their ranges: the poly6 gradient's numerator
+// 6 c1 t^2 in the division's; h^6 |r| and |r|^3, EPS_D <= |r| < h, in the
+// reciprocal's; quot()'s numerators, from the smallest positive h - |r|, large
+// enough for an exact residual and a normal quotient.
 bool adj_fast(const pbf::SimConst& k) {
   const float tmin = k.h2 - nextafterf(k.h2, 0.0f), lo = 6.0f * k.c1 * tmin * tmin;
-  const float e = k.eps_d, cube = e * e * e;
+  const float e = k.eps_d, zlo = std::min(e * e * e, k.h6 * e), zhi = std::max(k.h2 * k.h, k.h6 * k.h);
+  const float q = k.h - nextafterf(k.h, 0.0f), m = fabsf(k.m3c2);
+  const float n1 = m * q * q, n2 = (m / k.h6) * q * k.h;
   return k.fast_div && k.fast_rcp && k.fast_sqrt && lo >= k.c1 * ((tmin * tmin) * tmin) &&
-         lo >= 0x1p-120f && 6.0f * k.c1 * k.h2 * k.h2 < pbf::div_hi(k) && e >= 0x1p-40f &&
-         cube >= 0x1p-124f && k.h2 * k.h < 0x1p100f;
+         lo >= 0x1p-120f && 6.0f * k.c1 * k.h2 * k.h2 < pbf::div_hi(k) &&
+         std::isfinite(6.0f * k.c1s) && e >= 0x1p-40f && zlo >= 0x1p-124f && zhi < 0x1p100f &&
+         std::min(n1, n2) >= 0x1p-100f && n1 / (k.h6 * k.h) >= 0x1p-126f &&
+         n2 / (k.h2 * k.h) >= 0x1p-126f;
 }
 
 int backward_step(pbf_adj* a, const pbf::SimConst& k, int t, const AdjTape& T) {

@@ -194,7 +194,7 @@ int ensure_device(Ctx* x) {
 struct MathVerdict {
   bool checked = false;
   int rcp = 0, sqrt = 0;
-  std::map<uint64_t, int> div;  // keyed by the bits of h^9 and the lowest binade
+  std::map<uint64_t, int> div;  // keyed by the bits of h^9, the lowest binade and the scale
 };
 std::mutex g_math_mu;
 std::map<int, MathVerdict> g_math;
@@ -211,7 +211,8 @@ int verify_math(Ctx* x) {
   const int e_hi = ilogbf(pbf::div_hi(k)), e_lo = div_range ? ilogbf(amin) : e_hi;
   uint32_t hb9;
   memcpy(&hb9, &k.h9, sizeof hb9);
-  const uint64_t key = ((uint64_t)hb9 << 32) | (uint32_t)(e_lo + 1024);
+  const uint64_t key =
+      ((uint64_t)hb9 << 32) | (uint32_t)(2 * (e_lo + 1024) + (k.h9s != k.h9 ? 1 : 0));
   std::lock_guard<std::mutex> lock(g_math_mu);
   MathVerdict& v = g_math[x->device];
   auto it = v.div.find(key);

@@ -583,8 +583,8 @@ __device__ __forceinline__ float sqrt_rn(float x) {
 }
 
 // rcp_seq: hardware reciprocal refined by one Newton step with FMA.
-//   Checked on [2^-100, 2^100]; the spiky kernel passes h^6 |r| with
-//   EPS_D <= |r| < h, or 1.
+//   Checked on [2^-124, 2^100); the spiky kernel passes h^6 |r| with
+//   EPS_D <= |r| < h, or 1, the adjoint also |r|^3.
 __device__ __forceinline__ float rcp_seq(float z) {
   const float y = rcp_hw(z);
   const float e = fmaf(-z, y, 1.0f);

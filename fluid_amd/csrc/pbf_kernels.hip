@@ -1868,7 +1868,7 @@ __global__ __launch_bounds__(kBlock) void k_nbr_stats(uint32_t n, const uint32_t
 // sequences against the IEEE operations: thread m takes significand m and
 // runs it through every binade of the checked ranges.  bad[0..2] count the
 // mismatches of the division by b (0 and [2^div_e_lo, 2^div_e_hi)), the
-// reciprocal ([2^-100, 2^100)) and the square root ([2^-96, 2^128); below
+// reciprocal ([2^-124, 2^100)) and the square root ([2^-96, 2^128); below
 // 2^-96, including 0 and the subnormals, a result neither NaN nor under
 // 2^-47 counts as a mismatch).
 __global__ __launch_bounds__(kBlock) void k_verify_math(SimConst c, float scale, int div_e_lo,
@@ -1882,7 +1882,7 @@ __global__ __launch_bounds__(kBlock) void k_verify_math(SimConst c, float scale,
     const float a = __uint_as_float(((uint32_t)(e + 127) << 23) | m);
     nd += differ(div_seq(a * scale, c.h9s, c.r9s), a / c.h9);
   }
-  for (int e = -100; e < 100; e++) {
+  for (int e = -124; e < 100; e++) {
     const float z = __uint_as_float(((uint32_t)(e + 127) << 23) | m);
     nr += differ(rcp_seq(z), 1.0f / z);
   }
