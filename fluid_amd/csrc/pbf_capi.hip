@@ -108,21 +108,25 @@ void free_device(Ctx* x) {
   x->alloc_cells = 0;
 }
 
-// Drops the captured step graphs (buffers, dt or schedule changed), once no
-// asynchronous call replays them any more.  The flat schedule then captures
-// again only after two calls of the same dt: a caller who asks for densities
-// between its calls (which swaps buffers) is not made to capture every time.
+// Drops captured steps once no asynchronous call replays them any more.
+void drop_one(Ctx* x, pbf::StepGraph& g) {
+  if (g.exec) {
+    (void)hipStreamSynchronize(x->stream);
+    (void)hipGraphExecDestroy(g.exec);
+  }
+  if (g.graph) (void)hipGraphDestroy(g.graph);
+  g = pbf::StepGraph{};
+}
+
+// Drops all captured steps (buffers or schedule changed).  Four steps at a
+// time, and the flat schedule's, are then captured again only after two calls
+// of the same dt: a caller who asks for densities between its calls (which
+// swaps buffers) is not made to capture every time.
 void drop_graph(Ctx* x) {
   x->last_dt1 = x->last_dtn = -1.0f;
-  if (x->graph_exec || x->graph1_exec) (void)hipStreamSynchronize(x->stream);
-  if (x->graph_exec) (void)hipGraphExecDestroy(x->graph_exec);
-  if (x->graph) (void)hipGraphDestroy(x->graph);
-  x->graph_exec = nullptr;
-  x->graph = nullptr;
-  if (x->graph1_exec) (void)hipGraphExecDestroy(x->graph1_exec);
-  if (x->graph1) (void)hipGraphDestroy(x->graph1);
-  x->graph1_exec = nullptr;
-  x->graph1 = nullptr;
+  drop_one(x, x->graph1);
+  drop_one(x, x->graph_in);
+  drop_one(x, x->graph_ins);
 }
 
 template <class T>
@@ -928,6 +932,30 @@ int sync_check(Ctx* x) {
 // Capturing four steps costs one call 0.1-1.1 ms.
 constexpr int kGraphSteps = 4;
 constexpr int64_t kFlatGraphMax = 8192;
+constexpr int kGraphLong = 40;  // steps over which the gain repays that capture
+
+// Captures steps into g, unless they are there.  inner: steps between the
+// first and the last of a call, which start from the prediction of the step
+// before and end with the next; else whole steps.
+int capture_steps(Ctx* x, const SimConst& k, float dt, int steps, bool inner, pbf::StepGraph& g) {
+  if (g.exec && g.dt == dt) return PBF_OK;
+  drop_one(x, g);
+  int rc = PBF_OK;
+  const bool has_nbrs = x->has_nbrs, tile_lists = x->tile_lists;
+  HIPCHK(x, hipStreamBeginCapture(x->stream, hipStreamCaptureModeThreadLocal));
+  for (int s = 0; s < steps && rc == PBF_OK; s++) rc = run_step(x, k, 0, nullptr, inner, inner);
+  x->has_nbrs = has_nbrs;  // nothing has run yet
+  x->tile_lists = tile_lists;
+  const hipError_t e = hipStreamEndCapture(x->stream, &g.graph);
+  if (rc != PBF_OK) {
+    drop_one(x, g);
+    return rc;
+  }
+  if (e != hipSuccess) return fail(x, PBF_ERR_HIP, std::string("capture: ") + hipGetErrorString(e));
+  HIPCHK(x, hipGraphInstantiate(&g.exec, g.graph, nullptr, nullptr, 0));
+  g.dt = dt;
+  return PBF_OK;
+}
 
 // Enqueues nsteps steps with the context's schedule.
 int enqueue_steps(Ctx* x, float dt, int nsteps) {
@@ -941,40 +969,29 @@ int enqueue_steps(Ctx* x, float dt, int nsteps) {
     x->has_nbrs = true;
     x->tile_lists = false;
     x->dbg_vel = x->d.velA;
-  } else if (nsteps >= kGraphSteps + 2 &&
-             (x->schedule == PBF_SCHED_GRAPH ||
-              (x->schedule == PBF_SCHED_FLAT && x->step_graph && x->n <= kFlatGraphMax &&
-               dt == x->last_dtn))) {
+  } else if ((x->schedule == PBF_SCHED_GRAPH && nsteps >= 3) ||
+             (x->schedule == PBF_SCHED_FLAT && x->step_graph && x->n <= kFlatGraphMax &&
+              nsteps >= kGraphSteps + 2 && dt == x->last_dtn)) {
     // The first step (it predicts) and the last (it commits without
-    // predicting) are plain launches; the steps between replay kGraphSteps
-    // captured steps at a time that start from the prediction fused into
-    // the previous step and end with the next one, as the flat schedule
-    // runs them, and what is left over is launched.  The flat schedule does
-    // so once a second call of several steps in a row has the same dt.
-    x->last_dtn = dt;
+    // predicting) are plain launches; the steps between replay captured
+    // ones, which start from the prediction fused into the previous step and
+    // end with the next one, as the flat schedule runs them.  The graph
+    // schedule replays one step at a time in calls too short for
+    // kGraphSteps, and in the first call of a dt that does not repay the
+    // longer capture (a caller who changes dt captures one step a call);
+    // else, and in the flat schedule from the second call in a row with the
+    // same dt, kGraphSteps are replayed at a time and the rest is launched.
+    const int inner = nsteps - 2;
+    const bool four = inner >= kGraphSteps && (dt == x->last_dtn || inner >= kGraphLong);
+    const int many = four ? inner / kGraphSteps : 0, one = four ? 0 : inner;
+    pbf::StepGraph& g = four ? x->graph_ins : x->graph_in;
+    if (g.dt != dt) drop_one(x, g);  // waits, so before the first step
+    if (inner >= kGraphSteps) x->last_dtn = dt;
     int rc = run_step(x, k, 0, nullptr, false, true);
+    if (rc == PBF_OK) rc = capture_steps(x, k, dt, four ? kGraphSteps : 1, true, g);
     if (rc != PBF_OK) return rc;
-    if (!x->graph_exec || x->graph_dt != dt) {
-      drop_graph(x);
-      x->last_dtn = dt;
-      HIPCHK(x, hipStreamBeginCapture(x->stream, hipStreamCaptureModeThreadLocal));
-      for (int s = 0; s < kGraphSteps && rc == PBF_OK; s++)
-        rc = run_step(x, k, 0, nullptr, true, true);
-      hipGraph_t g = nullptr;
-      const hipError_t e = hipStreamEndCapture(x->stream, &g);
-      if (rc != PBF_OK) {
-        if (g) (void)hipGraphDestroy(g);
-        return rc;
-      }
-      if (e != hipSuccess) return fail(x, PBF_ERR_HIP, std::string("capture: ") + hipGetErrorString(e));
-      x->graph = g;
-      HIPCHK(x, hipGraphInstantiate(&x->graph_exec, g, nullptr, nullptr, 0));
-      x->graph_dt = dt;
-    }
-    int s = 1;
-    for (; s + kGraphSteps < nsteps; s += kGraphSteps)
-      HIPCHK(x, hipGraphLaunch(x->graph_exec, x->stream));
-    for (; s < nsteps; s++)
+    for (int s = 0; s < many + one; s++) HIPCHK(x, hipGraphLaunch(g.exec, x->stream));
+    for (int s = 1 + many * kGraphSteps + one; s < nsteps; s++)
       if ((rc = run_step(x, k, 0, nullptr, true, s + 1 < nsteps)) != PBF_OK) return rc;
   } else if (nsteps == 1 &&
              (x->schedule == PBF_SCHED_GRAPH ||
@@ -985,26 +1002,9 @@ int enqueue_steps(Ctx* x, float dt, int nsteps) {
     // so once a second one-step call in a row has the same dt, so that a
     // caller who changes dt every call is not made to capture every call.
     x->last_dt1 = dt;
-    if (!x->graph1_exec || x->graph1_dt != dt) {
-      if (x->graph1_exec) (void)hipStreamSynchronize(x->stream);
-      if (x->graph1_exec) (void)hipGraphExecDestroy(x->graph1_exec);
-      if (x->graph1) (void)hipGraphDestroy(x->graph1);
-      x->graph1_exec = nullptr;
-      x->graph1 = nullptr;
-      HIPCHK(x, hipStreamBeginCapture(x->stream, hipStreamCaptureModeThreadLocal));
-      const int rc = run_step(x, k, 0, nullptr, false, false);
-      hipGraph_t g = nullptr;
-      const hipError_t e = hipStreamEndCapture(x->stream, &g);
-      if (rc != PBF_OK) {
-        if (g) (void)hipGraphDestroy(g);
-        return rc;
-      }
-      if (e != hipSuccess) return fail(x, PBF_ERR_HIP, std::string("capture: ") + hipGetErrorString(e));
-      x->graph1 = g;
-      HIPCHK(x, hipGraphInstantiate(&x->graph1_exec, g, nullptr, nullptr, 0));
-      x->graph1_dt = dt;
-    }
-    HIPCHK(x, hipGraphLaunch(x->graph1_exec, x->stream));
+    const int rc = capture_steps(x, k, dt, 1, false, x->graph1);
+    if (rc != PBF_OK) return rc;
+    HIPCHK(x, hipGraphLaunch(x->graph1.exec, x->stream));
     // What run_step notes of a step on the host: a load since the capture
     // has taken it back.
     x->has_nbrs = true;
@@ -1012,7 +1012,7 @@ int enqueue_steps(Ctx* x, float dt, int nsteps) {
     x->dbg_pred = x->d.predP;
     x->dbg_vel = x->d.velA;
   } else {
-    // Flat schedule, and the graph schedule for calls of a few steps.
+    // Flat schedule, and the graph schedule for calls of two steps.
     if (nsteps == 1) x->last_dt1 = dt;
     if (nsteps >= kGraphSteps + 2) x->last_dtn = dt;
     for (int s = 0; s < nsteps; s++) {

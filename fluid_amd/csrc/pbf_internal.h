@@ -159,6 +159,13 @@ constexpr int kDenseSlot = 12;
 constexpr uint32_t kDenseCell = 48;
 constexpr int kDenseBuildSlot = 13;  // in a tiled step: the particles without a tile
 
+// Steps captured in a hipGraph, for one dt.
+struct StepGraph {
+  hipGraph_t graph = nullptr;
+  hipGraphExec_t exec = nullptr;
+  float dt = 0.0f;
+};
+
 struct Ctx {
   pbf_params p{};
   int nscenes = 1;
@@ -226,13 +233,10 @@ struct Ctx {
   size_t load_cap = 0;               // floats
   unsigned long long* load_bad = nullptr;
   uint32_t* flag_host = nullptr;     // pinned word the per-call overflow check reads into
-  hipGraph_t graph = nullptr;        // captured steps, for calls of several
-  hipGraphExec_t graph_exec = nullptr;
-  float graph_dt = 0.0f;
-  hipGraph_t graph1 = nullptr;       // captured whole step, for calls of one step
-  hipGraphExec_t graph1_exec = nullptr;
-  float graph1_dt = 0.0f;
-  bool step_graph = true;            // flat schedule: replay graph1 when dt repeats
+  StepGraph graph1;                  // a whole step, for calls of one step
+  StepGraph graph_in;                // an inner step of calls of several
+  StepGraph graph_ins;               // kGraphSteps inner steps
+  bool step_graph = true;            // flat schedule: replay captured steps when dt repeats
   float last_dt1 = -1.0f;            // dt of the previous one-step call
   float last_dtn = -1.0f;            // dt of the previous call of several steps
   std::string err;

@@ -124,9 +124,15 @@ PBF_API int pbf_set_mesh(pbf_ctx *ctx, const float *pos, const float *nrm, int64
  * No counterpart in the reference (batched extension). */
 enum {
   PBF_SCHED_FLAT = 0,       /* one launch per pass over all scenes (default) */
-  PBF_SCHED_GRAPH = 1,      /* the flat launches of a step captured once in a
-                               hipGraph and replayed for every step of a call
-                               but its first and last (plain launches) */
+  PBF_SCHED_GRAPH = 1,      /* the flat launches of a step captured in a
+                               hipGraph and replayed for the steps of a call
+                               between its first and last (plain launches):
+                               one step at a time, or four once a dt repeats
+                               or the call is long (then up to three are
+                               launched); a call of one step replays a whole
+                               step, one of two is launched.  The flat
+                               schedule replays for small states, too, from
+                               the second call in a row of the same dt */
   PBF_SCHED_PERSISTENT = 2  /* one launch for all steps: each workgroup runs
                                whole scenes, largest first, all passes */
 };
