@@ -306,21 +306,20 @@ int finish_create(Ctx* x, pbf_ctx** out) {
   // PBF_STEP_GRAPH=0: the flat schedule replays no captured steps.
   if (const char* w = getenv("PBF_STEP_GRAPH")) x->step_graph = w[0] != '0';
   if (const char* w = getenv("PBF_WIDE_MAX"))
-    for (pbf::PassRule& r : x->rules) r.wave_max = r.wave_multi = atoll(w);
+    for (pbf::PassRule& r : x->rules) r.wave_max = atoll(w);
   if (const char* w = getenv("PBF_QUAD_MAX"))
     for (pbf::PassRule& r : x->rules) r.quad_max = atoll(w);
   // PBF_TILE_MIN=n: states of at least n particles step on LDS tiles.
   if (const char* w = getenv("PBF_TILE_MIN")) x->tile_min = atoll(w);
   if (const char* w = getenv("PBF_DENSE_LIST")) x->dense_list = (uint32_t)atoll(w);
   if (const char* w = getenv("PBF_DENSE_CELL")) x->dense_cell = (uint32_t)atoll(w);
-  // PBF_RULE_<PASS>=wave_max,quad_max sets one pass's bounds (wave_max for
-  // states of several scenes too).
+  // PBF_RULE_<PASS>=wave_max,quad_max sets one pass's bounds.
   static const char* const kRuleEnv[pbf::kListPasses] = {
       "PBF_RULE_BUILD", "PBF_RULE_LAMBDA", "PBF_RULE_DELTAP", "PBF_RULE_XSPH", "PBF_RULE_VORT"};
   for (int k = 0; k < pbf::kListPasses; k++) {
     long long wm = 0, qm = 0;
     if (const char* w = getenv(kRuleEnv[k]))
-      if (sscanf(w, "%lld,%lld", &wm, &qm) == 2) x->rules[k] = {wm, qm, wm};
+      if (sscanf(w, "%lld,%lld", &wm, &qm) == 2) x->rules[k] = {wm, qm};
   }
   if (verify_math(x) != PBF_OK) {
     std::string m = x->err;

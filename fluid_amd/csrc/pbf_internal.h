@@ -99,14 +99,14 @@ struct DevState {
 //   XSPH                   8,192:  5.5 / 7.8 / 13.9   16,384:  8.3 / 7.7 / 13.9
 //                         65,536:  -   / 12.6 / 15.2 131,072:  -   / 21.2 / 19.1
 //   vorticity              8,192: 10.3 / -   / 11.6   16,384: 13.8 / -    / 11.9
-// With the arguments preloaded (PBF_LIST_PARAMS) and the vorticity quad that
-// carries the prediction, wave / quad by events (+3 us) on the same blocks:
-//   build + first lambda  12,288: 19.4 / 22.9  16,384: 22.5 / 23.0  20,011: 25.7 / 24.3
-//   lambda                 8,192:  7.0 / 8.0   12,288:  8.5 / 8.0
-//   vorticity              4,096: 10.2 / 9.9    6,000: 10.8 / 9.9    8,192: 11.3 / 9.5
-//                         12,288: 13.4 / 9.3
 //   vorticity commit      16,384:  -   / 5.7 / 10.9   32,768:  -   / 6.6 / 11.3
 //                         65,536:  -   / 8.9 / 11.9   98,304:  -   / 13.6 / 12.6
+// Longer lists move the lines up, so they lie on the long side for blocks at
+// rest: lines of 16,384 (build), 11,264 (lambda) and 6,144 (vorticity) gained
+// 1% on such states and lost on dams once their column had compressed (800
+// steps; us per step, these lines / those: 20,011 particles at 34 neighbours
+// 98.7 / 97.4, at 69 262 / 291, at 120 379 / 416; 12,000 at 66 168 / 184; 6,500
+// at 57 99 / 106).
 // PBF_WIDE_MAX (every pass's wave_max), PBF_QUAD_MAX (every quad_max) and
 // PBF_RULE_<PASS>=wave_max,quad_max override them at context creation; 0
 // turns a variant off.
@@ -114,14 +114,13 @@ enum ListPass : int { kPassBuild, kPassLambda, kPassDeltap, kPassXsph, kPassVort
 struct PassRule {
   int64_t wave_max;
   int64_t quad_max;
-  int64_t wave_multi;  // wave_max of states of several scenes (no quads there)
 };
 constexpr PassRule kPassRules[kListPasses] = {
-    {16384, 114688, 20480},  // build + first lambda
-    {11264, 114688, 12288},  // lambda
-    {8192, 114688, 8192},    // delta-p
-    {12288, 114688, 12288},  // XSPH
-    {6144, 81920, 12288},    // vorticity (+ commit, + prediction)
+    {20480, 114688},  // build + first lambda
+    {12288, 114688},  // lambda
+    {8192, 114688},   // delta-p
+    {12288, 114688},  // XSPH
+    {12288, 81920},   // vorticity (+ commit, + prediction)
 };
 // The vorticity pass that carries the next step's prediction takes its quad
 // only up to this many particles: its histogram slots cost a quad one

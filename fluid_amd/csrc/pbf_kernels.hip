@@ -2022,7 +2022,7 @@ hipError_t launch_scatter_rank(Ctx& x, const float4* pred) {
 // k_*_quad, single scenes) or 1.
 static int lanes(const Ctx& x, ListPass p) {
   const PassRule& r = x.rules[p];
-  if (x.n <= (x.nscenes == 1 ? r.wave_max : r.wave_multi)) return 64;
+  if (x.n <= r.wave_max) return 64;
   // Quad kernels index 4n threads in 32 bits.
   if (x.nscenes == 1 && x.n <= r.quad_max && x.n < (int64_t{1} << 30)) return 4;
   return 1;
