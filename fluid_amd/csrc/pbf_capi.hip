@@ -103,7 +103,7 @@ void free_device(Ctx* x) {
   dfree(d.nbr); dfree(d.ncnt); dfree(d.flags);
   dfree(d.grids); dfree(d.first); dfree(d.slotScene); dfree(d.runs); dfree(d.stage); dfree(d.dense);
   dfree(d.dense_b);
-  dfree(d.titem); dfree(d.trec); dfree(d.town); dfree(d.tnbr); dfree(d.tflag);
+  dfree(d.titem); dfree(d.trec); dfree(d.town); dfree(d.tnbr);
   x->alloc_n = 0;
   x->alloc_cells = 0;
 }
@@ -148,9 +148,8 @@ void alloc_tiles(Ctx* x) {
   if (e == hipSuccess) e = dalloc(d.trec, items);
   if (e == hipSuccess) e = dalloc(d.town, units * 64);
   if (e == hipSuccess) e = dalloc(d.tnbr, units * 64 * 8 * pbf::kTileChunks);
-  if (e == hipSuccess) e = dalloc(d.tflag, x->tile_blocks);
   if (e != hipSuccess) {
-    dfree(d.titem); dfree(d.trec); dfree(d.town); dfree(d.tnbr); dfree(d.tflag);
+    dfree(d.titem); dfree(d.trec); dfree(d.town); dfree(d.tnbr);
     (void)hipGetLastError();
     return;
   }
@@ -1562,7 +1561,6 @@ size_t carve_state(unsigned char* base, size_t n, size_t ncell, size_t K, pbf::D
   d->dense = nullptr;  // no dense split here
   d->dense_b = nullptr;
   d->titem = nullptr;  // no LDS tiles either (tile_step): they are the context's own state's
-  d->tflag = nullptr;
   d->trec = nullptr;
   d->town = nullptr;
   d->tnbr = nullptr;

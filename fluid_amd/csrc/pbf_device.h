@@ -805,12 +805,37 @@ __device__ __forceinline__ void quad_sums(uint32_t i, int cnt, int K4,
   }
 }
 
-// Chooses the visit of the lists: pipelined or grouped by U.
+// The same visit a chunk at a time with only its next index chunk in flight:
+// the fewest registers, for kernels that carry it beside another loop.  The
+// slots past the end of the last chunk hold a particle index.
+template <class Load, class Body>
+__device__ __forceinline__ void for_each_neighbor_small(uint32_t i, int cnt, int K4,
+                                                        const uint32_t* __restrict__ nbr,
+                                                        Load load, Body body) {
+  const int nch = (cnt + 3) >> 2;
+  if (nch == 0) return;
+  uint4 e = load_chunk(nbr + nbr_chunk(i, 0, K4));
+  for (int ch = 0; ch < nch; ch++) {
+    const auto d0 = load(e.x), d1 = load(e.y), d2 = load(e.z), d3 = load(e.w);
+    uint4 en = e;
+    if (ch + 1 < nch) en = load_chunk(nbr + nbr_chunk(i, ch + 1, K4));
+    const int m = cnt - 4 * ch;
+    body(e.x, d0);
+    if (m > 1) body(e.y, d1);
+    if (m > 2) body(e.z, d2);
+    if (m > 3) body(e.w, d3);
+    e = en;
+  }
+}
+
+// Chooses the visit of the lists: pipelined, grouped by U, or small (U = 0).
 template <int U, class Load, class Body>
 __device__ __forceinline__ void visit_neighbors(uint32_t i, int cnt, int K4,
                                                 const uint32_t* __restrict__ nbr, Load load,
                                                 Body body) {
-  if (PBF_PIPE && U == 4)
+  if constexpr (U == 0)
+    for_each_neighbor_small(i, cnt, K4, nbr, load, body);
+  else if (PBF_PIPE && U == 4)
     for_each_neighbor_pipe(i, cnt, K4, nbr, load, body);
   else
     for_each_neighbor<U>(i, cnt, K4, nbr, load, body);

@@ -74,7 +74,6 @@ struct DevState {
   uint32_t* dense = nullptr;      // particles with long lists, queued by the build (n)
   uint32_t* dense_b = nullptr;    // particles in crowded cells, queued by the sort (n)
   TileItem* titem = nullptr;      // LDS tiles of the step (pbf_tiles.h)
-  uint8_t* tflag = nullptr;       // base blocks whose particles are tiled
   TileRec* trec = nullptr;        // rows of each tile
   uint2* town = nullptr;          // particle, own slot and list length of each lane
   uint16_t* tnbr = nullptr;       // lists of the tiles, as LDS byte offsets
@@ -156,7 +155,7 @@ constexpr int kDenseSlot = 12;
 // PBF_DENSE_CELL overrides the threshold (0: off).  178.2 ms at 48 and lists of
 // 96, 178.4 at 40 and 56, 178.4 at 64.
 constexpr uint32_t kDenseCell = 48;
-constexpr int kDenseBuildSlot = 13;  // in a tiled step: the particles without a tile
+constexpr int kDenseBuildSlot = 13;  // in a tiled step: the particles of sparse blocks
 
 // Steps captured in a hipGraph, for one dt.
 struct StepGraph {

@@ -72,7 +72,6 @@ struct Dev {
 // arguments do not carry.
 struct TileDev : Dev {
   TileItem* titem;
-  uint8_t* tflag;
   TileRec* trec;
   uint2* town;
   uint16_t* tnbr;
@@ -115,7 +114,6 @@ Dev dev_of(const Ctx& x) {
   if (x.tile_on) {
     d.dense = s.dense;
     d.dense_b = s.dense_b;
-    d.dense_cell = 0xffffffffu;
   }
   d.n = (uint32_t)x.n;
   d.K4 = k4_of(x);
@@ -127,7 +125,6 @@ static TileDev tile_dev_of(const Ctx& x) {
   TileDev d;
   static_cast<Dev&>(d) = dev_of(x);
   d.titem = s.titem;
-  d.tflag = s.tflag;
   d.trec = s.trec;
   d.town = s.town;
   d.tnbr = s.tnbr;
@@ -435,8 +432,8 @@ __device__ __forceinline__ void scatter_one(uint32_t i, const Dev& d) {
 // Everything the particle moves is loaded before the count, and the cell's
 // ids are read four at a time with independent loads, so the loads of one
 // particle overlap instead of waiting on each other.
-__device__ __forceinline__ uint32_t rank_one(uint32_t i, const Dev& d,
-                                             const float4* __restrict__ pred) {
+__device__ __forceinline__ void rank_one(uint32_t i, const Dev& d,
+                                         const float4* __restrict__ pred) {
   const float4 x = d.posA[i];
   const float4 v = d.move_v ? d.velA[i] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
   const float4 q = pred[i];
@@ -457,7 +454,7 @@ __device__ __forceinline__ uint32_t rank_one(uint32_t i, const Dev& d,
             (uint32_t)(t + 2 < e && a2 < id) + (uint32_t)(t + 3 < e && a3 < id);
   }
   const uint32_t dst = s + rank;
-  if (dst >= d.n) return 0xffffffffu;
+  if (dst >= d.n) return;
   d.posB[dst] = x;
   if (d.move_v) d.velB[dst] = v;
   d.predQ[dst] = q;
@@ -467,7 +464,6 @@ __device__ __forceinline__ uint32_t rank_one(uint32_t i, const Dev& d,
     const uint32_t slot = atomicAdd(&d.flags[kDenseBuildSlot], 1u);
     if (slot < d.n) d.dense_b[slot] = dst;  // each particle once per step: slot < n
   }
-  return dst;
 }
 
 // Distance from coordinate x to the near face of cell k+side of the axis
@@ -660,7 +656,7 @@ __device__ __forceinline__ float lambda_of(const SimConst& c, float dens, float 
 // newtonStepCalculateLambda (src/particles.cpp:185-204).  out = (x*, lambda).
 // x* comes from `in` (after the sort), or with PACKED from the 12-byte
 // records that the previous delta-p pass wrote (then `in` is not read).
-template <bool PACKED>
+template <bool PACKED, int U = kUnroll>
 __device__ __forceinline__ void lambda_one(uint32_t i, const Dev& d, const SimConst& c,
                                            const float4* __restrict__ in,
                                            float4* __restrict__ out) {
@@ -668,7 +664,7 @@ __device__ __forceinline__ void lambda_one(uint32_t i, const Dev& d, const SimCo
   const int cnt = (int)d.ncnt[i];
   float dens = 0.0f, denom = 0.0f, Gx = 0.0f, Gy = 0.0f, Gz = 0.0f;
   const float3* __restrict__ xs3 = d.xs3;
-  visit_neighbors<kUnroll>(
+  visit_neighbors<U>(
       i, cnt, d.K4, d.nbr,
       [&](uint32_t j) {
         if (PACKED) return at(xs3, j);
@@ -703,14 +699,14 @@ __device__ __forceinline__ void deltap_finish(uint32_t i, const Dev& d, const Si
 // iteration also forms v = (x* - x) / dt (updateVelocity, :215-217).  NT >= 0
 // is the tensile exponent N known at compile time (the scenes' 4): the
 // same products, unrolled; NT < 0 reads it from c.
-template <bool LAST, int NT = -1>
+template <bool LAST, int NT = -1, int U = kUnroll>
 __device__ __forceinline__ void deltap_one(uint32_t i, const Dev& d, const SimConst& c,
                                            const SceneGrid& g, const float4* __restrict__ in,
                                            float4* __restrict__ out) {
   const float4 xi = in[i];
   const int cnt = (int)d.ncnt[i];
   float dx = 0.0f, dy = 0.0f, dz = 0.0f;
-  visit_neighbors<kUnroll>(
+  visit_neighbors<U>(
       i, cnt, d.K4, d.nbr, [&](uint32_t j) { return at(in, j); },
       [&](uint32_t, const float4& xj) {
         float t[3];
@@ -764,6 +760,7 @@ __device__ __forceinline__ void xsph_finish(uint32_t i, const Dev& d, const SimC
 // calculateVorticityApplyXSPHViscosity (src/particles.cpp:219-234), Jacobi:
 // every neighbour velocity is the pre-XSPH v.  out = (x*, |omega|),
 // vxsph = (v + C*visc, density), vort = (omega, 0).
+template <int U = kUnroll>
 __device__ __forceinline__ void xsph_one(uint32_t i, const Dev& d, const SimConst& c,
                                          float4* __restrict__ out) {
   const float3* __restrict__ xv = reinterpret_cast<const float3*>(d.xv);
@@ -773,7 +770,7 @@ __device__ __forceinline__ void xsph_one(uint32_t i, const Dev& d, const SimCons
   struct XV {
     float3 x, v;
   };
-  visit_neighbors<kUnroll>(
+  visit_neighbors<U>(
       i, cnt, d.K4, d.nbr, [&](uint32_t j) { return XV{at(xv, 2 * j), at(xv, 2 * j + 1)}; },
       [&](uint32_t, const XV& q) {
         float t[7];
@@ -797,13 +794,14 @@ __device__ __forceinline__ void vort_finish(uint32_t i, const Dev& d, const SimC
 // in = (x*, |omega|).  Commits posA = (x*, id), velA = (v, density).
 // Returns the committed x (xyz, id) and v of particle i; writes them unless
 // the caller goes on with the next step's prediction (commit = false).
+template <int U = kUnroll>
 __device__ __forceinline__ void vort_one(uint32_t i, const Dev& d, const SimConst& c,
                                          const float4* __restrict__ in, float4* x_out = nullptr,
                                          float4* v_out = nullptr, bool commit = true) {
   const float4 xi = in[i];
   const int cnt = (int)d.ncnt[i];
   float ex = 0.0f, ey = 0.0f, ez = 0.0f;
-  visit_neighbors<kUnroll>(
+  visit_neighbors<U>(
       i, cnt, d.K4, d.nbr, [&](uint32_t j) { return at(in, j); },
       [&](uint32_t, const float4& xj) {
         float t[3];
@@ -2004,14 +2002,12 @@ static unsigned tile_grid(const Ctx& x) {
 }
 
 hipError_t launch_scatter_rank(Ctx& x, const float4* pred) {
-  const Dev d = dev_of(x);
+  Dev d = dev_of(x);
   k_scatter<<<blocks_for(x.n), kBlock, 0, x.stream>>>(d.cell, d.arrival, d.cellStart, d.posA,
                                                       d.tmpId, d.n, d, x.tile_on);
   if (x.tile_on) {
     k_tile_items<<<blocks_for(x.tile_blocks), kBlock, 0, x.stream>>>(tile_dev_of(x), x.grids[0]);
-    k_rank_tiled<<<(unsigned)((x.n + kRankBlock - 1) / kRankBlock), kRankBlock, 0, x.stream>>>(
-        tile_dev_of(x), pred ? pred : d.predP, x.grids[0]);
-    return hipGetLastError();
+    d.dense = d.dense_b = nullptr;  // the tiles have laid out both queues
   }
   k_rank<<<blocks_for(x.n), kBlock, 0, x.stream>>>(pred ? pred : d.predP, d.posA, d.cell,
                                                    d.cellStart, d.tmpId, d.n, d);

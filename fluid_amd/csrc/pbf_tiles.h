@@ -32,9 +32,11 @@
 // histogram atomics while they hold its LDS: 288 us against 260).
 //
 // Blocks that do not fit (more than kTileCap - 1 records) are cut into parts,
-// level after level; particles of nearly empty blocks, and particles whose
-// cell or list stands out of its tile, go to the queue of the dense split and
-// run on quads with global gathers.
+// level after level.  Particles of sparse blocks (fewer than kTileMin) go to a
+// queue that workgroups without a tile take, a lane per particle, with the
+// per-lane passes' lists and gathers; those of blocks that fit at no level, and
+// particles whose cell or list stands out of its tile, to the queue of the
+// dense split, a quad per particle.
 #pragma once
 
 constexpr int kTX = 5, kTY = 4, kTZ = 3;   // cells of a block
@@ -44,9 +46,13 @@ constexpr uint32_t kTileWaves = kTileBlock / 64;
 // Records of a tile, the padding record included: 40 KB of 16-byte records,
 // so four workgroups (all 32 waves) share a CU's 160 KB.
 constexpr uint32_t kTileCap = 2556;
-// Particles of a tiled block: below, a workgroup's fill is worth less than
-// quads with global gathers.
-constexpr uint32_t kTileMin = 24;
+// Particles of a tiled block: below, a workgroup's fill and its idle waves cost
+// more than a lane per particle with global gathers (1,000,000 particles, ms per
+// step, per-lane passes / this line / 24: random at 20 a block 0.34 / 0.42 / 1.04,
+// at 100 0.50 / 0.61 / 1.07, at 200 0.64 / 0.80 / 0.80, at 480 0.98 / 0.74 / 0.74;
+// the dam's first and last 30 of 120 steps 0.94, 1.40 / 0.75, 1.35 / 0.75, 1.39;
+// lines of 200 and 256 are slower at 480 a block, 0.78 and 0.80).
+constexpr uint32_t kTileMin = 128;
 constexpr int kTileLevels = 6;
 constexpr unsigned kTileQuads = 256;      // workgroups of a pass that take the queue
 constexpr unsigned kQueueBuildGrid = 2048;
@@ -194,6 +200,41 @@ __global__ __launch_bounds__(kBlock) void k_tile_items(TileDev d, SceneGrid g) {
   const bool tiled = level >= 0 && bi + m <= d.tile_items && bu + w <= d.tile_units;
   if (level == 0 && bi < d.tile_items)
     d.titem[bi] = tile_item(x0, y0, z0, kTX, kTY, kTZ, bu, tiled ? N : 0u);
+  // Particles of sparse blocks, in block order, to the queue of the lanes.
+  const uint32_t sn = N < kTileMin ? N : 0u, is = wave_incl_scan(sn), ts = __shfl(is, 63);
+  uint32_t sb = 0;
+  if (lane == 0 && ts) sb = atomicAdd(&d.flags[kDenseBuildSlot], ts);
+  uint32_t slot = __shfl(sb, 0) + is - sn;
+  if (sn) {
+    for (int r = 0; r < kTY * kTZ; r++) {
+      const int y = y0 + r % kTY, z = z0 + r / kTY;
+      if (y >= g.dims[1] || z >= g.dims[2]) continue;
+      const uint32_t* c = d.cellStart + g.cell_base +
+                          ((uint32_t)z * (uint32_t)g.dims[1] + (uint32_t)y) * (uint32_t)g.dims[0];
+      for (uint32_t j = c[x0], e = c[min(x0 + kTX, g.dims[0])]; j < e; j++, slot++)
+        if (slot < d.n) d.dense_b[slot] = j;  // each particle once per step: slot < n
+    }
+  }
+  // Those of blocks that fit at no level, or beyond the capacity, to the
+  // queue of the quads, a wave per block.
+  for (unsigned long long s = __ballot(N >= kTileMin && !tiled); s; s &= s - 1ull) {
+    const int l = __ffsll((long long)s) - 1;
+    const int bx = __shfl(x0, l), by = __shfl(y0, l), bz = __shfl(z0, l);
+    const uint32_t all = __shfl(N, l);
+    uint32_t q = 0;
+    if (lane == 0) q = atomicAdd(&d.flags[kDenseSlot], all);
+    q = __shfl(q, 0);
+    for (int r = 0; r < kTY * kTZ; r++) {
+      const int y = by + r % kTY, z = bz + r / kTY;
+      if (y >= g.dims[1] || z >= g.dims[2]) continue;
+      const uint32_t* c = d.cellStart + g.cell_base +
+                          ((uint32_t)z * (uint32_t)g.dims[1] + (uint32_t)y) * (uint32_t)g.dims[0];
+      const uint32_t j = c[bx], m = c[min(bx + kTX, g.dims[0])] - j;
+      for (uint32_t k = (uint32_t)lane; k < m; k += 64u)
+        if (q + k < d.n) d.dense[q + k] = j + k;
+      q += m;
+    }
+  }
   for (unsigned long long s = __ballot(level > 0); s; s &= s - 1ull) {
     const int l = __ffsll((long long)s) - 1;
     const int bx = __shfl(x0, l), by = __shfl(y0, l), bz = __shfl(z0, l);
@@ -206,18 +247,6 @@ __global__ __launch_bounds__(kBlock) void k_tile_items(TileDev d, SceneGrid g) {
       d.titem[i] = tile_item(bx + p.px, by + p.py, bz + p.pz, min(p.px + p.sx, kTX) - p.px, p.sy,
                              p.sz, first + (ex & 0xffffu), ok ? p.pn : 0u);
   }
-  if (b < nb) d.tflag[b] = tiled ? 1 : 0;
-}
-
-// Whether the base block of cell c is tiled.
-__device__ __forceinline__ bool cell_tiled(const TileDev& d, const SceneGrid& g, uint32_t c) {
-  const uint32_t l = c - g.cell_base;
-  const uint32_t nx = (uint32_t)g.dims[0], ny = (uint32_t)g.dims[1];
-  const uint32_t r = l / nx, x = l - r * nx;
-  const uint32_t z = r / ny, y = r - z * ny;
-  uint32_t nbx, nby;
-  tile_blocks(g, &nbx, &nby);
-  return d.tflag[((z / kTZ) * nby + y / kTY) * nbx + x / kTX] != 0;
 }
 
 // Appends i to a queue (count in flags[slot]) for the lanes with q set (every
@@ -235,35 +264,7 @@ __device__ __forceinline__ void wave_queue(const TileDev& d, uint32_t* queue, in
   if (q && slot < d.n) queue[slot] = i;
 }
 
-// The rank pass of a tiled step: particles of the blocks without a tile go
-// to the queue, one counter atomic per workgroup.
-constexpr int kRankBlock = 1024;
-__global__ __launch_bounds__(kRankBlock) void k_rank_tiled(TileDev d, const float4* pred, SceneGrid g) {
-  __shared__ uint32_t cnt[kRankBlock / 64 + 1];
-  const uint32_t i = blockIdx.x * kRankBlock + threadIdx.x;
-  uint32_t dst = 0xffffffffu;
-  if (i < d.n) dst = rank_one(i, d, pred);
-  const bool q = dst != 0xffffffffu && !cell_tiled(d, g, d.cell[i]);
-  const unsigned long long mask = __ballot(q);
-  const uint32_t lane = __lane_id(), wid = threadIdx.x >> 6;
-  if (lane == 0) cnt[wid] = (uint32_t)__popcll(mask);
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    uint32_t t = 0;
-    for (int w = 0; w < kRankBlock / 64; w++) {
-      const uint32_t k = cnt[w];
-      cnt[w] = t;
-      t += k;
-    }
-    cnt[kRankBlock / 64] = t ? atomicAdd(&d.flags[kDenseBuildSlot], t) : 0u;
-  }
-  __syncthreads();
-  const uint32_t slot =
-      cnt[kRankBlock / 64] + cnt[wid] + (uint32_t)__popcll(mask & ((1ull << lane) - 1ull));
-  if (q && slot < d.n) d.dense_b[slot] = dst;  // each particle once per step
-}
-
-// Workgroup b of a pass takes item tile_order(b), then every gridDim - kTileQuads
+// Workgroup b of the G that take tiles runs item tile_order(b), then every G
 // items further: the XCDs take runs of kTileRun items in turn.
 __device__ __forceinline__ uint32_t tile_order(uint32_t b) {
   return (b & ~(8u * kTileRun - 1u)) + (b & 7u) * kTileRun + ((b >> 3) & (kTileRun - 1u));
@@ -273,6 +274,18 @@ __device__ __forceinline__ uint32_t tile_span(uint32_t ni) {
 }
 __device__ __forceinline__ uint32_t tile_count(const TileDev& d) {
   return min(d.flags[kTileItemsSlot], d.tile_items);
+}
+// The particles of sparse blocks, a lane each, in chunks of kTileBlock over the
+// G workgroups that take tiles, from the first that has none on.
+template <class F>
+__device__ __forceinline__ void tile_lanes(const TileDev& d, uint32_t b, uint32_t G, F f) {
+  const uint32_t nq = min(d.flags[kDenseBuildSlot], d.n);
+  const uint32_t nc = (nq + (uint32_t)kTileBlock - 1u) / (uint32_t)kTileBlock;
+  const uint32_t first = tile_span(tile_count(d)) % G;
+  for (uint32_t k = b >= first ? b - first : b + G - first; k < tile_span(nc); k += G) {
+    const uint32_t q = tile_order(k) * (uint32_t)kTileBlock + threadIdx.x;
+    if (q < nq) f(d.dense_b[q]);
+  }
 }
 // The wave's index in its workgroup, known to be uniform: what it addresses
 // comes through scalar loads into scalar registers.
@@ -513,22 +526,10 @@ __global__ __launch_bounds__(kTileBlock, 6) void k_tile_build(TileDev d, SimCons
   __shared__ uint32_t cs[kTRows][8];
   __shared__ uint32_t rowO[kTRows];
   __shared__ uint32_t intr[kTY * kTZ + 1];
-  if (blockIdx.x < kTileQuads) {
-    // The particles without a tile, a quad each.
-    const uint32_t qn = min(d.flags[kDenseBuildSlot], d.n);
-    for (uint32_t q = blockIdx.x * (kTileBlock / 4) + (threadIdx.x >> 2); q < qn;
-         q += kTileQuads * (kTileBlock / 4)) {
-      const uint32_t i = d.dense_b[q];
-      nbr_quad_one<16>(i, d, c0.h2, g);
-      __threadfence_block();
-      lambda_quad_one<false>(i, d, c0, d.predQ, out);
-    }
-    return;
-  }
   const SimConst c = tile_const(c0);
   const uint32_t ni = tile_count(d);
   const uint32_t tid = threadIdx.x, wave = tile_wave(), lane = tid & 63u;
-  for (uint32_t b = blockIdx.x - kTileQuads; b < tile_span(ni); b += gridDim.x - kTileQuads) {
+  for (uint32_t b = blockIdx.x; b < tile_span(ni); b += gridDim.x) {
     const uint32_t item = tile_order(b);
     if (item >= ni) continue;
     const TileItem it = d.titem[item];
@@ -699,23 +700,29 @@ __global__ __launch_bounds__(kTileBlock, 6) void k_tile_build(TileDev d, SimCons
     }
     __syncthreads();
   }
+  tile_lanes(d, blockIdx.x, gridDim.x, [&](uint32_t i) {
+    nbr_one(i, d, c0.h2, g);
+    lambda_one<false, 0>(i, d, c0, d.predQ, out);
+  });
 }
 
-// The first kTileQuads workgroups of a pass take the particles without a
-// tile list (both queues), a quad each.
+// The first kTileQuads workgroups of a pass take the queue of long lists, a
+// quad each.
 template <class F>
 __device__ __forceinline__ bool tile_queue(const TileDev& d, F f) {
   if (blockIdx.x >= kTileQuads) return false;
-  const uint32_t nb = min(d.flags[kDenseBuildSlot], d.n), nl = min(d.flags[kDenseSlot], d.n);
-  for (uint32_t q = blockIdx.x * (kTileBlock / 4) + (threadIdx.x >> 2); q < nb + nl;
+  const uint32_t nl = min(d.flags[kDenseSlot], d.n);
+  for (uint32_t q = blockIdx.x * (kTileBlock / 4) + (threadIdx.x >> 2); q < nl;
        q += kTileQuads * (kTileBlock / 4))
-    f(q < nb ? d.dense_b[q] : d.dense[q - nb]);
+    f(d.dense[q]);
   return true;
 }
 
-// Runs unit(head) for every unit of every tile of this workgroup.
-template <class Load, class Store, class Unit>
-__device__ __forceinline__ void tile_run(const TileDev& d, Load load, Store store, Unit unit) {
+// Runs unit(head) for every unit of every tile of this workgroup, then
+// lane(i) for its particles of sparse blocks.
+template <class Load, class Store, class Unit, class Lane>
+__device__ __forceinline__ void tile_run(const TileDev& d, Load load, Store store, Unit unit,
+                                         Lane lane) {
   const uint32_t wave = tile_wave(), step = gridDim.x - kTileQuads;
   const uint32_t ni = tile_count(d);
   for (uint32_t b = blockIdx.x - kTileQuads; b < tile_span(ni); b += step) {
@@ -729,6 +736,7 @@ __device__ __forceinline__ void tile_run(const TileDev& d, Load load, Store stor
     }
     __syncthreads();  // the next tile's fill
   }
+  tile_lanes(d, blockIdx.x - kTileQuads, step, lane);
 }
 
 // The passes after the build: lambda_one<true>, deltap_one, xsph_one and
@@ -736,7 +744,7 @@ __device__ __forceinline__ void tile_run(const TileDev& d, Load load, Store stor
 // records in flight per lane; four need 78 VGPRs, 198 us against 189), the
 // others run three (delta-p, at 80 VGPRs) or two (XSPH, whose records take
 // 60 KB).
-__global__ __launch_bounds__(kTileBlock) void k_tile_lambda(TileDev d, SimConst c0, float4* out) {
+__global__ __launch_bounds__(kTileBlock, 8) void k_tile_lambda(TileDev d, SimConst c0, float4* out) {
   __shared__ float4 rec[kTileCap + 4];
   if (tile_queue(d, [&](uint32_t i) { lambda_quad_one<true>(i, d, c0, nullptr, out); })) return;
   const SimConst c = tile_const(c0);
@@ -750,7 +758,8 @@ __global__ __launch_bounds__(kTileBlock) void k_tile_lambda(TileDev d, SimConst 
         const float3 xi = make_float3(x4.x, x4.y, x4.z);
         const float lam = tile_lambda(c, lp, h.q0, (int)(h.own.y >> 16), rb, xi);
         out[h.own.x] = make_float4(xi.x, xi.y, xi.z, lam);
-      });
+      },
+      [&](uint32_t i) { lambda_one<true, 0>(i, d, c0, nullptr, out); });
 }
 
 template <bool LAST, int NT>
@@ -781,7 +790,8 @@ __global__ __launch_bounds__(kTileBlock, 6) void k_tile_deltap(TileDev d, SimCon
               add(poly6_sel(c, p.r2), spiky_sel(c, p.rx, p.ry, p.rz, p.r2), q.w);
             });
         deltap_finish<LAST>(h.own.x, d, c, g, xi, dx, dy, dz);
-      });
+      },
+      [&](uint32_t i) { deltap_one<LAST, NT, 0>(i, d, c0, g, in, nullptr); });
 }
 
 __global__ __launch_bounds__(kTileBlock) void k_tile_xsph(TileDev d, SimConst c0, float4* out) {
@@ -823,7 +833,8 @@ __global__ __launch_bounds__(kTileBlock) void k_tile_xsph(TileDev d, SimConst c0
               add(poly6_sel(c, p.r2), spiky_sel(c, p.rx, p.ry, p.rz, p.r2), q);
             });
         xsph_finish(h.own.x, d, c, xi, vi, ox, oy, oz, sx, sy, sz, dens, out);
-      });
+      },
+      [&](uint32_t i) { xsph_one<0>(i, d, c0, out); });
 }
 
 __global__ __launch_bounds__(kTileBlock) void k_tile_vort(TileDev d, SimConst c0, const float4* in) {
@@ -859,7 +870,8 @@ __global__ __launch_bounds__(kTileBlock) void k_tile_vort(TileDev d, SimConst c0
               add(spiky_sel(c, p.rx, p.ry, p.rz, p.r2), q.w);
             });
         vort_finish(h.own.x, d, c, xi, ex, ey, ez, nullptr, nullptr, true);
-      });
+      },
+      [&](uint32_t i) { vort_one<0>(i, d, c0, in); });
 }
 
 // The lists of the tiles by load id (k_nbr_export's output): slots back to

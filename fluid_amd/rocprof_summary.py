@@ -30,7 +30,7 @@ PASS_OF = [
     ("k_scan_partials", "scan"),
     ("k_scan_add", "scan"),
     ("k_scatter", "sort"),
-    ("k_rank", "sort"),                 # also k_rank_tiled
+    ("k_rank", "sort"),
     ("k_tile_items", "sort"),
     ("k_tile_build", "neighbors"),      # over LDS tiles, with the first lambda
     ("k_queue_build", "neighbors"),
@@ -47,7 +47,7 @@ PASS_OF = [
 ]
 # Kernels that stand in for one another in a pass (one or the other runs in a
 # given step): averaged by dispatches like template variants, not added up.
-VARIANT_OF = {"k_vort_commit_predict": "k_vort_commit", "k_rank_tiled": "k_rank"}
+VARIANT_OF = {"k_vort_commit_predict": "k_vort_commit"}
 COPY_BYTES = 256 << 20
 
 
