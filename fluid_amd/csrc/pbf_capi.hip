@@ -308,8 +308,12 @@ int finish_create(Ctx* x, pbf_ctx** out) {
     for (pbf::PassRule& r : x->rules) r.wave_max = atoll(w);
   if (const char* w = getenv("PBF_QUAD_MAX"))
     for (pbf::PassRule& r : x->rules) r.quad_max = atoll(w);
-  // PBF_TILE_MIN=n: states of at least n particles step on LDS tiles.
-  if (const char* w = getenv("PBF_TILE_MIN")) x->tile_min = atoll(w);
+  // PBF_TILE_MIN=n: states of at least n particles step on LDS tiles, sparse
+  // ones too.
+  if (const char* w = getenv("PBF_TILE_MIN")) {
+    x->tile_min = atoll(w);
+    x->tile_forced = true;
+  }
   if (const char* w = getenv("PBF_DENSE_LIST")) x->dense_list = (uint32_t)atoll(w);
   if (const char* w = getenv("PBF_DENSE_CELL")) x->dense_cell = (uint32_t)atoll(w);
   // PBF_RULE_<PASS>=wave_max,quad_max sets one pass's bounds.
@@ -812,6 +816,21 @@ int load_check(Ctx* x, const float* xyz, const float* v, const float* rho, int64
   return PBF_OK;
 }
 
+// Enqueues a copy of the flag words into the context's pinned ones (a small
+// copy into pageable memory is staged by the runtime on every call).
+int read_flags(Ctx* x) {
+  if (!x->flag_host) HIPCHK(x, hipHostMalloc((void**)&x->flag_host, 64, hipHostMallocDefault));
+  HIPCHK(x, hipMemcpyAsync(x->flag_host, x->d.flags, pbf::kFlagWords * sizeof(uint32_t),
+                           hipMemcpyDeviceToHost, x->stream));
+  return PBF_OK;
+}
+
+// Whether a state with that many particles in thin blocks leaves the tiles
+// (half of all), or stays off them.
+bool mostly_sparse(const Ctx* x, uint32_t sparse) {
+  return (x->tile_sparse ? 5.0 : 4.0) * (double)sparse > 2.0 * (double)x->n;
+}
+
 // pbf_load, with the last densities (rho, may be NULL) restored as well.
 int load_impl(Ctx* x, const float* xyz, const float* v, const float* rho, int64_t n) {
   if (!xyz || n < 1) return fail(x, PBF_ERR_INVALID, "xyz must be non-NULL and n >= 1");
@@ -890,7 +909,15 @@ int load_impl(Ctx* x, const float* xyz, const float* v, const float* rho, int64_
   HIPCHK(x, hipMemcpyAsync(d.runs, runs.data(), runs.size() * sizeof(pbf::SceneRun),
                            hipMemcpyHostToDevice, x->stream));
   HIPCHK(x, pbf::launch_fill_u32(d.flags, 64, 0u, x->stream));
+  x->tile_sparse = false;
+  x->census_steps = 0;
+  const bool census = d.titem && !x->tile_forced;
+  if (census) {
+    HIPCHK(x, pbf::launch_tile_census(*x));
+    if ((rc = read_flags(x)) != PBF_OK) return rc;
+  }
   HIPCHK(x, hipStreamSynchronize(x->stream));
+  if (census) x->tile_sparse = mostly_sparse(x, x->flag_host[pbf::kTileSparseSlot]);
   x->sim_time = 0.0;
   x->loaded = true;
   x->debug_dirty = false;
@@ -904,12 +931,15 @@ namespace {
 
 // Waits for the stream, then reports (and clears) a neighbour-list overflow.
 int sync_check(Ctx* x) {
-  // The flag word returns through a pinned word of the context: a small
-  // copy into pageable memory is staged by the runtime on every call.
-  if (!x->flag_host) HIPCHK(x, hipHostMalloc((void**)&x->flag_host, 64, hipHostMallocDefault));
-  HIPCHK(x, hipMemcpyAsync(x->flag_host, x->d.flags, sizeof(uint32_t), hipMemcpyDeviceToHost,
-                           x->stream));
+  const int rc = read_flags(x);
+  if (rc != PBF_OK) return rc;
   HIPCHK(x, hipStreamSynchronize(x->stream));
+  if (x->d.titem && !x->tile_forced && x->has_nbrs &&
+      (x->tile_lists || x->census_steps < pbf::kTileCensus)) {
+    const bool was = x->tile_sparse;
+    x->tile_sparse = mostly_sparse(x, x->flag_host[pbf::kTileSparseSlot]);
+    if (x->tile_sparse && !was) x->census_steps = pbf::kTileCensus;  // the count is an old one
+  }
   const uint32_t over = x->flag_host[0];
   if (over == 0) return PBF_OK;
   HIPCHK(x, pbf::launch_fill_u32(x->d.flags, 1, 0u, x->stream));
@@ -936,7 +966,8 @@ constexpr int kGraphLong = 40;  // steps over which the gain repays that capture
 // first and the last of a call, which start from the prediction of the step
 // before and end with the next; else whole steps.
 int capture_steps(Ctx* x, const SimConst& k, float dt, int steps, bool inner, pbf::StepGraph& g) {
-  if (g.exec && g.dt == dt) return PBF_OK;
+  const bool tiles = pbf::tile_step(*x, k);
+  if (g.exec && g.dt == dt && g.tiles == tiles) return PBF_OK;
   drop_one(x, g);
   int rc = PBF_OK;
   const bool has_nbrs = x->has_nbrs, tile_lists = x->tile_lists;
@@ -952,6 +983,7 @@ int capture_steps(Ctx* x, const SimConst& k, float dt, int steps, bool inner, pb
   if (e != hipSuccess) return fail(x, PBF_ERR_HIP, std::string("capture: ") + hipGetErrorString(e));
   HIPCHK(x, hipGraphInstantiate(&g.exec, g.graph, nullptr, nullptr, 0));
   g.dt = dt;
+  g.tiles = tiles;
   return PBF_OK;
 }
 
@@ -983,7 +1015,8 @@ int enqueue_steps(Ctx* x, float dt, int nsteps) {
     const bool four = inner >= kGraphSteps && (dt == x->last_dtn || inner >= kGraphLong);
     const int many = four ? inner / kGraphSteps : 0, one = four ? 0 : inner;
     pbf::StepGraph& g = four ? x->graph_ins : x->graph_in;
-    if (g.dt != dt) drop_one(x, g);  // waits, so before the first step
+    // Waits, so before the first step.
+    if (g.dt != dt || g.tiles != pbf::tile_step(*x, k)) drop_one(x, g);
     if (inner >= kGraphSteps) x->last_dtn = dt;
     int rc = run_step(x, k, 0, nullptr, false, true);
     if (rc == PBF_OK) rc = capture_steps(x, k, dt, four ? kGraphSteps : 1, true, g);
@@ -1019,6 +1052,10 @@ int enqueue_steps(Ctx* x, float dt, int nsteps) {
     }
   }
   for (int s = 0; s < nsteps; s++) x->sim_time += (double)dt;
+  if (x->tile_sparse && (x->census_steps += nsteps) >= pbf::kTileCensus) {
+    x->census_steps = 0;
+    HIPCHK(x, pbf::launch_tile_census(*x));
+  }
   return PBF_OK;
 }
 

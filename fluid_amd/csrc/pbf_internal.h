@@ -36,8 +36,11 @@ struct TileRec {
   uint2 row[kTileRows];
 };
 constexpr int kTileChunks = 32;  // 16-byte list chunks of 8 entries per lane
-constexpr int kTileZeroSlot = 12;  // kDenseSlot, kDenseBuildSlot, kTileUnitsSlot, kTileItemsSlot
+constexpr int kTileZeroSlot = 11, kTileZeroWords = 5;  // all of these, kDenseSlot, kDenseBuildSlot
 constexpr int kTileUnitsSlot = 14, kTileItemsSlot = 15;  // low and high word of one counter
+constexpr int kTileSparseSlot = 11;  // particles of thin blocks (kTileFull, launch_tile_census)
+constexpr int kTileCensus = 32;
+constexpr int kFlagWords = 16;       // the words of flags that a sync reads back
 
 // Device state of one context.  All particle arrays are float4 and are kept
 // in cell-sorted order between steps; posA.w carries the particle's load
@@ -162,6 +165,7 @@ struct StepGraph {
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   float dt = 0.0f;
+  bool tiles = false;  // its steps run on LDS tiles
 };
 
 struct Ctx {
@@ -215,6 +219,16 @@ struct Ctx {
   // per step, per-lane passes / tiles: 300,000 particles 0.341 / 0.345, 350,000
   // 0.397 / 0.385, 400,000 0.451 / 0.417, 700,000 0.695 / 0.578).
   int64_t tile_min = 400000;
+  // States with most of their particles in thin blocks (below kTileFull) keep
+  // the per-lane passes: those are up to a third faster there, the tiles where
+  // blocks are full (1,000,000 random particles, ms per step, per-lane / tiles:
+  // 20 a block 0.34 / 0.42, 100 0.50 / 0.61, 150 0.58 / 0.85, 250 0.70 / 0.78, 350
+  // 0.81 / 0.77, 480 0.98 / 0.74).  Known from a count at the load and from the
+  // last steps' tiles; while tiles are off, from a count every kTileCensus
+  // steps.  Which passes run changes no bit.
+  bool tile_sparse = false;
+  bool tile_forced = false;          // PBF_TILE_MIN is set: tiles whatever the density
+  int census_steps = 0;              // steps since the last count
   uint32_t tile_cap = 0;             // items allocated
   uint32_t tile_units = 0;           // units allocated
   // Density-field output on the device, kept between calls, and two pinned
@@ -318,9 +332,12 @@ hipError_t launch_nbr_stats(Ctx& x, unsigned long long* sum, uint32_t* mx);
 // Exclusive scan of in[0..n) into out[0..n], out[n] = total; with clear_in
 // the counts are zero afterwards.
 hipError_t launch_scan_u32(uint32_t* in, uint32_t* out, uint32_t n, uint32_t* partials,
-                           hipStream_t s, bool clear_in = false, uint32_t* zero4 = nullptr);
+                           hipStream_t s, bool clear_in = false, uint32_t* zero = nullptr);
 // Whether a step of x runs on LDS tiles; base blocks of one scene's grid.
 bool tile_step(const Ctx& x, const SimConst& c);
+// Counts the committed particles in thin blocks into flags[kTileSparseSlot]
+// (overwrites the cell histogram, which every call's first prediction clears).
+hipError_t launch_tile_census(Ctx& x);
 size_t tile_block_count(const SceneGrid& g);
 
 }  // namespace pbf

@@ -179,9 +179,9 @@ constexpr int kScanTile = kBlock * kScanItems;
 __global__ __launch_bounds__(kBlock) void k_scan_block(uint32_t* __restrict__ in,
                                                        uint32_t* __restrict__ out, uint32_t n,
                                                        uint32_t* __restrict__ partials, bool clear,
-                                                       uint32_t* __restrict__ zero4) {
+                                                       uint32_t* __restrict__ zero) {
   __shared__ uint32_t wsum[kBlock / 64];
-  if (zero4 && blockIdx.x == 0 && threadIdx.x < 4) zero4[threadIdx.x] = 0u;
+  if (zero && blockIdx.x == 0 && threadIdx.x < kTileZeroWords) zero[threadIdx.x] = 0u;
   const uint32_t base = blockIdx.x * kScanTile + threadIdx.x * kScanItems;
   uint32_t v[kScanItems];
   if (base + kScanItems <= n) {
@@ -1919,9 +1919,9 @@ hipError_t launch_fill_u32(uint32_t* p, size_t n, uint32_t v, hipStream_t s) {
 }
 
 hipError_t launch_scan_u32(uint32_t* in, uint32_t* out, uint32_t n, uint32_t* partials,
-                           hipStream_t s, bool clear_in, uint32_t* zero4) {
+                           hipStream_t s, bool clear_in, uint32_t* zero) {
   const uint32_t nb = (n + kScanTile - 1) / kScanTile;
-  if (nb > 0) k_scan_block<<<nb, kBlock, 0, s>>>(in, out, n, partials, clear_in, zero4);
+  if (nb > 0) k_scan_block<<<nb, kBlock, 0, s>>>(in, out, n, partials, clear_in, zero);
   if (nb > 0 && nb <= kScanFold) {
     k_scan_add<true><<<nb, kBlock, 0, s>>>(out, n, partials, nb);
     return hipGetLastError();
@@ -1992,8 +1992,19 @@ size_t tile_block_count(const SceneGrid& g) {
 }
 
 bool tile_step(const Ctx& x, const SimConst& c) {
-  return x.d.titem && x.n >= x.tile_min && c.inv_dt * x.tile_reach < 1e37f && x.fast_div && x.fast_rcp && x.fast_sqrt &&
+  return x.d.titem && x.n >= x.tile_min && !x.tile_sparse && c.inv_dt * x.tile_reach < 1e37f && x.fast_div && x.fast_rcp && x.fast_sqrt &&
          x.schedule != PBF_SCHED_PERSISTENT && !(x.small_sort && sort_in_one_workgroup(x));
+}
+
+hipError_t launch_tile_census(Ctx& x) {
+  hipError_t e = launch_fill_u32(x.d.cellCount, x.tile_blocks, 0u, x.stream);
+  if (e == hipSuccess) e = launch_fill_u32(x.d.flags + kTileSparseSlot, 1, 0u, x.stream);
+  if (e != hipSuccess) return e;
+  k_tile_census<<<blocks_for(x.n), kBlock, 0, x.stream>>>(x.d.posA, (uint32_t)x.n, x.grids[0],
+                                                          x.d.cellCount);
+  k_tile_sparse<<<blocks_for(x.tile_blocks), kBlock, 0, x.stream>>>(x.d.cellCount, x.tile_blocks,
+                                                                    x.d.flags + kTileSparseSlot);
+  return hipGetLastError();
 }
 
 static unsigned tile_grid(const Ctx& x) {

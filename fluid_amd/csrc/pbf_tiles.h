@@ -53,6 +53,9 @@ constexpr uint32_t kTileCap = 2556;
 // the dam's first and last 30 of 120 steps 0.94, 1.40 / 0.75, 1.35 / 0.75, 1.39;
 // lines of 200 and 256 are slower at 480 a block, 0.78 and 0.80).
 constexpr uint32_t kTileMin = 128;
+// Particles from which a block is worth its tile in a state full of its like
+// (Ctx::tile_sparse).
+constexpr uint32_t kTileFull = 300;
 constexpr int kTileLevels = 6;
 constexpr unsigned kTileQuads = 256;      // workgroups of a pass that take the queue
 constexpr unsigned kQueueBuildGrid = 2048;
@@ -200,6 +203,8 @@ __global__ __launch_bounds__(kBlock) void k_tile_items(TileDev d, SceneGrid g) {
   const bool tiled = level >= 0 && bi + m <= d.tile_items && bu + w <= d.tile_units;
   if (level == 0 && bi < d.tile_items)
     d.titem[bi] = tile_item(x0, y0, z0, kTX, kTY, kTZ, bu, tiled ? N : 0u);
+  const uint32_t thin = wave_incl_scan(N < kTileFull ? N : 0u);
+  if (lane == 63 && thin) atomicAdd(&d.flags[kTileSparseSlot], thin);
   // Particles of sparse blocks, in block order, to the queue of the lanes.
   const uint32_t sn = N < kTileMin ? N : 0u, is = wave_incl_scan(sn), ts = __shfl(is, 63);
   uint32_t sb = 0;
@@ -247,6 +252,29 @@ __global__ __launch_bounds__(kBlock) void k_tile_items(TileDev d, SceneGrid g) {
       d.titem[i] = tile_item(bx + p.px, by + p.py, bz + p.pz, min(p.px + p.sx, kTX) - p.px, p.sy,
                              p.sz, first + (ex & 0xffffu), ok ? p.pn : 0u);
   }
+}
+
+// The particles of every base block (block has to be zero), then of the
+// thin ones together (flags[kTileSparseSlot] likewise).
+__global__ __launch_bounds__(kBlock) void k_tile_census(const float4* __restrict__ pos, uint32_t n,
+                                                        SceneGrid g, uint32_t* __restrict__ block) {
+  const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+  uint32_t nbx, nby, b = 0xffffffffu;
+  tile_blocks(g, &nbx, &nby);
+  if (i < n) {
+    const float4 x = pos[i];
+    int c[3];
+    cell_lin(g, make_float3(x.x, x.y, x.z), c);
+    b = ((uint32_t)(c[2] / kTZ) * nby + (uint32_t)(c[1] / kTY)) * nbx + (uint32_t)(c[0] / kTX);
+  }
+  wave_run_slot(b, i < n, block);
+}
+__global__ __launch_bounds__(kBlock) void k_tile_sparse(const uint32_t* __restrict__ block,
+                                                        uint32_t nb, uint32_t* __restrict__ sum) {
+  const uint32_t b = blockIdx.x * kBlock + threadIdx.x;
+  const uint32_t c = b < nb ? block[b] : 0u;
+  const uint32_t t = wave_incl_scan(c < kTileFull ? c : 0u);
+  if ((threadIdx.x & 63u) == 63u && t) atomicAdd(sum, t);
 }
 
 // Appends i to a queue (count in flags[slot]) for the lanes with q set (every
