@@ -785,10 +785,14 @@ int load_check(Ctx* x, const float* xyz, const float* v, const float* rho, int64
   if (!x->flag_host) HIPCHK(x, hipHostMalloc((void**)&x->flag_host, 64, hipHostMallocDefault));
   if (x->nscenes > 1) {
     // The boxes and first particles of the scenes (their sizes are fixed, so
-    // this never replaces the buffers of a loaded state).
+    // this never replaces the buffers of a loaded state).  The count is the
+    // context's once the input is accepted.
+    const int64_t n0 = x->n, npad0 = x->npad;
     x->n = n;
     x->npad = (n + 63) / 64 * 64;
     const int rc = ensure_device(x);
+    x->n = n0;
+    x->npad = npad0;
     if (rc != PBF_OK) return rc;
     std::vector<uint32_t> first_of(x->offsets.begin(), x->offsets.end());
     HIPCHK(x, hipMemcpyAsync(x->d.grids, x->grids.data(), x->grids.size() * sizeof(SceneGrid),
