@@ -134,16 +134,25 @@ hipError_t dalloc(T*& p, size_t count) {
   return hipMalloc((void**)&p, std::max<size_t>(count, 1) * sizeof(T));
 }
 
-// Buffers of the LDS tiles, for states that step on them.  Without them (no
-// memory left) the state keeps the other list passes.
+// Buffers of the LDS tiles, for states that step on them: ~860 bytes a particle.
+// They are optional: where they would take more than half of the memory that
+// is free (what is left is the caller's, and this context's later buffers'),
+// the state keeps the other list passes.
 void alloc_tiles(Ctx* x) {
   pbf::DevState& d = x->d;
   x->tile_cap = x->tile_units = 0;
   const size_t n = (size_t)x->n;
   if (x->n < x->tile_min || x->tile_blocks == 0 || x->tile_blocks > n) return;
-  // A tile of 24 particles or more takes a unit per 64, so tiles this full
-  // need n / 24 units at most; blocks past the capacity go to the queue.
+  // A tile holds kTileMin = 128 particles or more (but for the parts of a cut
+  // block) and takes a unit per 64; blocks past the capacity go to the queue.
   const size_t units = n / 40 + 1024, items = n / 64 + 1024;
+  const size_t need = items * (sizeof(pbf::TileItem) + sizeof(pbf::TileRec)) +
+                      units * 64 * (sizeof(uint2) + 16 * (size_t)pbf::kTileChunks);
+  size_t avail = 0, total = 0;
+  if (hipMemGetInfo(&avail, &total) != hipSuccess || need > avail / 2) {
+    (void)hipGetLastError();
+    return;
+  }
   hipError_t e = dalloc(d.titem, items);
   if (e == hipSuccess) e = dalloc(d.trec, items);
   if (e == hipSuccess) e = dalloc(d.town, units * 64);
@@ -182,6 +191,7 @@ int ensure_device(Ctx* x) {
   DA(d.dense_b, np);
 #undef DA
   if (e != hipSuccess) {
+    (void)hipGetLastError();
     free_device(x);
     return fail(x, PBF_ERR_NOMEM, std::string("device allocation failed: ") + hipGetErrorString(e));
   }
@@ -768,20 +778,30 @@ namespace {
 // from pageable memory, ~29 GB/s, is what remains).
 constexpr int64_t kLoadDeviceMin = 3072;
 
+void free_load_buffer(Ctx* x) {
+  dfree(x->load_dev);
+  x->load_cap = 0;
+}
+
+// The buffers of a load on the device (kept between loads: 24 bytes a particle,
+// 28 with rho).  False, and the load takes the host path, where they do not fit.
+bool load_buffers(Ctx* x, size_t need) {
+  if (x->load_cap < need) {
+    free_load_buffer(x);
+    if (dalloc(x->load_dev, need) == hipSuccess) x->load_cap = need;
+  }
+  if (!x->load_bad && x->load_cap) (void)dalloc(x->load_bad, 1);
+  if (x->load_cap >= need && x->load_bad) return true;
+  (void)hipGetLastError();
+  free_load_buffer(x);
+  return false;
+}
+
 // Uploads xyz, v and rho (v, rho may be NULL) into load_dev and runs the
 // checks of host::validate_pack there.  The particle state is untouched.
 int load_check(Ctx* x, const float* xyz, const float* v, const float* rho, int64_t n, int* code,
                int64_t* first) {
-  const size_t m = (size_t)n * 3, need = 2 * m + (rho ? (size_t)n : 0);
-  if (x->load_cap < need) {
-    dfree(x->load_dev);
-    x->load_cap = 0;
-    if (dalloc(x->load_dev, need) != hipSuccess)
-      return fail(x, PBF_ERR_NOMEM, "device allocation failed: load buffer");
-    x->load_cap = need;
-  }
-  if (!x->load_bad && dalloc(x->load_bad, 1) != hipSuccess)
-    return fail(x, PBF_ERR_NOMEM, "device allocation failed: load check");
+  const size_t m = (size_t)n * 3;
   if (!x->flag_host) HIPCHK(x, hipHostMalloc((void**)&x->flag_host, 64, hipHostMallocDefault));
   if (x->nscenes > 1) {
     // The boxes and first particles of the scenes (their sizes are fixed, so
@@ -849,15 +869,21 @@ int load_impl(Ctx* x, const float* xyz, const float* v, const float* rho, int64_
   HIPCHK(x, hipSetDevice(x->device));
   // Small loads are checked and packed on the host; larger ones travel as
   // they are (24 bytes per particle instead of 36) and the device checks and
-  // packs them.
-  const bool on_device = n >= kLoadDeviceMin;
+  // packs them, unless the state and that buffer do not fit together.
+  bool on_device = n >= kLoadDeviceMin && load_buffers(x, (size_t)n * (rho ? 7 : 6));
   host::Packed pk;
   int code = PBF_OK;
   int64_t bad = 0;
   if (on_device) {
     const int rc = load_check(x, xyz, v, rho, n, &code, &bad);
-    if (rc != PBF_OK) return rc;
-  } else {
+    if (rc == PBF_ERR_NOMEM) {
+      on_device = false;
+      free_load_buffer(x);
+    } else if (rc != PBF_OK) {
+      return rc;
+    }
+  }
+  const auto on_host = [&] {
     std::vector<float> boxes;
     for (const SceneGrid& g : x->grids) {
       boxes.insert(boxes.end(), g.lo, g.lo + 3);
@@ -866,7 +892,8 @@ int load_impl(Ctx* x, const float* xyz, const float* v, const float* rho, int64_
     host::validate_pack(xyz, v, rho, n, x->offsets, boxes, 8, &pk);
     code = pk.code;
     bad = pk.first;
-  }
+  };
+  if (!on_device) on_host();
   if (code == PBF_ERR_INVALID)
     return fail(x, PBF_ERR_INVALID, "particle " + std::to_string(bad) + " is not finite");
   if (code == PBF_ERR_OUT_OF_BOX)
@@ -883,6 +910,12 @@ int load_impl(Ctx* x, const float* xyz, const float* v, const float* rho, int64_
   x->n = n;
   x->npad = (n + 63) / 64 * 64;
   int rc = ensure_device(x);
+  if (rc == PBF_ERR_NOMEM && x->load_dev) {
+    free_load_buffer(x);
+    if (on_device) on_host();
+    on_device = false;
+    rc = ensure_device(x);
+  }
   if (rc != PBF_OK) return rc;
   pbf::DevState& d = x->d;
   if (on_device) {
