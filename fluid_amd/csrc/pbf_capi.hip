@@ -950,7 +950,7 @@ int load_impl(Ctx* x, const float* xyz, const float* v, const float* rho, int64_
   x->census_steps = 0;
   const bool census = d.titem && !x->tile_forced;
   if (census) {
-    HIPCHK(x, pbf::launch_tile_census(*x));
+    HIPCHK(x, pbf::launch_tile_census(*x, false));
     if ((rc = read_flags(x)) != PBF_OK) return rc;
   }
   HIPCHK(x, hipStreamSynchronize(x->stream));

@@ -337,7 +337,8 @@ hipError_t launch_scan_u32(uint32_t* in, uint32_t* out, uint32_t n, uint32_t* pa
 bool tile_step(const Ctx& x, const SimConst& c);
 // Counts the committed particles in thin blocks into flags[kTileSparseSlot]
 // (overwrites the cell histogram, which every call's first prediction clears).
-hipError_t launch_tile_census(Ctx& x);
+// clear = false: that word is zero already.
+hipError_t launch_tile_census(Ctx& x, bool clear = true);
 size_t tile_block_count(const SceneGrid& g);
 
 }  // namespace pbf

@@ -53,6 +53,7 @@ constexpr uint32_t kTileCap = 2556;
 // the dam's first and last 30 of 120 steps 0.94, 1.40 / 0.75, 1.35 / 0.75, 1.39;
 // lines of 200 and 256 are slower at 480 a block, 0.78 and 0.80).
 constexpr uint32_t kTileMin = 128;
+constexpr uint32_t kTileFew = 24;  // sparse blocks that one thread stores
 // Particles from which a block is worth its tile in a state full of its like
 // (Ctx::tile_sparse).
 constexpr uint32_t kTileFull = 300;
@@ -67,7 +68,9 @@ constexpr uint32_t kTileRun = 8;          // consecutive tiles per XCD
 constexpr float kTileSpike = 4.0f;
 // Cells up to kTileCrowd and lists up to kTileLong never stand out.
 constexpr uint32_t kTileCrowd = 32, kTileLong = 128;
-static_assert(kTRows <= kTileRows && kTX <= 5 && kTX * kTY * kTZ <= 64 && kTileCap <= 4096, "tile");
+static_assert(kTRows <= kTileRows && kTX <= 5 && kTX * kTY * kTZ <= 64 && kTileCap <= 4096 &&
+                  kTileMin <= 128,
+              "tile");
 
 __device__ __forceinline__ uint32_t tile_blocks(const SceneGrid& g, uint32_t* nbx, uint32_t* nby) {
   *nbx = (uint32_t)(g.dims[0] + kTX - 1) / kTX;
@@ -156,6 +159,9 @@ __global__ __launch_bounds__(kBlock) void k_tile_items(TileDev d, SceneGrid g) {
   const int x0 = (int)(b % nbx) * kTX, y0 = (int)((b / nbx) % nby) * kTY,
             z0 = (int)(b / (nbx * nby)) * kTZ;
   uint32_t N = 0, H = 0;
+  uint32_t first[kTY * kTZ], len[kTY * kTZ];  // its rows
+#pragma unroll
+  for (int r = 0; r < kTY * kTZ; r++) first[r] = len[r] = 0;
   if (b < nb) {
     const int xs = max(x0 - 1, 0), xa = min(x0 + kTX, g.dims[0]),
               xe = min(x0 + kTX + 1, g.dims[0]);
@@ -165,7 +171,9 @@ __global__ __launch_bounds__(kBlock) void k_tile_items(TileDev d, SceneGrid g) {
       if (y >= g.dims[1] || z >= g.dims[2]) continue;
       const uint32_t* c = d.cellStart + g.cell_base +
                           ((uint32_t)z * (uint32_t)g.dims[1] + (uint32_t)y) * (uint32_t)g.dims[0];
-      N += c[xa] - c[x0];
+      first[r] = c[x0];
+      len[r] = c[xa] - first[r];
+      N += len[r];
     }
     if (N >= kTileMin) {
 #pragma unroll
@@ -210,15 +218,27 @@ __global__ __launch_bounds__(kBlock) void k_tile_items(TileDev d, SceneGrid g) {
   uint32_t sb = 0;
   if (lane == 0 && ts) sb = atomicAdd(&d.flags[kDenseBuildSlot], ts);
   uint32_t slot = __shfl(sb, 0) + is - sn;
-  if (sn) {
+  // (Each particle once per step, so the slots stay below n.)  A thread stores
+  // the few of its own block; the lanes of the wave store the others together.
+  if (sn && sn < kTileFew) {
+#pragma unroll
+    for (int r = 0; r < kTY * kTZ; r++)
+      for (uint32_t k = 0; k < len[r]; k++, slot++)
+        if (slot < d.n) d.dense_b[slot] = first[r] + k;
+  }
+  for (unsigned long long s = __ballot(sn >= kTileFew); s; s &= s - 1ull) {
+    const int l = __ffsll((long long)s) - 1;
+    const uint32_t q = __shfl(slot, l) + (uint32_t)lane, end = __shfl(slot + sn, l);
+    uint32_t o = (uint32_t)lane, j0 = 0, j1 = 0;  // places lane and lane + 64 of the block
+#pragma unroll
     for (int r = 0; r < kTY * kTZ; r++) {
-      const int y = y0 + r % kTY, z = z0 + r / kTY;
-      if (y >= g.dims[1] || z >= g.dims[2]) continue;
-      const uint32_t* c = d.cellStart + g.cell_base +
-                          ((uint32_t)z * (uint32_t)g.dims[1] + (uint32_t)y) * (uint32_t)g.dims[0];
-      for (uint32_t j = c[x0], e = c[min(x0 + kTX, g.dims[0])]; j < e; j++, slot++)
-        if (slot < d.n) d.dense_b[slot] = j;  // each particle once per step: slot < n
+      const uint32_t j = __builtin_amdgcn_readlane(first[r], l), m = __builtin_amdgcn_readlane(len[r], l);
+      if (o < m) j0 = j + o;
+      if (o + 64u < m) j1 = j + o + 64u;
+      o -= m;
     }
+    if (q < end && q < d.n) d.dense_b[q] = j0;
+    if (q + 64u < end && q + 64u < d.n) d.dense_b[q + 64u] = j1;
   }
   // Those of blocks that fit at no level, or beyond the capacity, to the
   // queue of the quads, a wave per block.
@@ -292,8 +312,8 @@ __device__ __forceinline__ void wave_queue(const TileDev& d, uint32_t* queue, in
   if (q && slot < d.n) queue[slot] = i;
 }
 
-// Workgroup b of the G that take tiles runs item tile_order(b), then every G
-// items further: the XCDs take runs of kTileRun items in turn.
+// Consecutive workgroups go to the XCDs in turn: a run of kTileRun consecutive
+// pieces of work for each.
 __device__ __forceinline__ uint32_t tile_order(uint32_t b) {
   return (b & ~(8u * kTileRun - 1u)) + (b & 7u) * kTileRun + ((b >> 3) & (kTileRun - 1u));
 }
@@ -303,16 +323,24 @@ __device__ __forceinline__ uint32_t tile_span(uint32_t ni) {
 __device__ __forceinline__ uint32_t tile_count(const TileDev& d) {
   return min(d.flags[kTileItemsSlot], d.tile_items);
 }
-// The particles of sparse blocks, a lane each, in chunks of kTileBlock over the
-// G workgroups that take tiles, from the first that has none on.
-template <class F>
-__device__ __forceinline__ void tile_lanes(const TileDev& d, uint32_t b, uint32_t G, F f) {
-  const uint32_t nq = min(d.flags[kDenseBuildSlot], d.n);
-  const uint32_t nc = (nq + (uint32_t)kTileBlock - 1u) / (uint32_t)kTileBlock;
-  const uint32_t first = tile_span(tile_count(d)) % G;
-  for (uint32_t k = b >= first ? b - first : b + G - first; k < tile_span(nc); k += G) {
-    const uint32_t q = tile_order(k) * (uint32_t)kTileBlock + threadIdx.x;
-    if (q < nq) f(d.dense_b[q]);
+// The work of a pass: the particles of sparse blocks, a lane each, in chunks of
+// kTileBlock, then the tiles.  Workgroup b of G takes every G-th piece, the
+// XCDs runs of kTileRun consecutive ones.  Chunks come first: as the last
+// workgroups to start, their gathers would run on after the tiles (two spheres
+// of 500,009 particles 0.45 ms per step, 0.49 in that order).
+template <class Lane, class Tile>
+__device__ __forceinline__ void tile_work(const TileDev& d, uint32_t b, uint32_t G, Lane lane,
+                                          Tile tile) {
+  const uint32_t ni = tile_count(d), nq = min(d.flags[kDenseBuildSlot], d.n);
+  const uint32_t sc = tile_span((nq + (uint32_t)kTileBlock - 1u) / (uint32_t)kTileBlock);
+  uint32_t w = b;
+  for (; w < sc; w += G) {
+    const uint32_t q = tile_order(w) * (uint32_t)kTileBlock + threadIdx.x;
+    if (q < nq) lane(d.dense_b[q]);
+  }
+  for (w -= sc; w < tile_span(ni); w += G) {
+    const uint32_t item = tile_order(w);
+    if (item < ni) tile(item);
   }
 }
 // The wave's index in its workgroup, known to be uniform: what it addresses
@@ -555,11 +583,8 @@ __global__ __launch_bounds__(kTileBlock, 6) void k_tile_build(TileDev d, SimCons
   __shared__ uint32_t rowO[kTRows];
   __shared__ uint32_t intr[kTY * kTZ + 1];
   const SimConst c = tile_const(c0);
-  const uint32_t ni = tile_count(d);
   const uint32_t tid = threadIdx.x, wave = tile_wave(), lane = tid & 63u;
-  for (uint32_t b = blockIdx.x; b < tile_span(ni); b += gridDim.x) {
-    const uint32_t item = tile_order(b);
-    if (item >= ni) continue;
+  const auto tile = [&](uint32_t item) {
     const TileItem it = d.titem[item];
     const int bx = (int)(it.dims & 15u), by = (int)((it.dims >> 4) & 15u), bz = (int)(it.dims >> 8);
     const int ry = by + 2, R = ry * (bz + 2), wx = bx + 2;
@@ -727,11 +752,14 @@ __global__ __launch_bounds__(kTileBlock, 6) void k_tile_build(TileDev d, SimCons
       }
     }
     __syncthreads();
-  }
-  tile_lanes(d, blockIdx.x, gridDim.x, [&](uint32_t i) {
-    nbr_one(i, d, c0.h2, g);
-    lambda_one<false, 0>(i, d, c0, d.predQ, out);
-  });
+  };
+  tile_work(
+      d, blockIdx.x, gridDim.x,
+      [&](uint32_t i) {
+        nbr_one(i, d, c0.h2, g);
+        lambda_one<false, 0>(i, d, c0, d.predQ, out);
+      },
+      tile);
 }
 
 // The first kTileQuads workgroups of a pass take the queue of long lists, a
@@ -746,16 +774,13 @@ __device__ __forceinline__ bool tile_queue(const TileDev& d, F f) {
   return true;
 }
 
-// Runs unit(head) for every unit of every tile of this workgroup, then
-// lane(i) for its particles of sparse blocks.
+// Runs lane(i) for this workgroup's particles of sparse blocks and unit(head)
+// for every unit of its tiles.
 template <class Load, class Store, class Unit, class Lane>
 __device__ __forceinline__ void tile_run(const TileDev& d, Load load, Store store, Unit unit,
                                          Lane lane) {
-  const uint32_t wave = tile_wave(), step = gridDim.x - kTileQuads;
-  const uint32_t ni = tile_count(d);
-  for (uint32_t b = blockIdx.x - kTileQuads; b < tile_span(ni); b += step) {
-    const uint32_t item = tile_order(b);
-    if (item >= ni) continue;
+  const uint32_t wave = tile_wave();
+  tile_work(d, blockIdx.x - kTileQuads, gridDim.x - kTileQuads, lane, [&](uint32_t item) {
     TileHead h = tile_fill(d, item, load, store);
     __syncthreads();
     for (uint32_t u = wave; u < h.nu; u += kTileWaves) {
@@ -763,15 +788,14 @@ __device__ __forceinline__ void tile_run(const TileDev& d, Load load, Store stor
       if (h.own.x != 0xffffffffu) unit(h, tile_list(d, h.unit + u));
     }
     __syncthreads();  // the next tile's fill
-  }
-  tile_lanes(d, blockIdx.x - kTileQuads, step, lane);
+  });
 }
 
 // The passes after the build: lambda_one<true>, deltap_one, xsph_one and
 // vort_one over tiles.  64 VGPRs keep four workgroups of λ on a CU (two
 // records in flight per lane; four need 78 VGPRs, 198 us against 189), the
-// others run three (delta-p, at 80 VGPRs) or two (XSPH, whose records take
-// 60 KB).
+// others run three (delta-p, at 80 VGPRs, of which it spills 8 to 16 bytes a
+// lane) or two (XSPH, whose records take 60 KB).
 __global__ __launch_bounds__(kTileBlock, 8) void k_tile_lambda(TileDev d, SimConst c0, float4* out) {
   __shared__ float4 rec[kTileCap + 4];
   if (tile_queue(d, [&](uint32_t i) { lambda_quad_one<true>(i, d, c0, nullptr, out); })) return;
