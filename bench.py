@@ -353,7 +353,7 @@ def mesh_bench(sc, warmup: int, steps: int):
     }
 
 
-def pass_table(prof, sc, steps: int, nbar: float, counters) -> dict:
+def pass_table(prof, sc, steps: int, nbar: float, counters, tiled: bool) -> dict:
     """Per pass: ms per step, launches, mean launch time and state-only and
     state+list GB/s from HIP-event times `prof` ({pass: (ms, launches)} over
     `steps` steps); HBM GB/s, VALU fraction, LDS bank-conflict rate and TA
@@ -367,8 +367,7 @@ def pass_table(prof, sc, steps: int, nbar: float, counters) -> dict:
             continue
         per_launch_s = ms / launches * 1e-3
         state = STATE_BYTES[name] * sc.n + (8 * ncell if name == "scan" else 0)
-        # Tiled lists (states of 400,000 particles or more) hold 16-bit entries.
-        entry = 2.0 if sc.n >= 400_000 else 4.0
+        entry = 2.0 if tiled else 4.0  # the tiles' lists hold 16-bit entries
         listb = (entry * nbar + 4.0) * sc.n if name in LIST_PASSES else 0.0
         pd = {
             "ms_per_step": ms / steps,
@@ -431,6 +430,7 @@ def dam_break_bench(warmup: int):
                 m0, n0 = prof.get(k, (0.0, 0))
                 prof[k] = (m0 + ms, n0 + n)
         nbar, nmax = c.neighbor_stats()
+        tiled = c.tiled()
     counters = (load_counters(sc.name) or {}).get("passes", {})
     res = {
         "workload": sc.name,
@@ -441,7 +441,7 @@ def dam_break_bench(warmup: int):
         "mean_neighbors": nbar,
         "max_neighbors": nmax,
         "windows": windows,
-        "passes": pass_table(prof, sc, steps, nbar, counters),
+        "passes": pass_table(prof, sc, steps, nbar, counters, tiled),
     }
     log(f"dam break {sc.n}: {steps} steps at {res['ms_per_step']:.3f} ms/step, neighbours "
         f"mean {nbar:.1f} max {nmax} at the end")
@@ -628,6 +628,7 @@ def main() -> int:
         log(f"profiled steps {a + 1}-{b}: {ww / (b - a) * 1e3:.3f} ms/step, neighbours "
             f"mean {wbar:.2f} max {wmax}")
     nbar, nmax = ctx.neighbor_stats()
+    tiled = ctx.tiled()
     ctx.read()  # first call allocates the pinned staging slabs
     t0 = time.perf_counter()
     ctx.read()
@@ -647,7 +648,7 @@ def main() -> int:
     snap = snapshot_bench(ctx, sc)
     ctx.close()
     counters = (load_counters(sc.name) or {}).get("passes", {})
-    passes = pass_table(prof, sc, args.steps, nbar, counters)
+    passes = pass_table(prof, sc, args.steps, nbar, counters, tiled)
     dom = max(passes, key=lambda k: passes[k]["ms_per_step"])
     d = passes[dom]
     per_launch_bytes = STATE_BYTES[dom] * sc.n

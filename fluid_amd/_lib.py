@@ -86,6 +86,7 @@ SIGNATURES = {
     "pbf_step_profiled": (C.c_int, [_P, C.c_float, C.c_int32, _F, C.POINTER(C.c_int32), C.c_int32]),
     "pbf_debug_read": (C.c_int, [_P, C.c_int32, _F]),
     "pbf_debug_derived": (C.c_int, [_P, _F, C.c_int32]),
+    "pbf_debug_tiled": (C.c_int, [_P, C.POINTER(C.c_int32)]),
 }
 
 ERRORS = {

@@ -1903,4 +1903,11 @@ PBF_API int pbf_debug_derived(const pbf_ctx* c, float* out, int32_t cap) {
   return 28;
 }
 
+PBF_API int pbf_debug_tiled(const pbf_ctx* c, int32_t* tiled) {
+  const Ctx* x = C(c);
+  if (!x || !tiled) return fail(const_cast<Ctx*>(x), PBF_ERR_INVALID, "NULL argument");
+  *tiled = x->has_nbrs && x->tile_lists;
+  return PBF_OK;
+}
+
 }  // extern "C"

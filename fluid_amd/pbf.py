@@ -214,5 +214,11 @@ class Particles:
         check(lib().pbf_debug_derived(self._ctx, _fptr(out), 32), self._ctx)
         return {"div": bool(out[25]), "rcp": bool(out[26]), "sqrt": bool(out[27])}
 
+    def tiled(self) -> bool:
+        """Whether the last step ran its list passes over LDS tiles."""
+        t = C.c_int32()
+        check(lib().pbf_debug_tiled(self._ctx, C.byref(t)), self._ctx)
+        return bool(t.value)
+
 
 PbfError = _lib.PbfError

@@ -240,8 +240,8 @@ PBF_API const char *pbf_last_error(const pbf_ctx *ctx);
  * keeps (x, v) every checkpoint_every steps; the backward pass replays each
  * segment once from its checkpoint, recording every step's sorted state,
  * neighbour lists and solver iterates in a device tape of checkpoint_every
- * slots (about (5 + 4 (iterations + 1)) * 16 + 4 (max_neighbors + 1) bytes
- * per particle each), then runs hand-written adjoint kernels of the lambda,
+ * slots (about (5 + iterations) * 16 + 4 (max_neighbors + 1) bytes per
+ * particle each), then runs hand-written adjoint kernels of the lambda,
  * delta-p, XSPH and vorticity passes over the tape in reverse. */
 typedef struct pbf_adj pbf_adj;
 PBF_API int pbf_adj_create(const pbf_params *p, int64_t n, int32_t nsteps,
@@ -332,6 +332,10 @@ PBF_API int pbf_step_profiled(pbf_ctx *ctx, float dt, int32_t nsteps, float *pas
  * and are in use (28).  Setting PBF_IEEE_MATH in the environment before
  * pbf_create keeps the IEEE expansions; both give the same bits. */
 PBF_API int pbf_debug_derived(const pbf_ctx *ctx, float *out, int32_t cap);
+
+/* Whether the last step ran its list passes over LDS tiles (measurement: a
+ * tiled list entry has 2 bytes, others 4; both give the same bits). */
+PBF_API int pbf_debug_tiled(const pbf_ctx *ctx, int32_t *tiled);
 
 #ifdef __cplusplus
 }

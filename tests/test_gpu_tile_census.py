@@ -58,3 +58,29 @@ def test_states_that_change_their_density(schedule):
             assert np.array_equal(ca, cb)
             keep = np.arange(8)[None, :] < np.minimum(ca, 8)[:, None]
             assert np.array_equal(ia[keep], ib[keep])
+
+
+def test_which_passes_run():
+    """Sparse states stay off the tiles and full ones take them, from the first
+    step after a load on; a state that spreads leaves them."""
+    r = np.random.default_rng(2)
+    p = scene_params(0.1, 0.05, (0, 0, 0), (12.0,) * 3, dt=0.005, max_neighbors=512)
+    p = p.replace(gravity=0.0)
+    gas = r.uniform(0, 12, (N, 3)).astype(np.float32)
+    k = int(np.ceil(N ** (1 / 3)))
+    block = scenes.lattice_block(k, k, k, 0.05, (4, 4, 4))[:N].astype(np.float32)
+    burst = (40.0 * (block - block.mean(0))).astype(np.float32)
+    with Particles(p) as c, plain(p) as off:
+        assert not c.tiled()
+        for x, v, first, last in ((gas, None, False, False), (block, None, True, True),
+                                  (gas, None, False, False), (block, burst, True, False)):
+            c.load(x, v)
+            assert not c.tiled()
+            c.time_step()
+            assert c.tiled() == first
+            c.time_step(nsteps=20)
+            c.time_step()
+            assert c.tiled() == last
+        off.load(block, None)
+        off.time_step()
+        assert not off.tiled()
