@@ -228,7 +228,7 @@ struct Ctx {
   // steps.  Which passes run changes no bit.
   bool tile_sparse = false;
   bool tile_forced = false;          // PBF_TILE_MIN is set: tiles whatever the density
-  int census_steps = 0;              // steps since the last count
+  int64_t census_steps = 0;          // steps since the last count
   uint32_t tile_cap = 0;             // items allocated
   uint32_t tile_units = 0;           // units allocated
   // Density-field output on the device, kept between calls, and two pinned
@@ -335,7 +335,7 @@ hipError_t launch_scan_u32(uint32_t* in, uint32_t* out, uint32_t n, uint32_t* pa
                            hipStream_t s, bool clear_in = false, uint32_t* zero = nullptr);
 // Whether a step of x runs on LDS tiles; base blocks of one scene's grid.
 bool tile_step(const Ctx& x, const SimConst& c);
-// Counts the committed particles in thin blocks into flags[kTileSparseSlot]
+// Estimates the committed particles in thin blocks in flags[kTileSparseSlot]
 // (overwrites the cell histogram, which every call's first prediction clears).
 // clear = false: that word is zero already.
 hipError_t launch_tile_census(Ctx& x, bool clear = true);
