@@ -108,14 +108,33 @@ void free_device(Ctx* x) {
   x->alloc_cells = 0;
 }
 
-// Drops captured steps once no asynchronous call replays them any more.
-void drop_one(Ctx* x, pbf::StepGraph& g) {
-  if (g.exec) {
-    (void)hipStreamSynchronize(x->stream);
-    (void)hipGraphExecDestroy(g.exec);
-  }
+void destroy_graph(pbf::StepGraph& g) {
+  if (g.exec) (void)hipGraphExecDestroy(g.exec);
   if (g.graph) (void)hipGraphDestroy(g.graph);
   g = pbf::StepGraph{};
+}
+
+// The stream has finished: captured steps that were replaced can go.
+void finished(Ctx* x) {
+  x->pending = false;
+  for (pbf::StepGraph& g : x->retired) destroy_graph(g);
+  x->retired.clear();
+}
+
+// Drops captured steps.  Those that enqueued calls may still replay are kept
+// until the next wait, so that pbf_step_async does not wait itself, up to
+// kRetired of them.
+constexpr size_t kRetired = 16;
+void drop_one(Ctx* x, pbf::StepGraph& g) {
+  if (!x->pending || !g.exec) {
+    destroy_graph(g);
+    return;
+  }
+  x->retired.push_back(g);
+  g = pbf::StepGraph{};
+  if (x->retired.size() < kRetired) return;
+  (void)hipStreamSynchronize(x->stream);
+  finished(x);
 }
 
 // Drops all captured steps (buffers or schedule changed).  Four steps at a
@@ -134,7 +153,7 @@ hipError_t dalloc(T*& p, size_t count) {
   return hipMalloc((void**)&p, std::max<size_t>(count, 1) * sizeof(T));
 }
 
-// Buffers of the LDS tiles, for states that step on them: ~860 bytes a particle.
+// Buffers of the LDS tiles, for states that step on them: ~840 bytes a particle.
 // They are optional: where they would take more than half of the memory that
 // is free (what is left is the caller's, and this context's later buffers'),
 // the state keeps the other list passes.
@@ -170,6 +189,8 @@ int ensure_device(Ctx* x) {
   if (x->alloc_n == (size_t)x->n && x->alloc_cells == (size_t)x->ncell && x->d.posA) return PBF_OK;
   // The captured steps hold these buffers' addresses; a load into the same
   // buffers keeps them.
+  if (x->pending) (void)hipStreamSynchronize(x->stream);
+  finished(x);
   drop_graph(x);
   free_device(x);
   pbf::DevState& d = x->d;
@@ -734,6 +755,7 @@ PBF_API int pbf_destroy(pbf_ctx* c) {
   if (!x) return PBF_OK;
   (void)hipSetDevice(x->device);
   if (x->stream) (void)hipStreamSynchronize(x->stream);
+  finished(x);
   drop_graph(x);
   free_device(x);
   dfree(x->d.meshTri);
@@ -971,6 +993,7 @@ int sync_check(Ctx* x) {
   const int rc = read_flags(x);
   if (rc != PBF_OK) return rc;
   HIPCHK(x, hipStreamSynchronize(x->stream));
+  finished(x);
   if (x->d.titem && !x->tile_forced && x->has_nbrs &&
       (x->tile_lists || x->census_steps < pbf::kTileCensus)) {
     const bool was = x->tile_sparse;
@@ -1028,6 +1051,7 @@ int capture_steps(Ctx* x, const SimConst& k, float dt, int steps, bool inner, pb
 int enqueue_steps(Ctx* x, float dt, int nsteps) {
   if (nsteps == 0) return PBF_OK;
   x->field_ready = false;
+  x->pending = true;
   const SimConst k = pbf::consts_for(*x, dt);
   if (x->schedule == PBF_SCHED_PERSISTENT) {
     const int per = pbf::persistent_max_blocks_per_cu(x->pblock);
@@ -1052,8 +1076,6 @@ int enqueue_steps(Ctx* x, float dt, int nsteps) {
     const bool four = inner >= kGraphSteps && (dt == x->last_dtn || inner >= kGraphLong);
     const int many = four ? inner / kGraphSteps : 0, one = four ? 0 : inner;
     pbf::StepGraph& g = four ? x->graph_ins : x->graph_in;
-    // Waits, so before the first step.
-    if (g.dt != dt || g.tiles != pbf::tile_step(*x, k)) drop_one(x, g);
     if (inner >= kGraphSteps) x->last_dtn = dt;
     int rc = run_step(x, k, 0, nullptr, false, true);
     if (rc == PBF_OK) rc = capture_steps(x, k, dt, four ? kGraphSteps : 1, true, g);

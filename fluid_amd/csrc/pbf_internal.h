@@ -248,6 +248,8 @@ struct Ctx {
   StepGraph graph1;                  // a whole step, for calls of one step
   StepGraph graph_in;                // an inner step of calls of several
   StepGraph graph_ins;               // kGraphSteps inner steps
+  std::vector<StepGraph> retired;    // replaced while enqueued steps may replay them
+  bool pending = false;              // steps enqueued since the last wait
   bool step_graph = true;            // flat schedule: replay captured steps when dt repeats
   float last_dt1 = -1.0f;            // dt of the previous one-step call
   float last_dtn = -1.0f;            // dt of the previous call of several steps
