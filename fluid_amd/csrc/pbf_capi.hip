@@ -970,13 +970,8 @@ int load_impl(Ctx* x, const float* xyz, const float* v, const float* rho, int64_
   HIPCHK(x, pbf::launch_fill_u32(d.flags, 64, 0u, x->stream));
   x->tile_sparse = false;
   x->census_steps = 0;
-  const bool census = d.titem && !x->tile_forced;
-  if (census) {
-    HIPCHK(x, pbf::launch_tile_census(*x, false));
-    if ((rc = read_flags(x)) != PBF_OK) return rc;
-  }
+  x->census_due = d.titem && !x->tile_forced;
   HIPCHK(x, hipStreamSynchronize(x->stream));
-  if (census) x->tile_sparse = mostly_sparse(x, x->flag_host[pbf::kTileSparseSlot]);
   x->sim_time = 0.0;
   x->loaded = true;
   x->debug_dirty = false;
@@ -994,7 +989,7 @@ int sync_check(Ctx* x) {
   if (rc != PBF_OK) return rc;
   HIPCHK(x, hipStreamSynchronize(x->stream));
   finished(x);
-  if (x->d.titem && !x->tile_forced && x->has_nbrs &&
+  if (x->d.titem && !x->tile_forced && !x->census_due && x->has_nbrs &&
       (x->tile_lists || x->census_steps < pbf::kTileCensus)) {
     const bool was = x->tile_sparse;
     x->tile_sparse = mostly_sparse(x, x->flag_host[pbf::kTileSparseSlot]);
@@ -1008,6 +1003,18 @@ int sync_check(Ctx* x) {
               "a particle had " + std::to_string(over) + " neighbours; the list capacity is " +
                   std::to_string(pbf::k4_of(*x) * pbf::kChunk) + " (max_neighbors " +
                   std::to_string(x->p.max_neighbors) + ")");
+}
+
+// Before the first step after a load: whether the state is for the tiles.
+int first_census(Ctx* x) {
+  if (!x->census_due || x->schedule == PBF_SCHED_PERSISTENT) return PBF_OK;
+  HIPCHK(x, pbf::launch_tile_census(*x));
+  const int rc = read_flags(x);
+  if (rc != PBF_OK) return rc;
+  HIPCHK(x, hipStreamSynchronize(x->stream));
+  x->tile_sparse = mostly_sparse(x, x->flag_host[pbf::kTileSparseSlot]);
+  x->census_due = false;
+  return PBF_OK;
 }
 
 // Steps per captured graph of calls of several steps, and the largest state
@@ -1051,6 +1058,8 @@ int capture_steps(Ctx* x, const SimConst& k, float dt, int steps, bool inner, pb
 int enqueue_steps(Ctx* x, float dt, int nsteps) {
   if (nsteps == 0) return PBF_OK;
   x->field_ready = false;
+  const int cs = first_census(x);
+  if (cs != PBF_OK) return cs;
   x->pending = true;
   const SimConst k = pbf::consts_for(*x, dt);
   if (x->schedule == PBF_SCHED_PERSISTENT) {
@@ -1208,6 +1217,7 @@ static int pbf_step_profiled_impl(pbf_ctx* c, float dt, int32_t nsteps, float* p
     if (pass_launches) pass_launches[i] = 0;
   }
   x->field_ready = false;
+  if ((rc = first_census(x)) != PBF_OK) return rc;
   HIPCHK(x, pbf::launch_fill_u32(x->d.flags, 1, 0u, x->stream));
   // Events of every launch of every step, read after one synchronisation at
   // the end, so the steps run back to back as in pbf_step.

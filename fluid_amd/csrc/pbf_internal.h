@@ -223,12 +223,13 @@ struct Ctx {
   // the per-lane passes: those are up to a third faster there, the tiles where
   // blocks are full (1,000,000 random particles, ms per step, per-lane / tiles:
   // 20 a block 0.34 / 0.42, 100 0.50 / 0.61, 150 0.58 / 0.85, 250 0.70 / 0.78, 350
-  // 0.81 / 0.77, 480 0.98 / 0.74).  Known from a count at the load and from the
-  // last steps' tiles; while tiles are off, from a count every kTileCensus
-  // steps.  Which passes run changes no bit.
+  // 0.81 / 0.77, 480 0.98 / 0.74).  Known from a count before the first step
+  // after a load and from the last steps' tiles; while tiles are off, from a
+  // count every kTileCensus steps.  Which passes run changes no bit.
   bool tile_sparse = false;
   bool tile_forced = false;          // PBF_TILE_MIN is set: tiles whatever the density
   int64_t census_steps = 0;          // steps since the last count
+  bool census_due = false;           // none since the load
   uint32_t tile_cap = 0;             // items allocated
   uint32_t tile_units = 0;           // units allocated
   // Density-field output on the device, kept between calls, and two pinned
@@ -339,8 +340,7 @@ hipError_t launch_scan_u32(uint32_t* in, uint32_t* out, uint32_t n, uint32_t* pa
 bool tile_step(const Ctx& x, const SimConst& c);
 // Estimates the committed particles in thin blocks in flags[kTileSparseSlot]
 // (overwrites the cell histogram, which every call's first prediction clears).
-// clear = false: that word is zero already.
-hipError_t launch_tile_census(Ctx& x, bool clear = true);
+hipError_t launch_tile_census(Ctx& x);
 size_t tile_block_count(const SceneGrid& g);
 
 }  // namespace pbf

@@ -1996,9 +1996,9 @@ bool tile_step(const Ctx& x, const SimConst& c) {
          x.schedule != PBF_SCHED_PERSISTENT && !(x.small_sort && sort_in_one_workgroup(x));
 }
 
-hipError_t launch_tile_census(Ctx& x, bool clear) {
+hipError_t launch_tile_census(Ctx& x) {
   hipError_t e = launch_fill_u32(x.d.cellCount, x.tile_blocks, 0u, x.stream);
-  if (e == hipSuccess && clear) e = launch_fill_u32(x.d.flags + kTileSparseSlot, 1, 0u, x.stream);
+  if (e == hipSuccess) e = launch_fill_u32(x.d.flags + kTileSparseSlot, 1, 0u, x.stream);
   if (e != hipSuccess) return e;
   k_tile_census<<<blocks_for((x.n + kCensusStep - 1) / kCensusStep), kBlock, 0, x.stream>>>(
       x.d.posA, (uint32_t)x.n, x.grids[0], x.d.cellCount);
